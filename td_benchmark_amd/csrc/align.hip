@@ -12,8 +12,10 @@
 // The within-expert order is the stable (ascending slot) order, so the result
 // is deterministic and bit-exact against the CPU restatement.
 //
-// Small problems (S <= 1024, E <= 256) take one launch (align_small_kernel);
-// otherwise three launches, none of which waits on another workgroup:
+// Up to 16384 slots one launch with a workgroup per expert (align_expert)
+// computes everything, alone or beside the activation quant in the same launch
+// (the two do not depend on each other); above that three launches, none of
+// which waits on another workgroup:
 //   1. count:  1024 slots per workgroup.  Slots with equal expert inside a wave
 //      are found with log2(E) ballots (a match-any built from per-bit ballots),
 //      giving each slot its rank among equal-expert slots of its wave; per-wave
@@ -28,8 +30,10 @@
 //      the offsets held in LDS).
 // Align moves well under 2 MB at every configuration, so it is latency-bound.
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
+#include "quant_group.hpp"
 
 namespace moe {
 
@@ -194,113 +198,116 @@ __global__ __launch_bounds__(256) void align_place_kernel(
   }
 }
 
-// Small problems (S <= 1024 slots, E <= 256 experts) in one launch: one
-// workgroup walks the slots 1024 at a time, keeping running per-expert counts
-// in LDS so every slot gets its rank within its expert (the same stable order
-// as the three-kernel path), then scans, places and fills like the wide pass.
-// Measured on MI355X: faster than the three launches for one chunk of slots
-// (and half the launches when the host issues them), slower from ~2 chunks on,
-// where the serial chunk loop outweighs the saved launches.
-constexpr int64_t kAlignSmallSlots = 1024;
-constexpr int kAlignSmallExperts = 256;
+// One launch, a workgroup per expert: every workgroup reads all slot ids (at
+// most 64 KiB, from L2 after the first reader), counts every expert's slots in
+// LDS, sums the padded sizes before its own expert, and compacts its expert's
+// slots in ascending order (each wave owns a contiguous stretch of the slots;
+// ballots give a slot its rank).  No workgroup waits on another one.
+// Bound by its chain of about four dependent steps, not by bytes.  Against the
+// three launches it replaces (kernel time): S = 8192, E = 64: 7.8 us with the
+// quant in the same launch, 19 us before (quant 5.0, count, scan and place 4.7
+// each); S = 2408, E = 128: 4.9 us, before 17; against the former single
+// workgroup for S <= 1024 with the quant: S = 128, E = 8: 3.1 us, before 6.6.
+struct AlignArgs {
+  const int32_t* ids;
+  const int32_t* expert_map;  // or null
+  int32_t* sorted;
+  int32_t* eids;
+  int32_t* ntpp;
+  int64_t max_padded;
+  int S, E, BM;
+};
 
-__global__ __launch_bounds__(kAlignChunk) void align_small_kernel(
-    const int32_t* __restrict__ ids, int64_t S, int E, int nbits, int BM,
-    const int32_t* __restrict__ expert_map, int32_t* __restrict__ sorted_ids,
-    int32_t* __restrict__ expert_ids, int32_t* __restrict__ ntpp_out, int64_t max_padded) {
-  extern __shared__ int32_t lds[];
-  int32_t* wcnt = lds;                         // [16][E]
-  int32_t* base = wcnt + 16 * E;               // [E] running counts
-  int32_t* s_off = base + E;                   // [E + 1]
-  int32_t* s_e = s_off + E + 1;                // [S] expert of each slot (-1 = dropped)
-  int32_t* s_rank = s_e + S;                   // [S] rank of the slot within its expert
-  __shared__ int32_t wave_tot[kAlignChunk / 64];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  for (int i = tid; i < E; i += kAlignChunk) base[i] = 0;
-  for (int64_t c0 = 0; c0 < S; c0 += kAlignChunk) {
-    for (int i = tid; i < 16 * E; i += kAlignChunk) wcnt[i] = 0;
-    const int64_t sl = c0 + tid;
-    int e = -1;
-    if (sl < S) e = ids[sl];
-    const bool valid = (e >= 0) && (e < E);
-    uint64_t m = __ballot(valid);
-    for (int b = 0; b < nbits; ++b) {
-      const bool bit = (e >> b) & 1;
-      const uint64_t bb = __ballot(bit);
-      m &= bit ? bb : ~bb;
-    }
-    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const int rank_in_wave = __popcll(m & lt);
-    __syncthreads();
-    if (valid && rank_in_wave == 0) wcnt[wave * E + e] = __popcll(m);
-    __syncthreads();
-    for (int x = tid; x < E; x += kAlignChunk) {
-      int run = base[x];
+constexpr int kAlignThreads = 512;
+constexpr int kAlignWaves = kAlignThreads / 64;
+
+// IT: ids a lane holds (IT * 512 >= S).
+template <int IT>
+MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
+  __shared__ int32_t hist[kAlignMaxExperts];
+  __shared__ int32_t wave_cnt[kAlignWaves], wave_before[kAlignWaves], wave_total[kAlignWaves];
+  const int sh = __builtin_ctz(a.BM);  // BM is a power of two
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  // wave w takes slots [w*IT*64, (w+1)*IT*64), 64 consecutive ones a step
+  const int first = wave * IT * 64 + lane;
+  int id[IT];
 #pragma unroll
-      for (int w = 0; w < 16; ++w) {
-        const int t = wcnt[w * E + x];
-        wcnt[w * E + x] = run;
-        run += t;
-      }
-      base[x] = run;
-    }
-    __syncthreads();
-    if (sl < S) {
-      s_e[sl] = valid ? e : -1;
-      s_rank[sl] = valid ? wcnt[wave * E + e] + rank_in_wave : 0;
-    }
-    __syncthreads();
-  }
-  // padded sizes and their exclusive scan across experts (E <= 256 < 1024 threads)
-  const int cnt = tid < E ? base[tid] : 0;
-  const int padded = (cnt + BM - 1) / BM * BM;
-  int incl = padded;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(incl, o);
-    if (lane >= o) incl += y;
-  }
-  if (lane == 63) wave_tot[wave] = incl;
+  for (int i = 0; i < IT; ++i) id[i] = first + 64 * i < a.S ? a.ids[first + 64 * i] : -1;
+  for (int i = tid; i < a.E; i += kAlignThreads) hist[i] = 0;
   __syncthreads();
-  if (tid < 64) {
-    const int t = tid < kAlignChunk / 64 ? wave_tot[tid] : 0;
-    int x = t;
+  int mine = 0;  // this wave's slots of expert e
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) {
-      const int y = __shfl_up(x, o);
-      if (lane >= o) x += y;
-    }
-    if (tid < kAlignChunk / 64) wave_tot[tid] = x - t;
-    if (tid == kAlignChunk / 64 - 1) {
-      s_off[E] = x;
-      *ntpp_out = x;
-    }
+  for (int i = 0; i < IT; ++i) {
+    if ((unsigned)id[i] < (unsigned)a.E) atomicAdd(&hist[id[i]], 1);
+    mine += __popcll(__ballot(id[i] == e));
+  }
+  if (lane == 0) wave_cnt[wave] = mine;
+  __syncthreads();
+  int before = 0, total = 0;  // padded sizes of the experts before e, and of all
+  for (int x = tid; x < a.E; x += kAlignThreads) {
+    const int p = (hist[x] + a.BM - 1) >> sh << sh;
+    total += p;
+    if (x < e) before += p;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    before += __shfl_xor(before, o);
+    total += __shfl_xor(total, o);
+  }
+  if (lane == 0) {
+    wave_before[wave] = before;
+    wave_total[wave] = total;
   }
   __syncthreads();
-  if (tid < E) s_off[tid] = wave_tot[wave] + incl - padded;
-  __syncthreads();
-  for (int64_t sl = tid; sl < S; sl += kAlignChunk) {
-    const int e = s_e[sl];
-    if (e >= 0) sorted_ids[s_off[e] + s_rank[sl]] = (int32_t)sl;
+  before = total = 0;
+  int rank = 0;  // of this wave's first slot of e
+#pragma unroll
+  for (int w = 0; w < kAlignWaves; ++w) {
+    before += wave_before[w];
+    total += wave_total[w];
+    rank += w < wave ? wave_cnt[w] : 0;
   }
-  const int total = s_off[E];
-  for (int64_t i = tid; i < max_padded; i += kAlignChunk) {
-    int e = -1;
-    bool pad = true;
-    if (i < total) {
-      int lo = 0, hi = E - 1;  // largest e with off[e] <= i
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (s_off[mid] <= i) lo = mid;
-        else hi = mid - 1;
-      }
-      e = lo;
-      pad = (i - s_off[e]) >= base[e];
-    }
-    if (pad) sorted_ids[i] = (int32_t)S;
-    if (i % BM == 0) expert_ids[i / BM] = (expert_map && e >= 0) ? expert_map[e] : e;
+  const int cnt = hist[e];
+  const int padded = (cnt + a.BM - 1) >> sh << sh;
+  const uint64_t lt = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const uint64_t m = __ballot(id[i] == e);
+    if (id[i] == e) a.sorted[before + rank + __popcll(m & lt)] = first + 64 * i;
+    rank += __popcll(m);
   }
+  for (int i = cnt + tid; i < padded; i += kAlignThreads) a.sorted[before + i] = a.S;
+  const int local = a.expert_map ? a.expert_map[e] : e;
+  for (int i = tid; i < padded >> sh; i += kAlignThreads) a.eids[(before >> sh) + i] = local;
+  // the positions and blocks past ntpp, shared out over the workgroups
+  for (int64_t i = total + (int64_t)e * kAlignThreads + tid; i < a.max_padded; i += (int64_t)a.E * kAlignThreads) {
+    a.sorted[i] = a.S;
+    if ((i & (a.BM - 1)) == 0) a.eids[i >> sh] = -1;
+  }
+  if (e == 0 && tid == 0) *a.ntpp = total;
 }
+
+template <int IT>
+__global__ __launch_bounds__(kAlignThreads) void align_expert_kernel(AlignArgs a) {
+  align_expert<IT>(a, blockIdx.x);
+}
+
+// The same workgroups followed by those of the 1x128 activation quant, one
+// launch for the layer's two first stages (they are independent, and each alone
+// leaves most of the chip idle at the sizes taken here).
+template <int IT, bool WHOLE>
+__global__ __launch_bounds__(kAlignThreads) void quant_align_kernel(AlignArgs a, QuantArgs q) {
+  if ((int)blockIdx.x < a.E)
+    align_expert<IT>(a, blockIdx.x);
+  else
+    quant_chunks<kAlignThreads, 1, false, WHOLE>(q, (int64_t)blockIdx.x - a.E);
+}
+
+// The one-launch form holds up to 32 ids a lane.
+constexpr int64_t kAlignOneLaunchSlots = 32 * kAlignThreads;
+// Chunks (16 B of input) up to which the quant runs beside align; larger ones
+// are bound by HBM and take the quant kernel's own block and unroll.
+constexpr int64_t kQuantBesideAlign = (int64_t)1 << 22;
 
 }  // namespace moe
 
@@ -334,18 +341,25 @@ static int align_args(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
   return kOk;
 }
 
+// f(ids a lane holds) for the one-launch form.
+template <class F>
+static void by_slots(int64_t S, F&& f) {
+  if (S <= 2 * kAlignThreads) f(std::integral_constant<int, 2>{});
+  else if (S <= 8 * kAlignThreads) f(std::integral_constant<int, 8>{});
+  else f(std::integral_constant<int, 32>{});
+}
+
 static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
                       int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded,
                       void* workspace, void* stream) {
   const int arg_rc = align_args(topk_ids, S, E, BM, sorted_ids, expert_ids, ntpp, max_padded, true, workspace);
   if (arg_rc != kOk) return arg_rc;
   hipStream_t st = (hipStream_t)stream;
-  int nbits0 = 0;
-  while ((1 << nbits0) < E) ++nbits0;
-  if (S > 0 && S <= kAlignSmallSlots && E <= kAlignSmallExperts) {
-    const size_t lds = (size_t)(16 * E + E + E + 1 + 2 * S) * sizeof(int32_t);
-    hipLaunchKernelGGL(align_small_kernel, dim3(1), dim3(kAlignChunk), lds, st, topk_ids, S, (int)E, nbits0,
-                       (int)BM, expert_map, sorted_ids, expert_ids, ntpp, max_padded);
+  if (S <= kAlignOneLaunchSlots) {
+    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, max_padded, (int)S, (int)E, (int)BM};
+    by_slots(S, [&](auto it) {
+      hipLaunchKernelGGL(align_expert_kernel<decltype(it)::value>, dim3((unsigned)E), dim3(kAlignThreads), 0, st, a);
+    });
     return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
   }
   const int64_t n_chunks = (S + kAlignChunk - 1) / kAlignChunk;
@@ -376,6 +390,37 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
                        topk_ids, S, (int)E, (int)BM, chunk_count, rank, off, cnt, expert_map,
                        sorted_ids, expert_ids, max_padded);
   }
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+extern "C" int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq, float* scales,
+                               const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
+                               const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp,
+                               int64_t max_padded, void* workspace, void* stream) {
+  // both halves' arguments before either is launched
+  if (T < 0 || H < 0 || ldq < (H + 127) / 128 * 128) return kErrBadShape;
+  if (T > 0 && H > 0) {
+    if (!x_bf16 || !q_fp8 || !scales) return kErrNullPointer;
+    if (((uintptr_t)x_bf16 & 1) != 0) return kErrBadShape;
+  }
+  const int rc = align_args(topk_ids, S, E, BM, sorted_ids, expert_ids, ntpp, max_padded, true, workspace);
+  if (rc != kOk) return rc;
+  const QuantArgs q = quant_args(x_bf16, T, H, q_fp8, ldq, scales);
+  if (S > kAlignOneLaunchSlots || q.n_chunks == 0 || q.n_chunks > kQuantBesideAlign ||
+      !quant_vectorised(x_bf16, H, q_fp8, ldq)) {
+    const int qrc = moe_quant_group128_padded(x_bf16, T, H, q_fp8, ldq, scales, stream);
+    if (qrc != kOk) return qrc;
+    return align_impl(topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp, max_padded, workspace, stream);
+  }
+  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, max_padded, (int)S, (int)E, (int)BM};
+  const unsigned grid = (unsigned)(E + (q.n_chunks + kAlignThreads - 1) / kAlignThreads);
+  by_slots(S, [&](auto it) {
+    constexpr int IT = decltype(it)::value;
+    if (quant_whole(q))
+      hipLaunchKernelGGL((quant_align_kernel<IT, true>), dim3(grid), dim3(kAlignThreads), 0, (hipStream_t)stream, a, q);
+    else
+      hipLaunchKernelGGL((quant_align_kernel<IT, false>), dim3(grid), dim3(kAlignThreads), 0, (hipStream_t)stream, a, q);
+  });
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 

@@ -7,13 +7,11 @@
 // code = e4m3fn_RNE(clamp(x / scale, +-448)).
 //
 // quant_group128 is HBM-bound: 2 B in + 1 B out per element + 4 B of scale per
-// 128 elements (widths that are not a multiple of 128, or unaligned rows, take
-// a general one-wave-per-group kernel instead).  Sixteen lanes own one 128-element group (16 B = 8 bf16 each),
-// so every wave reads 1 KiB and writes 512 B contiguously with 128-bit loads;
-// the group amax is a 16-lane xor-shuffle reduction.  Non-temporal
-// (streaming) loads and stores and a shallow per-thread unroll measured best
+// 128 elements (widths that are not a multiple of 8, or unaligned rows, take
+// a general one-wave-per-group kernel instead).  Non-temporal (streaming) loads and stores and a shallow per-thread unroll measured best
 // on MI355X: many short waves keep more requests in flight than a deep unroll.
 #include "common.hpp"
+#include "quant_group.hpp"
 
 namespace moe {
 
@@ -28,71 +26,13 @@ constexpr int quant_unroll() { return SWIGLU ? 4 : 2; }
 //   h = bf16(silu(gate) * up) (A6 then A7, the standalone form of what the
 //   fused W13 epilogue does), with the same rounding chain as the separate
 //   silu_and_mul and quant kernels, so the codes agree bit for bit.
-// A chunk is 8 consecutive output columns of one row; W/8 chunks per row.
-template <bool SWIGLU>
-__global__ __launch_bounds__(kQuantThreads) void quant_group128_kernel(
-    const uint16_t* __restrict__ x, uint8_t* __restrict__ q, float* __restrict__ s,
-    int64_t n_chunks, int64_t chunks_per_row) {
-  constexpr int kQuantUnroll = quant_unroll<SWIGLU>();
-  const int tid = threadIdx.x;
-  const int64_t base = (int64_t)blockIdx.x * kQuantThreads * kQuantUnroll;
-  constexpr int NLOAD = SWIGLU ? 2 : 1;
-  v4i raw[kQuantUnroll][NLOAD];
-#pragma unroll
-  for (int i = 0; i < kQuantUnroll; ++i) {
-    const int64_t ch = base + tid + i * kQuantThreads;
-    if (ch < n_chunks) {
-      if constexpr (SWIGLU) {
-        const int64_t r = ch / chunks_per_row, cc = ch % chunks_per_row;
-        const uint16_t* row = x + r * chunks_per_row * 16;
-        raw[i][0] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(row + cc * 8));
-        raw[i][NLOAD - 1] =
-            __builtin_nontemporal_load(reinterpret_cast<const v4i*>(row + chunks_per_row * 8 + cc * 8));
-      } else {
-        raw[i][0] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(x + ch * 8));
-      }
-    } else {
-#pragma unroll
-      for (int l = 0; l < NLOAD; ++l) raw[i][l] = (v4i){0, 0, 0, 0};
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < kQuantUnroll; ++i) {
-    const int64_t ch = base + tid + i * kQuantThreads;
-    float v[8];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t w = (uint32_t)raw[i][0][j];
-      if constexpr (SWIGLU) {
-        const uint32_t u = (uint32_t)raw[i][NLOAD - 1][j];
-        v[2 * j] = silu_mul_bf16(lo_bf16(w), lo_bf16(u));
-        v[2 * j + 1] = silu_mul_bf16(hi_bf16(w), hi_bf16(u));
-      } else {
-        v[2 * j] = lo_bf16(w);
-        v[2 * j + 1] = hi_bf16(w);
-      }
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-    // 16 lanes of one group are 16 consecutive lanes of the wave.
-    amax = fmaxf(amax, __shfl_xor(amax, 1));
-    amax = fmaxf(amax, __shfl_xor(amax, 2));
-    amax = fmaxf(amax, __shfl_xor(amax, 4));
-    amax = fmaxf(amax, __shfl_xor(amax, 8));
-    const float sc = group_scale(amax);
-    const float inv = 1.0f / sc;
-    const uint32_t lo = quant4_e4m3(v[0], v[1], v[2], v[3], sc, inv);
-    const uint32_t hi = quant4_e4m3(v[4], v[5], v[6], v[7], sc, inv);
-    if (ch < n_chunks) {
-      __builtin_nontemporal_store((v2u){lo, hi}, reinterpret_cast<v2u*>(q + ch * 8));
-      if ((tid & 15) == 0) s[ch >> 4] = sc;
-    }
-  }
+template <bool SWIGLU, bool WHOLE>
+__global__ __launch_bounds__(kQuantThreads) void quant_group128_kernel(QuantArgs a) {
+  quant_chunks<kQuantThreads, quant_unroll<SWIGLU>(), SWIGLU, WHOLE>(a, blockIdx.x);
 }
 
-// Any width and row strides (the vectorised kernel above needs W % 128 == 0
-// and aligned rows): one wave per 128-column group of one row, two columns
+// Any width and alignment (the vectorised kernel above needs W % 8 == 0 and
+// aligned rows): one wave per 128-column group of one row, two columns
 // per lane.  A row's last group holds W mod 128 columns when W is not a
 // multiple of 128; the reference zero-pads it to 128 (verify.py:111-113), and
 // zeros change neither the group's amax nor the other codes, so only the W
@@ -186,23 +126,36 @@ static int quant_any(const void* x_bf16, int64_t ldx, int64_t T, int64_t H, int6
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
+template <bool SWIGLU, bool WHOLE>
+static int launch_quant(const QuantArgs& a, void* stream) {
+  constexpr int64_t per_block = kQuantThreads * quant_unroll<SWIGLU>();
+  const int64_t blocks = (a.n_chunks + per_block - 1) / per_block;
+  hipLaunchKernelGGL((quant_group128_kernel<SWIGLU, WHOLE>), dim3((unsigned)blocks), dim3(kQuantThreads), 0,
+                     (hipStream_t)stream, a);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+// Rows of H columns into rows of ldq bytes (the padding, if any, up to pad_to).
+// A width that is a multiple of 8 on aligned rows takes the vectorised kernel
+// (a [777, 2200] layer input: see quant_group.hpp), whole groups its dense form.
+static int quant_rows(const void* x_bf16, int64_t T, int64_t H, int64_t pad_to, void* q_fp8, int64_t ldq,
+                      float* scales, void* stream) {
+  if (H % 128 != 0 && T * ((H + 127) / 128) > (int64_t)0xFFFFFFFF * 4) return kErrBadShape;
+  if (quant_vectorised(x_bf16, H, q_fp8, ldq)) {
+    const QuantArgs a = quant_args(x_bf16, T, H, q_fp8, ldq, scales);
+    return quant_whole(a) ? launch_quant<false, true>(a, stream) : launch_quant<false, false>(a, stream);
+  }
+  if (((uintptr_t)x_bf16 & 1) != 0) return kErrBadShape;
+  if (T * ((H + 127) / 128) > (int64_t)0xFFFFFFFF * 4) return kErrBadShape;
+  return quant_any(x_bf16, H, T, H, pad_to, q_fp8, ldq, scales, (H + 127) / 128, stream);
+}
+
 extern "C" int moe_quant_group128(const void* x_bf16, int64_t T, int64_t H, void* q_fp8,
                                   float* scales, void* stream) {
   if (T < 0 || H < 0) return kErrBadShape;
   if (T == 0 || H == 0) return kOk;
   if (!x_bf16 || !q_fp8 || !scales) return kErrNullPointer;
-  if ((H % 128 != 0 || ((uintptr_t)x_bf16 & 15) != 0 || ((uintptr_t)q_fp8 & 7) != 0)) {
-    if (((uintptr_t)x_bf16 & 1) != 0) return kErrBadShape;
-    if (T * ((H + 127) / 128) > (int64_t)0xFFFFFFFF * 4) return kErrBadShape;
-    return quant_any(x_bf16, H, T, H, H, q_fp8, H, scales, (H + 127) / 128, stream);
-  }
-  const int64_t n_chunks = T * H / 8;
-  constexpr int64_t per_block = kQuantThreads * quant_unroll<false>();
-  const int64_t blocks = (n_chunks + per_block - 1) / per_block;
-  hipLaunchKernelGGL(quant_group128_kernel<false>, dim3((unsigned)blocks), dim3(kQuantThreads), 0,
-                     (hipStream_t)stream, (const uint16_t*)x_bf16, (uint8_t*)q_fp8, scales,
-                     n_chunks, H / 8);
-  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+  return quant_rows(x_bf16, T, H, H, q_fp8, H, scales, stream);
 }
 
 extern "C" int moe_quant_group128_padded(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq,
@@ -212,10 +165,7 @@ extern "C" int moe_quant_group128_padded(const void* x_bf16, int64_t T, int64_t 
   if (ldq < hp) return kErrBadShape;
   if (T == 0 || H == 0) return kOk;
   if (!x_bf16 || !q_fp8 || !scales) return kErrNullPointer;
-  if (ldq == H) return moe_quant_group128(x_bf16, T, H, q_fp8, scales, stream);
-  if (((uintptr_t)x_bf16 & 1) != 0) return kErrBadShape;
-  if (T * (hp / 128) > (int64_t)0xFFFFFFFF * 4) return kErrBadShape;
-  return quant_any(x_bf16, H, T, H, hp, q_fp8, ldq, scales, hp / 128, stream);
+  return quant_rows(x_bf16, T, H, hp, q_fp8, ldq, scales, stream);
 }
 
 extern "C" int moe_silu_mul_quant_group128(const void* c_bf16, int64_t R, int64_t I, void* q_fp8,
@@ -225,13 +175,7 @@ extern "C" int moe_silu_mul_quant_group128(const void* c_bf16, int64_t R, int64_
   if (!c_bf16 || !q_fp8 || !scales) return kErrNullPointer;
   if (I % 128 != 0) return kErrBadShape;
   if (((uintptr_t)c_bf16 & 15) != 0 || ((uintptr_t)q_fp8 & 7) != 0) return kErrBadShape;
-  const int64_t n_chunks = R * I / 8;
-  constexpr int64_t per_block = kQuantThreads * quant_unroll<true>();
-  const int64_t blocks = (n_chunks + per_block - 1) / per_block;
-  hipLaunchKernelGGL(quant_group128_kernel<true>, dim3((unsigned)blocks), dim3(kQuantThreads), 0,
-                     (hipStream_t)stream, (const uint16_t*)c_bf16, (uint8_t*)q_fp8, scales,
-                     n_chunks, I / 8);
-  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+  return launch_quant<true, true>(quant_args(c_bf16, R, I, q_fp8, I, scales), stream);
 }
 
 extern "C" int moe_quant_block128(const float* w, int64_t E, int64_t N, int64_t K, void* q_fp8,

@@ -219,21 +219,25 @@ class AlignBuffers:
         self.workspace = torch.empty(align_workspace_bytes(num_slots, num_experts), dtype=torch.uint8,
                                      device=device)
 
+    def need_ids(self, topk_ids: torch.Tensor, expert_map: torch.Tensor | None) -> None:
+        _need(topk_ids, "topk_ids", torch.int32)
+        if topk_ids.numel() != self.S:
+            raise ValueError(f"topk_ids has {topk_ids.numel()} slots, buffers were sized for {self.S}")
+        if expert_map is not None:
+            _need(expert_map, "expert_map", torch.int32)
+            if expert_map.numel() != self.E:
+                raise ValueError(f"expert_map must have {self.E} entries")
+
     def run(self, topk_ids: torch.Tensor,
             expert_map: torch.Tensor | None = None) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
         """``expert_map`` (int32 [E], global -> local expert id or -1): block
         expert ids are reported as local ids (expert parallelism)."""
-        _need(topk_ids, "topk_ids", torch.int32)
-        if topk_ids.numel() != self.S:
-            raise ValueError(f"topk_ids has {topk_ids.numel()} slots, buffers were sized for {self.S}")
+        self.need_ids(topk_ids, expert_map)
         if expert_map is None:
             check(lib().moe_align_block_size(_ptr(topk_ids), self.S, self.E, self.BM, _ptr(self.sorted_ids),
                                              _ptr(self.expert_ids), _ptr(self.ntpp), self.max_padded,
                                              _ptr(self.workspace), _stream()), "moe_align_block_size")
         else:
-            _need(expert_map, "expert_map", torch.int32)
-            if expert_map.numel() != self.E:
-                raise ValueError(f"expert_map must have {self.E} entries")
             check(lib().moe_align_block_size_mapped(_ptr(topk_ids), self.S, self.E, self.BM, _ptr(expert_map),
                                                     _ptr(self.sorted_ids), _ptr(self.expert_ids), _ptr(self.ntpp),
                                                     self.max_padded, _ptr(self.workspace), _stream()),
@@ -821,10 +825,13 @@ class FusedExpertsRunner:
         # the top-k sum at the padded width, whose first H columns are y
         self.y_pad = self.y if Hp == H else torch.empty((self.T, Hp), dtype=torch.bfloat16, device=dev)
 
-    def stage_quant(self, hidden: torch.Tensor) -> None:
+    def _need_hidden(self, hidden: torch.Tensor) -> None:
         _need(hidden, "hidden_states", torch.bfloat16)
         if tuple(hidden.shape) != (self.T, self.H):
             raise ValueError(f"hidden_states must be [{self.T}, {self.H}]")
+
+    def stage_quant(self, hidden: torch.Tensor) -> None:
+        self._need_hidden(hidden)
         if self.Hp == self.H:
             check(lib().moe_quant_group128(_ptr(hidden), self.T, self.H, _ptr(self.q1), _ptr(self.s1),
                                            _stream()), "moe_quant_group128")
@@ -903,8 +910,13 @@ class FusedExpertsRunner:
             self.y.copy_(self.y_pad[:, : self.H])
 
     def run(self, hidden: torch.Tensor, topk_weights: torch.Tensor, topk_ids: torch.Tensor) -> torch.Tensor:
-        self.stage_quant(hidden)
-        self.stage_align(topk_ids)
+        self._need_hidden(hidden)
+        a = self.align
+        a.need_ids(topk_ids, self.expert_map)
+        check(lib().moe_quant_align(_ptr(hidden), self.T, self.H, _ptr(self.q1), self.Hp, _ptr(self.s1),
+                                    _ptr(topk_ids), self.S, a.E, self.BM, _ptr(self.expert_map), _ptr(a.sorted_ids),
+                                    _ptr(a.expert_ids), _ptr(a.ntpp), a.max_padded, _ptr(a.workspace), _stream()),
+              "moe_quant_align")
         self.stage_scales()
         self.stage_w13()
         self.stage_w2(topk_weights)

@@ -1,0 +1,105 @@
+"""GPU: the layer's first launch (moe_quant_align) and the one-launch align
+against the oracle, bit for bit, at the edges of their ranges: slot counts at
+the ids-per-lane limits and at the switch to three launches, one to 1000
+experts, skewed and dropped ids, expert maps, and quant widths that are whole
+groups, whole chunks of 8, and neither."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from moe_cases import u8_bits
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+# (T, k, E, BM, H, kind): S = T*k around 1024, 4096 and 16384
+CASES = [
+    (1, 1, 1, 16, 128, "uniform"),
+    (3, 2, 256, 32, 136, "uniform"),
+    (1024, 1, 8, 64, 256, "one"),
+    (205, 5, 60, 16, 200, "dropped"),      # S = 1025
+    (512, 8, 128, 256, 64, "uniform"),     # S = 4096
+    (4097, 1, 1000, 32, 100, "skewed"),    # S = 4097, general quant
+    (2048, 8, 256, 128, 1160, "mapped"),   # S = 16384
+    (16385, 1, 64, 16, 128, "mapped"),     # three launches
+]
+
+
+@pytest.mark.parametrize("T,k,E,BM,H,kind", CASES)
+def test_quant_align_equals_the_oracle(T, k, E, BM, H, kind):
+    from td_benchmark_amd import ops
+    from td_benchmark_amd._lib import check, lib
+    print(f"case: quant_align T={T} k={k} E={E} BM={BM} H={H} {kind}", flush=True)
+    rng = np.random.default_rng(T + E)
+    ids = rng.integers(0, E, (T, k)).astype(np.int32)
+    if kind == "one":
+        ids[:] = E - 1
+    elif kind == "skewed":
+        ids = (E * rng.random((T, k)) ** 6).astype(np.int32)
+    elif kind == "dropped":
+        ids[rng.random((T, k)) < 0.2] = -1
+        ids[rng.random((T, k)) < 0.2] = E
+    emap = None
+    if kind == "mapped":
+        emap = np.full(E, -1, np.int32)
+        emap[rng.choice(E, E // 4, replace=False)] = np.arange(E // 4, dtype=np.int32)
+    x = oracle.f32_to_bf16(rng.standard_normal((T, H), dtype=np.float32))
+    x[0] = 0
+    srt_ref, eids_ref, ntpp_ref = oracle.moe_align(ids, E, BM)
+    if emap is not None:
+        eids_ref = np.where(eids_ref >= 0, emap[np.maximum(eids_ref, 0)], -1)
+    q_ref, s_ref = oracle.quant_group128(x)
+    hp = (H + 127) // 128 * 128
+    dx = torch.from_numpy(x.view(np.int16)).cuda().view(torch.bfloat16)
+    dids = torch.from_numpy(ids).cuda()
+    dmap = None if emap is None else torch.from_numpy(emap).cuda()
+    for one_call in (True, False):
+        b = ops.AlignBuffers(T * k, E, BM, dx.device)
+        for t in (b.sorted_ids, b.expert_ids, b.ntpp):
+            t.fill_(-7)
+        q = torch.full((T, hp), 0x55, dtype=torch.uint8, device="cuda")
+        s = torch.full((T, hp // 128), -1.0, device="cuda")
+        if one_call:
+            check(lib().moe_quant_align(ops._ptr(dx), T, H, ops._ptr(q), hp, ops._ptr(s), ops._ptr(dids), T * k, E, BM,
+                                        ops._ptr(dmap), ops._ptr(b.sorted_ids), ops._ptr(b.expert_ids),
+                                        ops._ptr(b.ntpp), b.max_padded, ops._ptr(b.workspace), ops._stream()),
+                  "moe_quant_align")
+        else:
+            b.run(dids, dmap)
+        torch.cuda.synchronize()
+        assert int(b.ntpp.item()) == ntpp_ref
+        np.testing.assert_array_equal(b.sorted_ids.cpu().numpy(), srt_ref)
+        np.testing.assert_array_equal(b.expert_ids.cpu().numpy(), eids_ref)
+        if one_call:
+            q = u8_bits(q)
+            np.testing.assert_array_equal(q[:, :H], q_ref)
+            assert (q[:, H:] == 0).all()
+            np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32), s_ref.view(np.uint32))
+
+
+@pytest.mark.parametrize("H", [8, 136, 200, 2200])
+def test_vectorised_ragged_quant_equals_the_general_kernel(H):
+    """Random bit patterns (infinities, quiet and signalling NaNs, -0,
+    subnormals among them): aligned rows take the vectorised kernel, rows one
+    element off the general one."""
+    from td_benchmark_amd import ops
+    from td_benchmark_amd._lib import check, lib
+    print(f"case: ragged quant, any bits, H={H}", flush=True)
+    T, hp = 512, (H + 127) // 128 * 128
+    rng = np.random.default_rng(H)
+    bits = rng.integers(0, 65536, (T, H)).astype(np.uint16)
+    flat = torch.from_numpy(np.concatenate([[0], bits.ravel()]).astype(np.uint16).view(np.int16)).cuda()
+    off, dx = flat[1:], flat[1:].clone()
+    assert dx.data_ptr() % 16 == 0 and off.data_ptr() % 16 == 2
+    out = []
+    for x in (dx, off):
+        q = torch.full((T, hp), 0x55, dtype=torch.uint8, device="cuda")
+        s = torch.empty((T, hp // 128), dtype=torch.float32, device="cuda")
+        check(lib().moe_quant_group128_padded(ops._ptr(x), T, H, ops._ptr(q), hp, ops._ptr(s), ops._stream()), "quant")
+        torch.cuda.synchronize()
+        out.append((q.cpu().numpy(), s.cpu().numpy().view(np.uint32)))
+    np.testing.assert_array_equal(out[0][0], out[1][0])
+    np.testing.assert_array_equal(out[0][1], out[1][1])
