@@ -289,6 +289,56 @@ int moe_reduce_topk(const void* D_bf16, int64_t T, int32_t top_k, int64_t H, voi
 int moe_reduce_topk_add(const void* D_bf16, const void* addend_bf16, int64_t T, int32_t top_k,
                         int64_t H, void* y_bf16, void* stream);
 
+/* A10 -- the layer on prebuilt buffers (the chain of overlap/
+ * overlap_forward.py:252-313 on one device).  A moe_layer holds the sizes,
+ * weights and buffers of one layer; the caller fills it once and owns
+ * everything it points to.  The stages, in order, are moe_layer_quant_align,
+ * moe_layer_scales, moe_layer_w13, moe_layer_w2 and moe_layer_reduce; each
+ * checks its arguments as the entry points above do and enqueues the same
+ * kernels with the same results.
+ *
+ * With expert_map (global -> local expert id or -1, E_routed entries) the
+ * GEMMs run over the blocks of local experts only: hq and hs are written at
+ * their positions, D at their slots, and the top-k sum takes the other slots
+ * as zero without reading D there.  Without it E_routed == E. */
+typedef struct moe_layer {
+  int64_t T, H;               /* tokens, hidden size */
+  int64_t Hp, I;              /* hidden size padded to 128, intermediate size (a multiple of 128) */
+  int64_t max_padded;         /* moe_align_max_padded(T * top_k, E_routed, block_size_m) */
+  int32_t top_k, E, E_routed; /* experts here, experts the ids select from */
+  int32_t block_size_m;
+  int32_t tile_m;             /* GEMM tile rows, 0 = automatic */
+  int32_t exact_dot;          /* W13 in its exact-dot form */
+  const void* w13;            /* [E, 2I, Hp] e4m3fn and its block scales */
+  const float* w13_scale;
+  const void* w2;             /* [E, Hp, I] */
+  const float* w2_scale;
+  const int32_t* expert_map;  /* or NULL */
+  void* q1;                   /* [T, Hp] e4m3fn */
+  float* s1;                  /* [T, Hp/128] */
+  float* s1_pos;              /* [Hp/128, max_padded]: scales by sorted position, or NULL: row-major scales */
+  int32_t* sorted_ids;        /* align outputs and workspace, as moe_align_block_size */
+  int32_t* expert_ids;
+  int32_t* ntpp;
+  void* workspace;
+  int32_t* local_blocks;      /* moe_layer_local_blocks_bytes, with expert_map; else NULL */
+  void* hq;                   /* [max_padded, I] e4m3fn */
+  float* hs;                  /* [I/128, max_padded] with s1_pos, else [max_padded, I/128] */
+  void* D;                    /* [T * top_k, Hp] bf16 */
+} moe_layer;
+
+int64_t moe_layer_local_blocks_bytes(int64_t T, int64_t max_padded, int32_t block_size_m);
+/* hidden [T, H] bf16 (NULL: align alone), topk_ids [T, top_k]. */
+int moe_layer_quant_align(const moe_layer* layer, const void* hidden, const int32_t* topk_ids, void* stream);
+/* The activation scales by sorted position (nothing where s1_pos is NULL). */
+int moe_layer_scales(const moe_layer* layer, void* stream);
+int moe_layer_w13(const moe_layer* layer, void* stream);
+int moe_layer_w2(const moe_layer* layer, const float* topk_weights, void* stream);
+/* y [T, cols] = the first `cols` columns of the top-k sum (cols % 8 == 0), plus
+ * addend rows of stride addend_ld where addend is not NULL. */
+int moe_layer_reduce(const moe_layer* layer, const void* addend, int64_t addend_ld, int64_t cols, void* y,
+                     void* stream);
+
 /* FP8 reduce-scatter combine -- the dequantise-and-sum of the FP8 chunks a
  * rank receives in the FP8-compressed reduce-scatter leg, replacing
  * `(fp8.to(float32) * scale.repeat_interleave(128)).sum(dim=0).to(bfloat16)`

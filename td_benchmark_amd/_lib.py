@@ -31,6 +31,18 @@ _I32P = ctypes.c_void_p
 _i64 = ctypes.c_int64
 _i32 = ctypes.c_int32
 
+
+
+class MoeLayer(ctypes.Structure):
+    """struct moe_layer of include/moe_mi355x.h."""
+    _fields_ = ([(n, _i64) for n in ("T", "H", "Hp", "I", "max_padded")]
+                + [(n, _i32) for n in ("top_k", "E", "E_routed", "block_size_m", "tile_m", "exact_dot")]
+                + [(n, _P) for n in ("w13", "w13_scale", "w2", "w2_scale", "expert_map", "q1", "s1", "s1_pos",
+                                     "sorted_ids", "expert_ids", "ntpp", "workspace", "local_blocks", "hq", "hs", "D")])
+
+
+_LAYER = ctypes.POINTER(MoeLayer)
+
 # name -> (restype, argtypes); must match include/moe_mi355x.h
 SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "moe_quant_group128": (ctypes.c_int, [_P, _i64, _i64, _P, _P, _P]),
@@ -68,6 +80,12 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                                      _i64, _i32, _i32, _i64, _i32, _P, _P, _P]),
     "moe_gemm_w13_silu_quant_exact": (ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _i64, _i32, _i64,
                                                      _i64, _i32, _i32, _i64, _i32, _i32, _P, _P, _P]),
+    "moe_layer_local_blocks_bytes": (ctypes.c_int64, [_i64, _i64, _i32]),
+    "moe_layer_quant_align": (ctypes.c_int, [_LAYER, _P, _P, _P]),
+    "moe_layer_scales": (ctypes.c_int, [_LAYER, _P]),
+    "moe_layer_w13": (ctypes.c_int, [_LAYER, _P]),
+    "moe_layer_w2": (ctypes.c_int, [_LAYER, _P, _P]),
+    "moe_layer_reduce": (ctypes.c_int, [_LAYER, _P, _i64, _i64, _P, _P]),
     "moe_silu_and_mul": (ctypes.c_int, [_P, _i64, _i64, _P, _P]),
     "moe_reduce_topk": (ctypes.c_int, [_P, _i64, _i32, _i64, _P, _P]),
 }

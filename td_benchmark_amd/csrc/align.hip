@@ -33,6 +33,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "internal.hpp"
 #include "quant_group.hpp"
 
 namespace moe {
@@ -214,9 +215,20 @@ struct AlignArgs {
   int32_t* sorted;
   int32_t* eids;
   int32_t* ntpp;
+  int32_t* local;  // the lists of local blocks and slots, or null (see internal.hpp)
   int64_t max_padded;
-  int S, E, BM;
+  int S, E, BM, top_k;
 };
+
+// Bit i: the expert of token t's slot i is local.
+MOE_DEVICE int32_t local_slots(const int32_t* ids, const int32_t* expert_map, int E, int top_k, int t) {
+  uint32_t m = 0;
+  for (int i = 0; i < top_k && i < 32; ++i) {
+    const int x = ids[(int64_t)t * top_k + i];
+    if ((unsigned)x < (unsigned)E && expert_map[x] >= 0) m |= 1u << i;
+  }
+  return (int32_t)m;
+}
 
 constexpr int kAlignThreads = 512;
 constexpr int kAlignWaves = kAlignThreads / 64;
@@ -226,6 +238,7 @@ template <int IT>
 MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   __shared__ int32_t hist[kAlignMaxExperts];
   __shared__ int32_t wave_cnt[kAlignWaves], wave_before[kAlignWaves], wave_total[kAlignWaves];
+  __shared__ int32_t wave_lbefore[kAlignWaves], wave_ltotal[kAlignWaves];
   const int sh = __builtin_ctz(a.BM);  // BM is a power of two
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // wave w takes slots [w*IT*64, (w+1)*IT*64), 64 consecutive ones a step
@@ -243,28 +256,39 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   }
   if (lane == 0) wave_cnt[wave] = mine;
   __syncthreads();
-  int before = 0, total = 0;  // padded sizes of the experts before e, and of all
+  int before = 0, total = 0;    // padded sizes of the experts before e, and of all
+  int lbefore = 0, ltotal = 0;  // and of the local ones among them
   for (int x = tid; x < a.E; x += kAlignThreads) {
     const int p = (hist[x] + a.BM - 1) >> sh << sh;
     total += p;
     if (x < e) before += p;
+    if (a.local && a.expert_map[x] >= 0) {
+      ltotal += p;
+      if (x < e) lbefore += p;
+    }
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     before += __shfl_xor(before, o);
     total += __shfl_xor(total, o);
+    lbefore += __shfl_xor(lbefore, o);
+    ltotal += __shfl_xor(ltotal, o);
   }
   if (lane == 0) {
     wave_before[wave] = before;
     wave_total[wave] = total;
+    wave_lbefore[wave] = lbefore;
+    wave_ltotal[wave] = ltotal;
   }
   __syncthreads();
-  before = total = 0;
+  before = total = lbefore = ltotal = 0;
   int rank = 0;  // of this wave's first slot of e
 #pragma unroll
   for (int w = 0; w < kAlignWaves; ++w) {
     before += wave_before[w];
     total += wave_total[w];
+    lbefore += wave_lbefore[w];
+    ltotal += wave_ltotal[w];
     rank += w < wave ? wave_cnt[w] : 0;
   }
   const int cnt = hist[e];
@@ -279,17 +303,70 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   for (int i = cnt + tid; i < padded; i += kAlignThreads) a.sorted[before + i] = a.S;
   const int local = a.expert_map ? a.expert_map[e] : e;
   for (int i = tid; i < padded >> sh; i += kAlignThreads) a.eids[(before >> sh) + i] = local;
-  // the positions and blocks past ntpp, shared out over the workgroups
+  if (a.local && local >= 0) {
+    for (int i = tid; i < padded >> sh; i += kAlignThreads) {
+      local_blk(a.local)[(lbefore >> sh) + i] = (before >> sh) + i;
+      local_eid(a.local, a.max_padded, a.BM)[(lbefore >> sh) + i] = local;
+    }
+  }
+  // the tokens' local slots, and the positions and blocks past ntpp, shared out over the workgroups
+  if (a.local) {
+    int32_t* mask = local_mask(a.local, a.max_padded, a.BM);
+    for (int t = e * kAlignThreads + tid; t < a.S / a.top_k; t += a.E * kAlignThreads)
+      mask[t] = local_slots(a.ids, a.expert_map, a.E, a.top_k, t);
+  }
   for (int64_t i = total + (int64_t)e * kAlignThreads + tid; i < a.max_padded; i += (int64_t)a.E * kAlignThreads) {
     a.sorted[i] = a.S;
     if ((i & (a.BM - 1)) == 0) a.eids[i >> sh] = -1;
   }
-  if (e == 0 && tid == 0) *a.ntpp = total;
+  if (e == 0 && tid == 0) {
+    *a.ntpp = total;
+    if (a.local) *a.local = ltotal;
+  }
 }
 
 template <int IT>
 __global__ __launch_bounds__(kAlignThreads) void align_expert_kernel(AlignArgs a) {
   align_expert<IT>(a, blockIdx.x);
+}
+
+// The same lists after the three launches: the first workgroup compacts the
+// blocks whose (local) expert id is not -1, 1024 at a time, the others mark the
+// tokens' local slots.
+__global__ __launch_bounds__(1024) void local_blocks_kernel(const int32_t* __restrict__ ids, int64_t S, int E,
+                                                            int top_k, const int32_t* __restrict__ expert_map,
+                                                            const int32_t* __restrict__ eids,
+                                                            const int32_t* __restrict__ ntpp, int BM,
+                                                            int64_t max_padded, int32_t* __restrict__ local) {
+  __shared__ int32_t wave_cnt[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (blockIdx.x > 0) {
+    const int64_t t = (int64_t)(blockIdx.x - 1) * 1024 + tid;
+    if (t < S / top_k) local_mask(local, max_padded, BM)[t] = local_slots(ids, expert_map, E, top_k, (int)t);
+    return;
+  }
+  const int n = *ntpp / BM;
+  const uint64_t lt = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+  int done = 0;
+  for (int b0 = 0; b0 < n; b0 += 1024) {
+    const int b = b0 + tid;
+    const int e = b < n ? eids[b] : -1;
+    const uint64_t m = __ballot(e >= 0);
+    if (lane == 0) wave_cnt[wave] = __popcll(m);
+    __syncthreads();
+    int at = done;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      at += w < wave ? wave_cnt[w] : 0;
+      done += wave_cnt[w];
+    }
+    if (e >= 0) {
+      local_blk(local)[at + __popcll(m & lt)] = b;
+      local_eid(local, max_padded, BM)[at + __popcll(m & lt)] = e;
+    }
+    __syncthreads();
+  }
+  if (tid == 0) *local = done * BM;
 }
 
 // The same workgroups followed by those of the 1x128 activation quant, one
@@ -351,12 +428,14 @@ static void by_slots(int64_t S, F&& f) {
 
 static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
                       int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded,
-                      void* workspace, void* stream) {
+                      void* workspace, void* stream, int32_t* local = nullptr, int32_t top_k = 1) {
   const int arg_rc = align_args(topk_ids, S, E, BM, sorted_ids, expert_ids, ntpp, max_padded, true, workspace);
   if (arg_rc != kOk) return arg_rc;
+  if (!expert_map) local = nullptr;
   hipStream_t st = (hipStream_t)stream;
   if (S <= kAlignOneLaunchSlots) {
-    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, max_padded, (int)S, (int)E, (int)BM};
+    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local,
+                      max_padded, (int)S, (int)E, (int)BM, (int)top_k};
     by_slots(S, [&](auto it) {
       hipLaunchKernelGGL(align_expert_kernel<decltype(it)::value>, dim3((unsigned)E), dim3(kAlignThreads), 0, st, a);
     });
@@ -390,14 +469,18 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
                        topk_ids, S, (int)E, (int)BM, chunk_count, rank, off, cnt, expert_map,
                        sorted_ids, expert_ids, max_padded);
   }
+  if (local)
+    hipLaunchKernelGGL(local_blocks_kernel, dim3((unsigned)(1 + (S / top_k + 1023) / 1024)), dim3(1024), 0, st,
+                       topk_ids, S, (int)E, (int)top_k, expert_map, expert_ids, ntpp, (int)BM, max_padded, local);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
-extern "C" int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq, float* scales,
-                               const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
-                               const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp,
-                               int64_t max_padded, void* workspace, void* stream) {
+int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq, float* scales,
+                     const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
+                     int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded, void* workspace,
+                     int32_t* local, int32_t top_k, void* stream) {
   // both halves' arguments before either is launched
+  if (top_k <= 0) return kErrBadTopK;
   if (T < 0 || H < 0 || ldq < (H + 127) / 128 * 128) return kErrBadShape;
   if (T > 0 && H > 0) {
     if (!x_bf16 || !q_fp8 || !scales) return kErrNullPointer;
@@ -410,9 +493,12 @@ extern "C" int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q
       !quant_vectorised(x_bf16, H, q_fp8, ldq)) {
     const int qrc = moe_quant_group128_padded(x_bf16, T, H, q_fp8, ldq, scales, stream);
     if (qrc != kOk) return qrc;
-    return align_impl(topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp, max_padded, workspace, stream);
+    return align_impl(topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp, max_padded, workspace, stream,
+                      local, top_k);
   }
-  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, max_padded, (int)S, (int)E, (int)BM};
+  if (!expert_map) local = nullptr;
+  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local,
+                      max_padded, (int)S, (int)E, (int)BM, (int)top_k};
   const unsigned grid = (unsigned)(E + (q.n_chunks + kAlignThreads - 1) / kAlignThreads);
   by_slots(S, [&](auto it) {
     constexpr int IT = decltype(it)::value;
@@ -422,6 +508,14 @@ extern "C" int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q
       hipLaunchKernelGGL((quant_align_kernel<IT, false>), dim3(grid), dim3(kAlignThreads), 0, (hipStream_t)stream, a, q);
   });
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+extern "C" int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq, float* scales,
+                               const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
+                               const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp,
+                               int64_t max_padded, void* workspace, void* stream) {
+  return quant_align(x_bf16, T, H, q_fp8, ldq, scales, topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp,
+                     max_padded, workspace, nullptr, 1, stream);
 }
 
 extern "C" int moe_align_block_size(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,

@@ -19,6 +19,7 @@
 // bytes read and 2*N written per row; each thread owns 16 columns of one row
 // and keeps up to kDequantBatch ranks' loads in flight.
 #include "common.hpp"
+#include "internal.hpp"
 
 namespace moe {
 
@@ -28,22 +29,36 @@ constexpr int kMaxTopK = 32;
 // routed output and the shared expert's output (result + shared(hidden) of
 // schemes/vllm_tp.py:62-63 and schemes/vllm_ep.py:66-67), fused into the
 // reduce so the [T,H] sum is not re-read.
-template <int KMAX, bool ADD>
-__global__ __launch_bounds__(256) void reduce_topk_kernel(const uint16_t* __restrict__ D,
-                                                          const uint16_t* __restrict__ addend,
-                                                          uint16_t* __restrict__ y, int64_t T,
-                                                          int k, int64_t chunks_per_row) {
+// MAPPED: under an expert map the slots of experts on other devices have no
+// row in D; they are passed over (as zero rows would be, at none of the bytes).
+struct ReduceArgs {
+  const uint16_t* D;       // row stride ldd
+  const uint16_t* addend;  // row stride lda, or null
+  uint16_t* y;             // row stride 8 * cpr
+  int64_t ldd, lda, T;
+  int64_t cpr;             // 16 B chunks of an output row
+  const int32_t* mask;     // a word per token: bit i set = slot i has a row (MAPPED)
+  int k;
+};
+
+template <int KMAX, bool ADD, bool MAPPED>
+__global__ __launch_bounds__(256) void reduce_topk_kernel(ReduceArgs a) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= T * chunks_per_row) return;
-  const int64_t t = idx / chunks_per_row;
-  const int64_t cc = idx % chunks_per_row;
-  const int64_t H = chunks_per_row * 8;
+  const int64_t n = a.T * a.cpr;
+  if (idx >= n) return;
+  const int64_t t = n <= 0xFFFFFFFFll ? (int64_t)((uint32_t)idx / (uint32_t)a.cpr) : idx / a.cpr;
+  const int64_t cc = idx - t * a.cpr;
+  const int k = a.k;
+  const uint32_t here = MAPPED ? (uint32_t)a.mask[t] : ~0u;
   v4i rows[KMAX];
 #pragma unroll
-  for (int i = 0; i < KMAX; ++i)
-    if (i < k) rows[i] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(D + (t * k + i) * H + cc * 8));
+  for (int i = 0; i < KMAX; ++i) {
+    if constexpr (MAPPED) rows[i] = (v4i){0, 0, 0, 0};
+    if (i < k && (!MAPPED || (here >> i & 1)))
+      rows[i] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(a.D + (t * k + i) * a.ldd + cc * 8));
+  }
   v4i add = {0, 0, 0, 0};
-  if constexpr (ADD) add = *reinterpret_cast<const v4i*>(addend + t * H + cc * 8);
+  if constexpr (ADD) add = *reinterpret_cast<const v4i*>(a.addend + t * a.lda + cc * 8);
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int i = 0; i < KMAX; ++i) {
@@ -67,7 +82,7 @@ __global__ __launch_bounds__(256) void reduce_topk_kernel(const uint16_t* __rest
     }
     out[j] = (int)(lo | (hi << 16));
   }
-  __builtin_nontemporal_store(out, reinterpret_cast<v4i*>(y + t * H + cc * 8));
+  __builtin_nontemporal_store(out, reinterpret_cast<v4i*>(a.y + t * a.cpr * 8 + cc * 8));
 }
 
 constexpr int kMaxRanks = 64;
@@ -149,33 +164,29 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }  // nu
 
 
 
-static int launch_reduce(const void* D_bf16, const void* addend, int64_t T, int32_t top_k,
-                         int64_t H, void* y, void* stream) {
+template <int KMAX, bool ADD>
+static void launch_reduce(const ReduceArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)((a.T * a.cpr + 255) / 256));
+  if (a.mask)
+    hipLaunchKernelGGL((reduce_topk_kernel<KMAX, ADD, true>), grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((reduce_topk_kernel<KMAX, ADD, false>), grid, dim3(256), 0, st, a);
+}
+
+int reduce_topk(const void* D, int64_t ldd, const void* addend, int64_t lda, int64_t T, int32_t top_k, int64_t H,
+                const int32_t* mask, void* y, void* stream) {
   if (T < 0 || H < 0) return kErrBadShape;
   if (top_k <= 0 || top_k > kMaxTopK) return kErrBadTopK;
   if (T == 0 || H == 0) return kOk;
-  if (!D_bf16 || !y) return kErrNullPointer;
-  if (H % 8 != 0 || !aligned16(D_bf16) || !aligned16(y) || !aligned16(addend)) return kErrBadShape;
-  const int64_t cpr = H / 8;
-  const int64_t blocks = (T * cpr + 255) / 256;
+  if (!D || !y) return kErrNullPointer;
+  if (H % 8 != 0 || ldd % 8 != 0 || lda % 8 != 0 || !aligned16(D) || !aligned16(y) || !aligned16(addend))
+    return kErrBadShape;
+  const ReduceArgs a{(const uint16_t*)D, (const uint16_t*)addend, (uint16_t*)y, ldd, lda, T, H / 8, mask, (int)top_k};
   hipStream_t st = (hipStream_t)stream;
-  const uint16_t* d = (const uint16_t*)D_bf16;
-  const uint16_t* a = (const uint16_t*)addend;
-  uint16_t* out = (uint16_t*)y;
-  const dim3 grid((unsigned)blocks);
-  if (top_k <= 8) {
-    if (a)
-      hipLaunchKernelGGL((reduce_topk_kernel<8, true>), grid, dim3(256), 0, st, d, a, out, T, (int)top_k, cpr);
-    else
-      hipLaunchKernelGGL((reduce_topk_kernel<8, false>), grid, dim3(256), 0, st, d, a, out, T, (int)top_k, cpr);
-  } else {
-    if (a)
-      hipLaunchKernelGGL((reduce_topk_kernel<kMaxTopK, true>), grid, dim3(256), 0, st, d, a, out, T,
-                         (int)top_k, cpr);
-    else
-      hipLaunchKernelGGL((reduce_topk_kernel<kMaxTopK, false>), grid, dim3(256), 0, st, d, a, out, T,
-                         (int)top_k, cpr);
-  }
+  if (top_k <= 8)
+    addend ? launch_reduce<8, true>(a, st) : launch_reduce<8, false>(a, st);
+  else
+    addend ? launch_reduce<kMaxTopK, true>(a, st) : launch_reduce<kMaxTopK, false>(a, st);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
@@ -185,13 +196,13 @@ using namespace moe;
 
 extern "C" int moe_reduce_topk(const void* D_bf16, int64_t T, int32_t top_k, int64_t H, void* y,
                                void* stream) {
-  return launch_reduce(D_bf16, nullptr, T, top_k, H, y, stream);
+  return reduce_topk(D_bf16, H, nullptr, 0, T, top_k, H, nullptr, y, stream);
 }
 
 extern "C" int moe_reduce_topk_add(const void* D_bf16, const void* addend_bf16, int64_t T,
                                    int32_t top_k, int64_t H, void* y, void* stream) {
   if (T > 0 && H > 0 && !addend_bf16) return kErrNullPointer;
-  return launch_reduce(D_bf16, addend_bf16, T, top_k, H, y, stream);
+  return reduce_topk(D_bf16, H, addend_bf16, H, T, top_k, H, nullptr, y, stream);
 }
 
 extern "C" int moe_silu_and_mul(const void* c_bf16, int64_t R, int64_t I, void* h_bf16,

@@ -79,6 +79,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "internal.hpp"
 #include "mfma_frag.hpp"
 
 #define MOE_LDS(p) ((__attribute__((address_space(3))) void*)(p))
@@ -148,6 +149,10 @@ struct GemmArgs {
   const int32_t* sorted;   // [max_padded]
   const int32_t* eids;     // [max_blocks]
   const int32_t* ntpp;     // [1]
+  // Expert parallelism (else null): the align blocks of local experts in
+  // ascending order; eids and ntpp then describe this list, and the other
+  // blocks are no part of the launch.
+  const int32_t* blk;
   const float* topk_w;     // [S] or null
   uint16_t* C;             // bf16 [S, N]            (plain epilogue)
   uint8_t* hq;             // fp8 [max_padded, I]    (fused epilogue)
@@ -859,7 +864,8 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   const int64_t u = by_col ? in_grp % units : in_grp / gsz;  // row tile of the run
   const int64_t base = run / units, n_short = units - run % units;  // n_short tiles of `base` blocks
   const int64_t b = b0 + (u < n_short ? u * base : n_short * base + (u - n_short) * (base + 1));
-  const int64_t pos0 = b * vb;                  // sorted position of tile row 0
+  // sorted position of tile row 0 (a run's blocks are consecutive in the listed order too)
+  const int64_t pos0 = (g.blk ? ((int64_t)g.blk[b >> vsh] << vsh) + (b & ((1 << vsh) - 1)) : b) * vb;
   // tile rows that belong to this run (the rest are not read or written)
   const int rows_avail = (int)((u < n_short ? base : base + 1) * vb);
 
@@ -998,7 +1004,7 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 // weight tile is then fetched once per 256 rows instead of once per block) and
 // BM otherwise.  Returns -1 for a tile_m that is not a supported block size and
 // a multiple of BM.
-static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int32_t E) {
+static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int64_t E) {
   if (tile_m == 0) return S >= 160 * (int64_t)E ? 256 : BM;
   if (!block_m_ok(tile_m) || tile_m < BM || tile_m % BM != 0) return -1;
   return tile_m;
@@ -1016,17 +1022,17 @@ using namespace moe;
 
 // The plain grouped GEMM on dense operands; A_scale row-major by A row, or
 // K-major by sorted position when scales_by_pos (A then by position too).
-static int plain_gemm(const void* A, const float* A_scale, const void* B, const float* B_scale,
-                      const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* ntpp,
-                      const float* topk_weights, int64_t S, int32_t top_k, int32_t a_by_pos, int64_t N,
-                      int64_t K, int32_t E, int32_t BM, int64_t max_padded, int32_t tile_order,
-                      int32_t tile_m, bool scales_by_pos, void* C, void* stream) {
+int moe::plain_gemm(const void* A, const float* A_scale, const void* B, const float* B_scale,
+                    const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* ntpp,
+                    const float* topk_weights, int64_t S, int32_t top_k, int32_t a_by_pos, int64_t N,
+                    int64_t K, int32_t E, int32_t BM, int64_t max_padded, int32_t tile_order,
+                    int32_t tile_m, bool scales_by_pos, void* C, void* stream, LocalBlocks local) {
   if (S < 0 || N <= 0 || K <= 0 || max_padded < 0) return kErrBadShape;
   if (N % 128 != 0 || K % 128 != 0 || K > 128 * kMaxKB) return kErrBadShape;
   if (top_k <= 0) return kErrBadTopK;
   if (E <= 0) return kErrBadExperts;
   if (!block_m_ok(BM)) return kErrBadBlockSize;
-  const int TM = resolve_tile_m(tile_m, BM, S, E);
+  const int TM = resolve_tile_m(tile_m, BM, S, local.E_routed ? local.E_routed : E);
   if (TM < 0) return kErrBadBlockSize;
   if (tile_order < 0 || tile_order > 2) return kErrBadShape;
   if (max_padded == 0 || S == 0) return kOk;
@@ -1058,6 +1064,7 @@ static int plain_gemm(const void* A, const float* A_scale, const void* B, const 
   g.tile_order = tile_order;
   dense_strides(g);
   if (scales_by_pos) g.as_pos_ld = max_padded;
+  g.blk = local.blocks;
   return dispatch_gemm<false>(TM, g, (hipStream_t)stream);
 }
 
@@ -1210,16 +1217,17 @@ extern "C" int moe_grouped_gemm_k_split(const void* A, const float* A_scale, int
 // The fused W13 GEMM; scales row-major (A_scale by token, hs by position), or
 // both K-major by sorted position when scales_by_pos; exact dots on the bf16
 // matrix core when exact.
-static int w13_gemm(const void* Aq, const float* A_scale, const void* W13, const float* W13_scale,
-                    const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* ntpp, int64_t S,
-                    int32_t top_k, int64_t H, int64_t I, int32_t E, int32_t BM, int64_t max_padded,
-                    int32_t tile_m, bool scales_by_pos, bool exact, void* hq, float* hs, void* stream) {
+int moe::w13_gemm(const void* Aq, const float* A_scale, const void* W13, const float* W13_scale,
+                  const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* ntpp, int64_t S,
+                  int32_t top_k, int64_t H, int64_t I, int32_t E, int32_t BM, int64_t max_padded,
+                  int32_t tile_m, bool scales_by_pos, bool exact, void* hq, float* hs, void* stream,
+                  LocalBlocks local) {
   if (S < 0 || H <= 0 || I <= 0 || max_padded < 0) return kErrBadShape;
   if (H % 128 != 0 || I % 128 != 0 || H > 128 * kMaxKB) return kErrBadShape;
   if (top_k <= 0) return kErrBadTopK;
   if (E <= 0) return kErrBadExperts;
   if (!block_m_ok(BM)) return kErrBadBlockSize;
-  int TM = resolve_tile_m(tile_m, BM, S, E);
+  int TM = resolve_tile_m(tile_m, BM, S, local.E_routed ? local.E_routed : E);
   if (TM < 0) return kErrBadBlockSize;
   // The exact-dot form runs a 256-row tile as two 128-row bodies one after the
   // other; its automatic tile is 128 rows instead (separate 128-row workgroups
@@ -1260,6 +1268,7 @@ static int w13_gemm(const void* Aq, const float* A_scale, const void* W13, const
   g.E = E;
   dense_strides(g);
   if (scales_by_pos) g.as_pos_ld = g.hs_pos_ld = max_padded;
+  g.blk = local.blocks;
   return exact ? dispatch_gemm<true, true>(TM, g, (hipStream_t)stream) : dispatch_gemm<true>(TM, g, (hipStream_t)stream);
 }
 

@@ -1,0 +1,49 @@
+// Host functions shared by the C entry points and the layer (layer.hip).
+#pragma once
+
+#include "common.hpp"
+
+namespace moe {
+
+// The list of local blocks that align writes under an expert map (see
+// moe_layer's local_blocks): blocks == null without one.  E_routed: the experts
+// the slots are spread over, for the choice of the tile height (0: E).
+struct LocalBlocks {
+  const int32_t* blocks = nullptr;
+  int64_t E_routed = 0;
+};
+
+// local_blocks holds [0] local blocks * BM, then the blocks, then their local
+// expert ids, then a word per token whose bit i says that slot i's expert is local.
+inline const int32_t* local_rows(const int32_t* l) { return l; }
+template <class T>
+MOE_HOST_DEVICE T* local_blk(T* l) { return l + 1; }
+template <class T>
+MOE_HOST_DEVICE T* local_eid(T* l, int64_t max_padded, int32_t BM) { return l + 1 + (max_padded + BM - 1) / BM; }
+
+template <class T>
+MOE_HOST_DEVICE T* local_mask(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 2 * ((max_padded + BM - 1) / BM); }
+
+int plain_gemm(const void* A, const float* A_scale, const void* B, const float* B_scale, const int32_t* sorted_ids,
+               const int32_t* expert_ids, const int32_t* ntpp, const float* topk_weights, int64_t S, int32_t top_k,
+               int32_t a_by_pos, int64_t N, int64_t K, int32_t E, int32_t BM, int64_t max_padded, int32_t tile_order,
+               int32_t tile_m, bool scales_by_pos, void* C, void* stream, LocalBlocks local = {});
+
+int w13_gemm(const void* Aq, const float* A_scale, const void* W13, const float* W13_scale, const int32_t* sorted_ids,
+             const int32_t* expert_ids, const int32_t* ntpp, int64_t S, int32_t top_k, int64_t H, int64_t I, int32_t E,
+             int32_t BM, int64_t max_padded, int32_t tile_m, bool scales_by_pos, bool exact, void* hq, float* hs,
+             void* stream, LocalBlocks local = {});
+
+// T == 0: align alone.  local: the lists to write under an expert map, or null;
+// top_k: the slots of a token (for its mask).
+int quant_align(const void* x, int64_t T, int64_t H, void* q, int64_t ldq, float* scales, const int32_t* topk_ids,
+                int64_t S, int32_t E, int32_t BM, const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids,
+                int32_t* ntpp, int64_t max_padded, void* workspace, int32_t* local, int32_t top_k, void* stream);
+
+// The top-k sum of rows of H columns in D (row stride ldd) into y (row stride
+// H); addend rows (row stride lda) or null; with mask (a word per token) the
+// slots without a set bit are passed over.
+int reduce_topk(const void* D, int64_t ldd, const void* addend, int64_t lda, int64_t T, int32_t top_k, int64_t H,
+                const int32_t* mask, void* y, void* stream);
+
+}  // namespace moe

@@ -14,7 +14,7 @@ from typing import Any
 
 import torch
 
-from ._lib import check, lib
+from ._lib import MoeLayer, check, lib
 
 FP8 = torch.float8_e4m3fn
 BLOCK_SHAPE = [128, 128]
@@ -758,7 +758,11 @@ class FusedExpertsRunner:
     on the bf16 matrix core, about twice the matrix-core time of the FP8
     instruction, whose in-group product truncation otherwise moves about
     0.2 % of the intermediate codes.  W2 and every other stage are the same
-    in both modes, and a shared expert follows the layer's mode."""
+    in both modes, and a shared expert follows the layer's mode.
+
+    With ``expert_map`` (global -> local expert id or -1) the GEMMs run over
+    the local experts' blocks only: ``hq``, ``hs`` and ``D`` are written for
+    the slots of local experts, and the top-k sum takes the others as zero."""
 
     def __init__(self, w13: torch.Tensor, w13_scale: torch.Tensor, w2: torch.Tensor,
                  w2_scale: torch.Tensor, num_tokens: int, top_k: int, block_size_m: int | None = None,
@@ -776,7 +780,19 @@ class FusedExpertsRunner:
         self.Hp = Hp = _blocks128(H) * 128
         w13, w2 = _pad_fp8(w13, 2, Hp), _pad_fp8(w2, 1, Hp)
         self.S = num_tokens * top_k
-        self.BM = block_size_m or get_moe_config(num_tokens, E, top_k)["BLOCK_SIZE_M"]
+        # Expert parallelism: align over the global experts, GEMMs over the
+        # blocks of the local ones.
+        self.expert_map = None
+        n_align = E
+        if expert_map is not None:
+            self.expert_map = expert_map.to(device=w13.device, dtype=torch.int32).contiguous()
+            n_align = int(global_num_experts or self.expert_map.numel())
+            if self.expert_map.numel() != n_align:
+                raise ValueError("expert_map must have global_num_experts entries")
+        elif global_num_experts not in (None, -1, E):
+            raise ValueError("global_num_experts != local experts needs an expert_map")
+        # the slots are spread over all n_align experts, local or not
+        self.BM = block_size_m or get_moe_config(num_tokens, n_align, top_k)["BLOCK_SIZE_M"]
         if self.BM not in SUPPORTED_BLOCK_M:
             raise ValueError(f"block_size_m must be one of {SUPPORTED_BLOCK_M}")
         # GEMM workgroup tile rows (0 = automatic; never changes the results)
@@ -793,22 +809,11 @@ class FusedExpertsRunner:
         dev = w13.device
         self.q1 = torch.empty((self.T, Hp), dtype=FP8, device=dev)
         self.s1 = torch.empty((self.T, Hp // 128), dtype=torch.float32, device=dev)
-        # Expert parallelism: align over the global experts, GEMMs over the
-        # local ones (blocks of non-local experts are -1 and produce zeros).
-        self.expert_map = None
-        n_align = E
-        if expert_map is not None:
-            self.expert_map = expert_map.to(device=dev, dtype=torch.int32).contiguous()
-            n_align = int(global_num_experts or self.expert_map.numel())
-            if self.expert_map.numel() != n_align:
-                raise ValueError("expert_map must have global_num_experts entries")
-        elif global_num_experts not in (None, -1, E):
-            raise ValueError("global_num_experts != local experts needs an expert_map")
         self.align = AlignBuffers(self.S, n_align, self.BM, dev)
         mp = max(self.align.max_padded, 1)
         self.hq = torch.empty((mp, self.I), dtype=FP8, device=dev)
         if scales_by_position is None:
-            scales_by_position = gemm_tile_rows(self.BM, self.S, self.E, self.tile_m) >= 128
+            scales_by_position = gemm_tile_rows(self.BM, self.S, n_align, self.tile_m) >= 128
         self.scales_by_position = bool(scales_by_position)
         if self.scales_by_position:
             self.s1_pos = torch.empty((Hp // 128, mp), dtype=torch.float32, device=dev)
@@ -817,13 +822,30 @@ class FusedExpertsRunner:
         else:
             self.hs = torch.empty((mp, self.I // 128), dtype=torch.float32, device=dev)
         self.D = torch.empty((max(self.S, 1), Hp), dtype=torch.bfloat16, device=dev)
+        self.local_blocks = None
+        if self.expert_map is not None:
+            # written at the positions of local experts only: elsewhere what a run of zero rows leaves
+            self.hq.view(torch.uint8).zero_()
+            (self.hs_pos if self.scales_by_position else self.hs).fill_(1e-12)
+            n = int(lib().moe_layer_local_blocks_bytes(self.T, self.align.max_padded, self.BM))
+            self.local_blocks = torch.empty(n // 4, dtype=torch.int32, device=dev)
         if out is not None:
             _need(out, "out", torch.bfloat16)
             if tuple(out.shape) != (self.T, H):
                 raise ValueError(f"out must be [{self.T}, {H}]")
         self.y = out if out is not None else torch.empty((self.T, H), dtype=torch.bfloat16, device=dev)
-        # the top-k sum at the padded width, whose first H columns are y
-        self.y_pad = self.y if Hp == H else torch.empty((self.T, Hp), dtype=torch.bfloat16, device=dev)
+        # An H or an output the sum cannot write in place: the sum at the padded width, whose first H columns are y.
+        in_place = Hp == H or (H % 8 == 0 and self.y.data_ptr() % 16 == 0)
+        self.y_pad = self.y if in_place else torch.empty((self.T, Hp), dtype=torch.bfloat16, device=dev)
+        a = self.align
+        self._layer = MoeLayer(
+            T=self.T, H=H, Hp=Hp, I=self.I, max_padded=a.max_padded, top_k=top_k, E=E, E_routed=n_align,
+            block_size_m=self.BM, tile_m=self.tile_m, exact_dot=int(self.exact_dot), w13=_ptr(w13),
+            w13_scale=_ptr(w13_scale), w2=_ptr(w2), w2_scale=_ptr(w2_scale), expert_map=_ptr(self.expert_map),
+            q1=_ptr(self.q1), s1=_ptr(self.s1), s1_pos=_ptr(self.s1_pos) if self.scales_by_position else None,
+            sorted_ids=_ptr(a.sorted_ids), expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp),
+            workspace=_ptr(a.workspace), local_blocks=_ptr(self.local_blocks), hq=_ptr(self.hq),
+            hs=_ptr(self.hs_pos if self.scales_by_position else self.hs), D=_ptr(self.D))
 
     def _need_hidden(self, hidden: torch.Tensor) -> None:
         _need(hidden, "hidden_states", torch.bfloat16)
@@ -840,59 +862,32 @@ class FusedExpertsRunner:
                                                   _ptr(self.s1), _stream()), "moe_quant_group128_padded")
 
     def stage_align(self, topk_ids: torch.Tensor) -> None:
-        self.align.run(topk_ids, self.expert_map)
+        self.align.need_ids(topk_ids, self.expert_map)
+        check(lib().moe_layer_quant_align(self._layer, None, _ptr(topk_ids), _stream()), "moe_layer_quant_align")
+
+    def stage_quant_align(self, hidden: torch.Tensor, topk_ids: torch.Tensor) -> None:
+        """stage_quant and stage_align, which do not depend on each other, in
+        one launch where both are small."""
+        self._need_hidden(hidden)
+        self.align.need_ids(topk_ids, self.expert_map)
+        check(lib().moe_layer_quant_align(self._layer, _ptr(hidden), _ptr(topk_ids), _stream()),
+              "moe_layer_quant_align")
 
     def stage_scales(self) -> None:
         """The activation scales K-major by sorted position for the W13 GEMM
         (nothing to do on the row-major path)."""
         if self.scales_by_position:
-            a = self.align
-            check(lib().moe_gather_scales_by_position(_ptr(self.s1), self.T, self.Hp // 128, _ptr(a.sorted_ids),
-                                                      _ptr(a.ntpp), self.S, self.top_k, a.max_padded,
-                                                      _ptr(self.s1_pos), _stream()), "moe_gather_scales_by_position")
+            check(lib().moe_layer_scales(self._layer, _stream()), "moe_layer_scales")
 
     def stage_w13(self) -> None:
-        a = self.align
-        if self.exact_dot:
-            by_pos = self.scales_by_position
-            check(lib().moe_gemm_w13_silu_quant_exact(_ptr(self.q1), _ptr(self.s1_pos if by_pos else self.s1),
-                                                      _ptr(self.w13), _ptr(self.w13_scale), _ptr(a.sorted_ids),
-                                                      _ptr(a.expert_ids), _ptr(a.ntpp), self.S, self.top_k,
-                                                      self.Hp, self.I, self.E, self.BM, a.max_padded, self.tile_m,
-                                                      int(by_pos), _ptr(self.hq),
-                                                      _ptr(self.hs_pos if by_pos else self.hs), _stream()),
-                  "moe_gemm_w13_silu_quant_exact")
-            return
-        if self.scales_by_position:
-            check(lib().moe_gemm_w13_silu_quant_pos(_ptr(self.q1), _ptr(self.s1_pos), _ptr(self.w13),
-                                                    _ptr(self.w13_scale), _ptr(a.sorted_ids), _ptr(a.expert_ids),
-                                                    _ptr(a.ntpp), self.S, self.top_k, self.Hp, self.I, self.E,
-                                                    self.BM, a.max_padded, self.tile_m, _ptr(self.hq),
-                                                    _ptr(self.hs_pos), _stream()), "moe_gemm_w13_silu_quant_pos")
-            return
-        check(lib().moe_gemm_w13_silu_quant_tiled(_ptr(self.q1), _ptr(self.s1), _ptr(self.w13),
-                                                  _ptr(self.w13_scale), _ptr(a.sorted_ids), _ptr(a.expert_ids),
-                                                  _ptr(a.ntpp), self.S, self.top_k, self.Hp, self.I, self.E,
-                                                  self.BM, a.max_padded, self.tile_m, _ptr(self.hq),
-                                                  _ptr(self.hs), _stream()), "moe_gemm_w13_silu_quant")
+        self._layer.exact_dot = int(self.exact_dot)
+        check(lib().moe_layer_w13(self._layer, _stream()), "moe_layer_w13")
 
     def stage_w2(self, topk_weights: torch.Tensor) -> None:
         _need(topk_weights, "topk_weights", torch.float32)
         if topk_weights.numel() != self.S:
             raise ValueError(f"topk_weights has {topk_weights.numel()} entries for {self.S} slots")
-        a = self.align
-        if self.scales_by_position:
-            check(lib().moe_grouped_gemm_pos(_ptr(self.hq), _ptr(self.hs_pos), _ptr(self.w2), _ptr(self.w2_scale),
-                                             _ptr(a.sorted_ids), _ptr(a.expert_ids), _ptr(a.ntpp),
-                                             _ptr(topk_weights), self.S, self.Hp, self.I, self.E, self.BM,
-                                             a.max_padded, self.tile_m, _ptr(self.D), _stream()),
-                  "moe_grouped_gemm_pos")
-            return
-        check(lib().moe_grouped_gemm_tiled(_ptr(self.hq), _ptr(self.hs), _ptr(self.w2), _ptr(self.w2_scale),
-                                           _ptr(a.sorted_ids), _ptr(a.expert_ids), _ptr(a.ntpp),
-                                           _ptr(topk_weights), self.S, 1, 1, self.Hp, self.I, self.E, self.BM,
-                                           a.max_padded, 0, self.tile_m, _ptr(self.D), _stream()),
-              "moe_grouped_gemm")
+        check(lib().moe_layer_w2(self._layer, _ptr(topk_weights), _stream()), "moe_layer_w2")
 
     def stage_shared(self) -> None:
         """The shared expert on the layer's own FP8 input (no second quant),
@@ -902,21 +897,16 @@ class FusedExpertsRunner:
             self.shared_out = self.shared(self.q1, self.s1)
 
     def stage_reduce(self) -> None:
-        addend = None
+        addend, ld = None, 0
         if self.shared is not None:  # the shared expert's rows at the padded width
-            addend = self.shared.out[: self.T] if self.Hp != self.H else self.shared_out
-        moe_sum(self.D[: self.S], self.y_pad, self.top_k, addend=addend)
+            addend, ld = self.shared.out, self.Hp
+        check(lib().moe_layer_reduce(self._layer, _ptr(addend), ld, self.y_pad.shape[1], _ptr(self.y_pad), _stream()),
+              "moe_layer_reduce")
         if self.y_pad is not self.y:
             self.y.copy_(self.y_pad[:, : self.H])
 
     def run(self, hidden: torch.Tensor, topk_weights: torch.Tensor, topk_ids: torch.Tensor) -> torch.Tensor:
-        self._need_hidden(hidden)
-        a = self.align
-        a.need_ids(topk_ids, self.expert_map)
-        check(lib().moe_quant_align(_ptr(hidden), self.T, self.H, _ptr(self.q1), self.Hp, _ptr(self.s1),
-                                    _ptr(topk_ids), self.S, a.E, self.BM, _ptr(self.expert_map), _ptr(a.sorted_ids),
-                                    _ptr(a.expert_ids), _ptr(a.ntpp), a.max_padded, _ptr(a.workspace), _stream()),
-              "moe_quant_align")
+        self.stage_quant_align(hidden, topk_ids)
         self.stage_scales()
         self.stage_w13()
         self.stage_w2(topk_weights)
