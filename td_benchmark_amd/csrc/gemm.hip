@@ -98,35 +98,47 @@ constexpr int64_t kColMajorK = 8192;
 // reads a result that is complete, without hazard waits.
 constexpr int kScaleLag = 2;
 
-template <int BM>
+// GROUPS: 128-row weight groups of a tile (2, or 1 in the narrow form of plain
+// launches); DEEP: the form for launches whose tiles all run at once, one
+// workgroup per CU with as deep a ring as the LDS holds, filled by waves that do
+// nothing else (see flat_gemm_body).
+template <int BM_, int GROUPS_ = 2, bool DEEP_ = false>
 struct Tile {
-  static constexpr int NW = BM >= 32 ? 8 : 4;     // waves per workgroup (2 per SIMD at 8)
+  static constexpr int BM = BM_;
+  static constexpr int GROUPS = GROUPS_;
+  static_assert(GROUPS == 2 || (DEEP_ && BM <= 64), "narrow tiles are deep and short");
+  static constexpr bool DEEP = DEEP_;
+  static constexpr int NW = DEEP || BM >= 32 ? 8 : 4;  // waves per workgroup (2 per SIMD at 8)
   static constexpr int THREADS = 64 * NW;
-  // waves along M: 4 x 2 waves of 64 x 128 at BM = 256 (fewer LDS bytes per MFMA)
-  static constexpr int WM = BM == 256 ? 4 : ((NW == 8 || BM == 128) ? 2 : 1);
+  static constexpr int CW = DEEP ? 4 : NW;  // waves that compute: the first ones
+  static constexpr int PW = DEEP ? 4 : NW;  // waves that issue the loads: the last ones
+  // compute waves along M: 4 x 2 waves of 64 x 128 at BM = 256 (fewer LDS bytes per MFMA)
+  static constexpr int WM = BM == 256 ? 4 : ((CW == 8 || BM == 128) ? 2 : 1);
   // LDS ring depth: three 64 KiB stages of the 256-row tile exceed 160 KiB;
   // the 34 KiB stages of the 16-row tile (weight streaming) fit four; the
   // 32-row tile runs two workgroups per CU with two 36 KiB stages each, so one
   // workgroup's pipeline fill and epilogue overlap the other's weight stream
-  static constexpr int KS = (BM == 256 || BM == 32) ? 2 : (BM == 16 ? 4 : 3);
-  static constexpr int WG_PER_CU = BM == 32 ? 2 : 1;
-  static constexpr int WN = NW / WM;              // waves along N
+  static constexpr int KS = GROUPS == 1 ? (BM == 64 ? 6 : 7)
+                            : BM == 256 || (BM == 32 && !DEEP_) ? 2
+                                                                : (BM <= 32 ? 4 : 3);
+  static constexpr int WG_PER_CU = BM == 32 && !DEEP_ ? 2 : 1;
+  static constexpr int WN = CW / WM;              // compute waves along N
   static constexpr int RS = BM / WM / 16;         // 16-row subtiles per wave
   static constexpr int CS = 8 / WN;               // 16-col subtiles per wave per group
   static constexpr int A_BYTES = BM * 128;
-  static constexpr int B_BYTES = 256 * 128;
+  static constexpr int B_BYTES = GROUPS * 128 * 128;
   static constexpr int STAGE = A_BYTES + B_BYTES;
   static constexpr int NA = BM / 8;               // 1 KiB A DMA instructions per stage
-  static constexpr int NB = 32;                   // 1 KiB B DMA instructions per stage
+  static constexpr int NB = GROUPS * 16;          // 1 KiB B DMA instructions per stage
   static constexpr int NS = (BM + 63) / 64;       // 256 B A-scale DMA instructions per stage
-  static constexpr int NA_W = (NA + NW - 1) / NW; // A instructions of the busiest wave
-  static constexpr int NB_W = NB / NW;            // B instructions per wave
-  static constexpr int na(int w) { return w < NA ? (NA - w + NW - 1) / NW : 0; }
-  static constexpr int ns(int w) { return (NW - 1 - w) < NS ? 1 : 0; }  // the last waves issue scales
+  static constexpr int NA_W = (NA + PW - 1) / PW; // A instructions of the busiest loading wave
+  static constexpr int NB_W = NB / PW;            // B instructions per loading wave
+  static constexpr int na(int w) { return w < NA ? (NA - w + PW - 1) / PW : 0; }
+  static constexpr int ns(int w) { return (PW - 1 - w) < NS ? 1 : 0; }  // the last waves issue scales
   static constexpr int cnt(int w) { return na(w) + NB_W + ns(w); }
   static constexpr int vm_min() {
     int m = cnt(0);
-    for (int w = 1; w < NW; ++w) m = cnt(w) < m ? cnt(w) : m;
+    for (int w = 1; w < PW; ++w) m = cnt(w) < m ? cnt(w) : m;
     return m;
   }
   // loads of one stage per wave that may stay in flight while the older stage is consumed
@@ -134,9 +146,10 @@ struct Tile {
   static constexpr int OFF_SA = KS * STAGE;
   static constexpr int OFF_SB = OFF_SA + KS * NS * 256;
   static constexpr int OFF_RED = OFF_SB + 2 * kMaxKB * 4;
-  static constexpr int OFF_ROW = OFF_RED + WN * BM * 4;  // per-row slot id and routed weight
-  static constexpr int LDS_BYTES = OFF_ROW + BM * 8;
-  static_assert(BM * 512 <= OFF_SA, "bf16 output staging must fit in the operand ring");
+  static constexpr int OFF_ROW = OFF_RED + WN * BM * 4;   // per-row slot id
+  static constexpr int OFF_W = OFF_ROW + BM * 4;          // per-row routed weight, 64 rows a load
+  static constexpr int LDS_BYTES = OFF_W + NS * 256;
+  static_assert(BM * GROUPS * 256 <= OFF_SA, "bf16 output staging must fit in the operand ring");
   static_assert(LDS_BYTES * WG_PER_CU <= 160 * 1024, "LDS budget");
   static_assert(VM * (KS - 2) < 64, "vmcnt immediate");
 };
@@ -162,6 +175,7 @@ struct GemmArgs {
   int64_t K;
   int64_t I;
   int64_t max_blocks;      // (virtual) blocks that fit in max_padded
+  int64_t max_padded;      // entries of sorted
   int64_t n_tiles;         // 256-column n-tiles
   int bma;                 // rows per align block (block_size_m); a tile spans BM / bma of them
   // Exact-dot launches only: the tile map counts virtual blocks of bma >> vshift
@@ -245,10 +259,14 @@ MOE_DEVICE void dma4(const uint8_t* base, uint32_t off, uint8_t* lds) {
 #pragma clang diagnostic pop
 
 // Column scale groups of n-tile j: W13 gate group j and up group I/128 + j; the
-// plain GEMM groups 2j and 2j+1 (the second absent past N).
-template <bool FUSED>
+// plain GEMM groups 2j and 2j+1 (the second absent past N), or group j alone in
+// its narrow form.
+template <bool FUSED, int GROUPS = 2>
 MOE_DEVICE void groups_of(const GemmArgs& g, int64_t j, int64_t& g0, int64_t& g1, bool& g1_store) {
-  if (FUSED) {
+  if (GROUPS == 1) {
+    g0 = g1 = j;
+    g1_store = false;
+  } else if (FUSED) {
     g0 = j;
     g1 = g.I / 128 + j;
     g1_store = true;
@@ -271,12 +289,12 @@ MOE_DEVICE void groups_of(const GemmArgs& g, int64_t j, int64_t& g0, int64_t& g1
 // Staging rows XOR their 16-byte chunk index with the row (mod 8 for codes,
 // mod 16 for bf16), so the 16 tokens a write instruction covers hit distinct
 // bank groups.
-template <int BM, bool FUSED>
-__device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[Tile<BM>::RS][2][Tile<BM>::CS],
+template <class T, bool FUSED>
+__device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[T::RS][T::GROUPS][T::CS],
                                               int64_t j, int64_t pos0, int rows_avail, int64_t g0,
                                               int64_t g1, bool g1_store, uint8_t* staging, float* smRed,
                                               const int32_t* smSlot, const float* smW) {
-  using T = Tile<BM>;
+  constexpr int BM = T::BM, GROUPS = T::GROUPS;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -286,32 +304,37 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[Tile
   const int col_base = wn * T::CS * 16;
   const int fr = lane & 15;
   const int kseg = lane >> 4;
+  // whether this wave holds results (every wave, where all compute)
+  const bool holds = T::CW == T::NW || wave < T::CW;
   if constexpr (FUSED) {
-    float pmax[T::RS];
+    if (holds) {
+      float pmax[T::RS];
 #pragma unroll
-    for (int r = 0; r < T::RS; ++r) pmax[r] = 0.0f;
+      for (int r = 0; r < T::RS; ++r) pmax[r] = 0.0f;
 #pragma unroll
-    for (int r = 0; r < T::RS; ++r)
+      for (int r = 0; r < T::RS; ++r)
 #pragma unroll
-      for (int c = 0; c < T::CS; ++c)
+        for (int c = 0; c < T::CS; ++c)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const uint32_t gu = pack_bf16x2(acc[r][0][c][v], acc[r][1][c][v]);
-          const float h = silu_mul_bf16(lo_bf16(gu), hi_bf16(gu));
-          acc[r][0][c][v] = h;
-          pmax[r] = fmaxf(pmax[r], fabsf(h));
-        }
+          for (int v = 0; v < 4; ++v) {
+            const uint32_t gu = pack_bf16x2(acc[r][0][c][v], acc[r][1][c][v]);
+            const float h = silu_mul_bf16(lo_bf16(gu), hi_bf16(gu));
+            acc[r][0][c][v] = h;
+            pmax[r] = fmaxf(pmax[r], fabsf(h));
+          }
 #pragma unroll
-    for (int r = 0; r < T::RS; ++r) {
-      float m = pmax[r];
-      m = fmaxf(m, __shfl_xor(m, 16));
-      m = fmaxf(m, __shfl_xor(m, 32));
-      if (kseg == 0) smRed[wn * BM + row_base + r * 16 + fr] = m;
+      for (int r = 0; r < T::RS; ++r) {
+        float m = pmax[r];
+        m = fmaxf(m, __shfl_xor(m, 16));
+        m = fmaxf(m, __shfl_xor(m, 32));
+        if (kseg == 0) smRed[wn * BM + row_base + r * 16 + fr] = m;
+      }
     }
     __syncthreads();
     uint8_t* stage_out = staging;  // [BM][128] fp8 codes
 #pragma unroll
     for (int r = 0; r < T::RS; ++r) {
+      if (!holds) break;
       const int row = row_base + r * 16 + fr;
       float amax = 0.0f;
 #pragma unroll
@@ -333,15 +356,16 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[Tile
           *reinterpret_cast<const v4i*>(stage_out + row * 128 + ((cc ^ (row & 7)) << 4));
     }
   } else {
-    // Both 128-column groups staged at once as [BM][256] bf16, then each row's
-    // chunks (up to 512 B) written by slot.
+    // All 128-column groups staged at once as [BM][GROUPS * 128] bf16, then each
+    // row's chunks (up to 512 B) written by slot.
     uint16_t* stage_out = reinterpret_cast<uint16_t*>(staging);
 #pragma unroll
     for (int r = 0; r < T::RS; ++r) {
+      if (!holds) break;
       const int row = row_base + r * 16 + fr;
       const float w = smW[row];
 #pragma unroll
-      for (int gg = 0; gg < 2; ++gg)
+      for (int gg = 0; gg < GROUPS; ++gg)
 #pragma unroll
         for (int c = 0; c < T::CS; ++c) {
           v4f val = acc[r][gg][c];
@@ -350,38 +374,40 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[Tile
           v2u pk;
           pk[0] = pack_bf16x2(val[0], val[1]);
           pk[1] = pack_bf16x2(val[2], val[3]);
-          *reinterpret_cast<v2u*>(stage_out + row * 256 + (((col >> 3) ^ (row & 15)) << 3) + (col & 7)) = pk;
+          *reinterpret_cast<v2u*>(stage_out + row * (GROUPS * 128) + (((col >> 3) ^ (row & 15)) << 3) + (col & 7)) = pk;
         }
     }
     __syncthreads();
-    const int nchunks = g1_store ? 32 : 16;  // 16 B chunks of a row to store
+    constexpr int CH = GROUPS * 16;          // 16 B chunks of a staged row
+    const int nchunks = g1_store ? 32 : 16;  // of them to store
     if (!g.accumulate) {
-      for (int ci = tid; ci < BM * 32; ci += T::THREADS) {
-        const int row = ci >> 5, cc = ci & 31;
+      for (int ci = tid; ci < BM * CH; ci += T::THREADS) {
+        const int row = ci / CH, cc = ci % CH;
         if (cc >= nchunks) continue;
         const int64_t slot = smSlot[row];
         if (slot >= g.S) continue;
         const int64_t n = (cc < 16 ? g0 : g1) * 128 + (cc & 15) * 8;
         *reinterpret_cast<v4i*>(g.C + slot * g.ldc + n) =
-            *reinterpret_cast<const v4i*>(stage_out + row * 256 + ((cc ^ (row & 15)) << 3));
+            *reinterpret_cast<const v4i*>(stage_out + row * (GROUPS * 128) + ((cc ^ (row & 15)) << 3));
       }
     } else {
       // K-split accumulation: the bf16 partial is added to the bf16 C of the
       // earlier chunks and rounded again.  A thread's chunks are read in
       // batches of NBATCH before any of them is written back, so the reads of
       // C overlap instead of forming one round trip per chunk.
-      constexpr int PER = BM * 32 / T::THREADS;
+      constexpr int PER = (BM * CH + T::THREADS - 1) / T::THREADS;
       constexpr int NBATCH = PER < 8 ? PER : 8;
-      static_assert(PER * T::THREADS == BM * 32 && PER % NBATCH == 0, "copy-out batches");
+      static_assert((PER == 1 || PER * T::THREADS == BM * CH) && PER % NBATCH == 0, "copy-out batches");
       for (int b0 = 0; b0 < PER; b0 += NBATCH) {
         v4i old[NBATCH];
         v4i* dst[NBATCH];
 #pragma unroll
         for (int b = 0; b < NBATCH; ++b) {
           const int ci = tid + (b0 + b) * T::THREADS;
-          const int row = ci >> 5, cc = ci & 31;
-          const int64_t slot = smSlot[row];
+          const int row = ci / CH, cc = ci % CH;
           dst[b] = nullptr;
+          if (PER * T::THREADS > BM * CH && ci >= BM * CH) continue;
+          const int64_t slot = smSlot[row];
           if (cc < nchunks && slot < g.S) {
             const int64_t n = (cc < 16 ? g0 : g1) * 128 + (cc & 15) * 8;
             dst[b] = reinterpret_cast<v4i*>(g.C + slot * g.ldc + n);
@@ -392,8 +418,8 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[Tile
         for (int b = 0; b < NBATCH; ++b) {
           if (!dst[b]) continue;
           const int ci = tid + (b0 + b) * T::THREADS;
-          const int row = ci >> 5, cc = ci & 31;
-          v4i val = *reinterpret_cast<const v4i*>(stage_out + row * 256 + ((cc ^ (row & 15)) << 3));
+          const int row = ci / CH, cc = ci % CH;
+          v4i val = *reinterpret_cast<const v4i*>(stage_out + row * (GROUPS * 128) + ((cc ^ (row & 15)) << 3));
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             const uint32_t a = (uint32_t)old[b][q], v = (uint32_t)val[q];
@@ -406,25 +432,42 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[Tile
   }
 }
 
+// Waits until the loads of the oldest of a wave's stages in flight are
+// complete; `younger` stages were issued after it, at most MAX of them still in
+// flight by the ring's depth.
+template <class T, int MAX>
+MOE_DEVICE void wait_stage(int younger) {
+  if constexpr (MAX <= 0) {
+    wait_vmcnt<0>();
+  } else {
+    if (younger >= MAX)
+      wait_vmcnt<MAX * T::VM>();
+    else
+      wait_stage<T, MAX - 1>(younger);
+  }
+}
+
 // The K loop and epilogue of one tile: n-tile j of rows [pos0, pos0 +
 // rows_avail) of the sorted order (a prefix of nvalid of them hold slots) of
 // expert e, with BM-row operand tiles.  A body with BM smaller than the tile
 // computes its first BM rows; the caller has checked that the rest are padding.
-template <int BM, bool FUSED, bool EXACT = false>
+template <class T, bool FUSED, bool EXACT = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t pos0, int rows_avail, int e,
                                           int nvalid, bool b_nt) {
-  using T = Tile<BM>;
+  constexpr int BM = T::BM, GROUPS = T::GROUPS;
+  static_assert(GROUPS == 2 || !FUSED, "the fused epilogue takes a gate and an up group");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   float* smSB = reinterpret_cast<float*>(smem + T::OFF_SB);  // [2 groups][kMaxKB]
   float* smRed = reinterpret_cast<float*>(smem + T::OFF_RED);
   int32_t* smSlot = reinterpret_cast<int32_t*>(smem + T::OFF_ROW);
-  float* smW = reinterpret_cast<float*>(smem + T::OFF_ROW + BM * 4);
+  float* smW = reinterpret_cast<float*>(smem + T::OFF_W);
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   // wave-uniform values live in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / T::WN;
   const int wn = wave % T::WN;
+  const int lw = wave - (T::NW - T::PW);  // index among the loading waves (negative: loads nothing)
   const int64_t K = g.K;
   const int KB = (int)(K / 128);
   if (rows_avail > BM) rows_avail = BM;
@@ -437,38 +480,45 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
     return (slot < g.S) ? slot / g.top_k : 0;
   };
 
-  // The tile's slot ids (and routed weights) for the epilogues; the barriers
-  // of the K loop order these writes before their use.
-  if (tid < BM) {
-    const int32_t slot = tid < rows_avail ? g.sorted[pos0 + tid] : (int32_t)g.S;
-    smSlot[tid] = slot;
-    if (!FUSED) smW[tid] = (g.topk_w && slot < g.S) ? g.topk_w[slot] : 1.0f;
+  // The tile's slot ids for the epilogues; the barriers of the K loop order
+  // these writes before their use.  The slots' routed weights go straight to
+  // LDS, 64 rows a load, covered by the first step's wait: a load through
+  // registers would hold back the first operand loads by a round trip.  Rows
+  // without a slot read slot 0's weight; their results are not stored.
+  const int lrow = 64 * lw + lane;
+  if ((!T::DEEP || lw >= 0) && lrow < BM) {
+    const int32_t slot = lrow < rows_avail ? g.sorted[pos0 + lrow] : (int32_t)g.S;
+    smSlot[lrow] = slot;
+    if (!FUSED && g.topk_w)
+      dma4(reinterpret_cast<const uint8_t*>(g.topk_w), slot < g.S ? (uint32_t)slot * 4u : 0u,
+           reinterpret_cast<uint8_t*>(smW) + 256 * lw);
   }
 
   // ---- per-lane DMA offsets (32-bit, relative to uniform bases) ----------
-  // A instruction gi = wave + NW*i covers tile rows 8*gi .. 8*gi+7; lane L fills
+  // A instruction gi = w + PW*i (of loading wave w) covers tile rows 8*gi .. 8*gi+7; lane L fills
   // LDS slot L&7 of row R = 8*gi + L/8 with logical chunk slot_of(L&7, R).
   uint32_t a_off[T::NA_W > 0 ? T::NA_W : 1];
 #pragma unroll
   for (int i = 0; i < T::NA_W; ++i) {
-    const int gi = wave + T::NW * i;
-    const int row = (gi < T::NA) ? 8 * gi + (lane >> 3) : 0;
+    const int gi = lw + T::PW * i;
+    // a wave that loads nothing (lw < 0) must not read sorted[] below the tile either
+    const int row = ((!T::DEEP || lw >= 0) && gi < T::NA) ? 8 * gi + (lane >> 3) : 0;
     const int cc = slot_of(lane & 7, row);
     a_off[i] = (uint32_t)(a_row_of(row) * g.lda) + (uint32_t)(cc * 16);
   }
-  // B instruction gi = wave + NW*i covers B-tile rows 8*gi .. 8*gi+7; tile rows
+  // B instruction gi = w + PW*i covers B-tile rows 8*gi .. 8*gi+7; tile rows
   // 0..127 are scale group g0, rows 128..255 group g1.  The lane's row inside its
-  // group is 8*wave + 8*NW*(i mod NB_W/2) + L/8, and its rotation does not
-  // depend on i (8*NW*i leaves row mod 16 and bit 3 unchanged), so one lane
+  // group is 8*w + 8*PW*(i mod NB_W/GROUPS) + L/8, and its rotation does not
+  // depend on i (8*PW*i leaves row mod 16 and bit 3 unchanged), so one lane
   // offset serves every instruction; the rest is a uniform base.
   uint32_t b_off;
   {
-    const int r0 = 8 * wave + (lane >> 3);
+    const int r0 = 8 * lw + (lane >> 3);
     const int cc = slot_of(lane & 7, r0);
     b_off = (uint32_t)(r0 * g.ldb) + (uint32_t)(cc * 16);
   }
-  // A scales: instruction s (issued by wave NW-1-s) covers rows 64*s .. 64*s+63.
-  const int s_idx = T::NW - 1 - wave;
+  // A scales: instruction s (issued by loading wave PW-1-s) covers rows 64*s .. 64*s+63.
+  const int s_idx = T::PW - 1 - lw;
   uint32_t sa_off = 0;
   if (s_idx < T::NS) {
     const int row = 64 * s_idx + lane;
@@ -478,7 +528,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
   }
   int64_t g0, g1;
   bool g1_store;
-  groups_of<FUSED>(g, j, g0, g1, g1_store);
+  groups_of<FUSED, GROUPS>(g, j, g0, g1, g1_store);
   const uint8_t* b_expert = g.B + (int64_t)e * g.b_es;
   const float* bs_expert = g.Bs + (int64_t)e * g.bs_es;
   const uint8_t* bg0 = b_expert + g0 * 128 * g.ldb;  // the tile's two weight groups
@@ -498,13 +548,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
     // Weight rows first: they come from HBM, the A rows mostly from L2.
     uint32_t boff = b_off;
     asm volatile("" : "+v"(boff));
-    constexpr int HALF = T::NB_W / 2;
+    constexpr int HALF = T::NB_W / GROUPS;  // instructions of one group
     if constexpr (BM <= 32) {
       auto issue_b = [&](auto load) {
 #pragma unroll
         for (int i = 0; i < T::NB_W; ++i) {
-          const uint8_t* bbase = (i < HALF ? bg0 : bg1) + (int64_t)(8 * T::NW * (i % HALF)) * g.ldb + kk * 128;
-          load(bbase, boff, dst + T::A_BYTES + (wave + T::NW * i) * 1024);
+          const uint8_t* bbase = (i < HALF ? bg0 : bg1) + (int64_t)(8 * T::PW * (i % HALF)) * g.ldb + kk * 128;
+          load(bbase, boff, dst + T::A_BYTES + (lw + T::PW * i) * 1024);
         }
       };
       if (b_nt)
@@ -514,14 +564,14 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
     } else {
 #pragma unroll
       for (int i = 0; i < T::NB_W; ++i) {
-        const uint8_t* bbase = (i < HALF ? bg0 : bg1) + (int64_t)(8 * T::NW * (i % HALF)) * g.ldb + kk * 128;
-        dma16(bbase, boff, dst + T::A_BYTES + (wave + T::NW * i) * 1024);
+        const uint8_t* bbase = (i < HALF ? bg0 : bg1) + (int64_t)(8 * T::PW * (i % HALF)) * g.ldb + kk * 128;
+        dma16(bbase, boff, dst + T::A_BYTES + (lw + T::PW * i) * 1024);
       }
     }
     const uint8_t* abase = g.A + kk * 128;
 #pragma unroll
     for (int i = 0; i < T::NA_W; ++i) {
-      const int gi = wave + T::NW * i;
+      const int gi = lw + T::PW * i;
       uint32_t off = a_off[i];
       asm volatile("" : "+v"(off));
       if (gi < T::NA && 8 * gi < a_rows_needed) dma16(abase, off, dst + gi * 1024);
@@ -535,18 +585,18 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
   };
 
   // Weight scales of both groups for every K block, smSB[g * kMaxKB + kk]:
-  // one 4-byte direct-to-LDS load per lane of waves 0-3 (entry 64 * wave +
+  // one 4-byte direct-to-LDS load per lane of loading waves 0-3 (entry 64 * w +
   // lane), issued before stage 0, so that step 0's wait covers them.  Entries
   // past KB read a valid scale and are never used.
-  static_assert(2 * kMaxKB == 4 * 64 && Tile<BM>::NW >= 4, "four waves load the weight scales");
+  static_assert(2 * kMaxKB == 4 * 64 && T::PW >= 4, "two waves load a group's weight scales");
   auto issue_weight_scales = [&] {
-    if (wave < 4) {
-      const int idx = 64 * wave + lane;
+    if (lw < 2 * GROUPS) {
+      const int idx = 64 * lw + lane;
       const int kb = idx % kMaxKB;
       const int64_t grp = idx < kMaxKB ? g0 : g1;
       uint32_t off = (uint32_t)((grp * g.bs_ld + (kb < KB ? kb : 0)) * 4);
       asm volatile("" : "+v"(off));
-      dma4(reinterpret_cast<const uint8_t*>(bs_expert), off, reinterpret_cast<uint8_t*>(smSB) + 256 * wave);
+      dma4(reinterpret_cast<const uint8_t*>(bs_expert), off, reinterpret_cast<uint8_t*>(smSB) + 256 * lw);
     }
   };
 
@@ -563,20 +613,22 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
   const float* smSA = reinterpret_cast<const float*>(smem + T::OFF_SA);
   const int sa_lane = row_base + fr;  // the lane's token (the MFMA's second operand)
 
-  issue_weight_scales();
-  issue_stage(0, 0, bg0, bg1);
+  if (!T::DEEP || lw >= 0) {
+    issue_weight_scales();
+    issue_stage(0, 0, bg0, bg1);
 #pragma unroll
-  for (int st = 1; st < T::KS - 1; ++st)
-    if (st < KB) issue_stage(st, st, bg0, bg1);
+    for (int st = 1; st < T::KS - 1; ++st)
+      if (st < KB) issue_stage(st, st, bg0, bg1);
+  }
 
   int ra = (nvalid - row_base + 15) / 16;
   ra = ra < 0 ? 0 : (ra > T::RS ? T::RS : ra);
 
-  v4f acc[T::RS][2][T::CS];
+  v4f acc[T::RS][GROUPS][T::CS];
 #pragma unroll
   for (int r = 0; r < T::RS; ++r)
 #pragma unroll
-    for (int gg = 0; gg < 2; ++gg)
+    for (int gg = 0; gg < GROUPS; ++gg)
 #pragma unroll
       for (int c = 0; c < T::CS; ++c) acc[r][gg][c] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
 
@@ -586,16 +638,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
     for (int kk = 0; kk < KB; ++kk) {
       // Step kk's loads complete; the younger stages' loads (up to KS - 2 of
       // them, as many as were issued) may stay in flight.
-      if (T::KS == 4 && kk + 2 < KB) wait_vmcnt<2 * T::VM>();
-      else if (T::KS >= 3 && kk + 1 < KB) wait_vmcnt<T::VM>();
-      else wait_vmcnt<0>();
+      if constexpr (!T::DEEP) wait_stage<T, T::KS - 2>(KB - 1 - kk);
       block_barrier();
       // The buffer read at step kk-1 is free once every wave has passed the barrier.
       // The waves issue the stage's loads at raised priority, so that all of
       // them are in flight before the MFMAs of any wave take the issue slots.
-      __builtin_amdgcn_s_setprio(3);
-      if (kk + T::KS - 1 < KB) issue_stage(kk + T::KS - 1, stage == 0 ? T::KS - 1 : stage - 1, bg0, bg1);
-      __builtin_amdgcn_s_setprio(0);
+      if constexpr (!T::DEEP) {
+        __builtin_amdgcn_s_setprio(3);
+        if (kk + T::KS - 1 < KB) issue_stage(kk + T::KS - 1, stage == 0 ? T::KS - 1 : stage - 1, bg0, bg1);
+        __builtin_amdgcn_s_setprio(0);
+      }
       if constexpr (RA > 0) {
         const uint8_t* st = smem + stage * T::STAGE;
         const uint8_t* pa0 = st + a_lane0;
@@ -604,18 +656,19 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
         const uint8_t* pb1 = st + b_lane1;
         const float* tSA = smSA + stage * T::NS * 64 + sa_lane;
         // a_s * b_s of the step for each 16-row subtile and column group
-        float sab[2][RA];
+        float sab[GROUPS][RA];
         auto scale_products = [&] {
-          const float sb0 = smSB[kk];
-          const float sb1 = smSB[kMaxKB + kk];
+          float sb[GROUPS];
+#pragma unroll
+          for (int gg = 0; gg < GROUPS; ++gg) sb[gg] = smSB[gg * kMaxKB + kk];
 #pragma unroll
           for (int r = 0; r < RA; ++r) {
             const float sa = tSA[r * 16];
-            sab[0][r] = sa * sb0;
-            sab[1][r] = sa * sb1;
+#pragma unroll
+            for (int gg = 0; gg < GROUPS; ++gg) sab[gg][r] = sa * sb[gg];
           }
         };
-        constexpr int NQ = 2 * T::CS;  // weight fragments per step
+        constexpr int NQ = GROUPS * T::CS;  // weight fragments per step
         if constexpr (EXACT) {
 #pragma clang fp contract(off)
           // Exact dots on the bf16 matrix core: the step's A fragments are
@@ -719,18 +772,31 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
       stage = (stage == T::KS - 1) ? 0 : stage + 1;
     }
   };
-  switch (ra) {
-    case 0: kloop(std::integral_constant<int, 0>{}); break;
-    case 1: if constexpr (T::RS >= 1) kloop(std::integral_constant<int, (T::RS >= 1 ? 1 : 0)>{}); break;
-    case 2: if constexpr (T::RS >= 2) kloop(std::integral_constant<int, (T::RS >= 2 ? 2 : 0)>{}); break;
-    case 3: if constexpr (T::RS >= 3) kloop(std::integral_constant<int, (T::RS >= 3 ? 3 : 0)>{}); break;
-    default: if constexpr (T::RS >= 4) kloop(std::integral_constant<int, (T::RS >= 4 ? 4 : 0)>{}); break;
+  if (T::DEEP && lw >= 0) {
+    // A loading wave's K loop: the same barriers, between them the next stage's
+    // loads while the other waves compute.
+    __builtin_amdgcn_s_setprio(3);
+    int stage = 0;
+    for (int kk = 0; kk < KB; ++kk) {
+      wait_stage<T, T::KS - 2>(KB - 1 - kk);
+      block_barrier();
+      if (kk + T::KS - 1 < KB) issue_stage(kk + T::KS - 1, stage == 0 ? T::KS - 1 : stage - 1, bg0, bg1);
+      stage = (stage == T::KS - 1) ? 0 : stage + 1;
+    }
+    __builtin_amdgcn_s_setprio(0);
+  } else {
+    switch (ra) {
+      case 0: kloop(std::integral_constant<int, 0>{}); break;
+      case 1: if constexpr (T::RS >= 1) kloop(std::integral_constant<int, (T::RS >= 1 ? 1 : 0)>{}); break;
+      case 2: if constexpr (T::RS >= 2) kloop(std::integral_constant<int, (T::RS >= 2 ? 2 : 0)>{}); break;
+      case 3: if constexpr (T::RS >= 3) kloop(std::integral_constant<int, (T::RS >= 3 ? 3 : 0)>{}); break;
+      default: if constexpr (T::RS >= 4) kloop(std::integral_constant<int, (T::RS >= 4 ? 4 : 0)>{}); break;
+    }
   }
   // Every wave is done with the operand ring (the last step waited for all of
   // its loads); the epilogue stages the output at its base.
   block_barrier();
-  tile_epilogue<BM, FUSED>(g, acc, j, pos0, rows_avail, g0, g1, g1_store, smem, smRed, smSlot, smW);
-
+  tile_epilogue<T, FUSED>(g, acc, j, pos0, rows_avail, g0, g1, g1_store, smem, smRed, smSlot, smW);
 }
 
 // A tile of a BM-row launch whose valid rows fit SUB rows, run with the
@@ -740,7 +806,7 @@ template <int SUB, int BM, bool FUSED, bool EXACT>
 __device__ __forceinline__ void short_tile(const GemmArgs& g, int64_t j, int64_t pos0, int rows_avail, int e,
                                            int nvalid) {
   static_assert(Tile<SUB>::THREADS == Tile<BM>::THREADS, "same workgroup size");
-  gemm_tile<SUB, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, false);
+  gemm_tile<Tile<SUB>, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, false);
   if (FUSED) {
     const int tid = threadIdx.x;
     for (int ci = SUB * 8 + tid; ci < rows_avail * 8; ci += Tile<BM>::THREADS) {
@@ -748,6 +814,34 @@ __device__ __forceinline__ void short_tile(const GemmArgs& g, int64_t j, int64_t
       *reinterpret_cast<v4i*>(g.hq + (pos0 + row) * g.I + j * 128 + cc * 16) = (v4i){0, 0, 0, 0};
     }
     for (int row = SUB + tid; row < rows_avail; row += Tile<BM>::THREADS) *hs_at(g, pos0 + row, j) = kScaleFloor;
+  }
+}
+
+// Expert not local: zero output rows (kernels.py:112-120).
+template <class T, bool FUSED>
+__device__ __forceinline__ void zero_tile(const GemmArgs& g, int64_t j, int64_t pos0, int rows_avail) {
+  if (!FUSED && g.accumulate) return;  // later K chunks leave C as it is (kernels.py:112-120)
+  const int tid = threadIdx.x;
+  int64_t g0, g1;
+  bool g1_store;
+  groups_of<FUSED, T::GROUPS>(g, j, g0, g1, g1_store);
+  if (FUSED) {
+    for (int ci = tid; ci < rows_avail * 8; ci += T::THREADS) {
+      const int row = ci >> 3, cc = ci & 7;
+      *reinterpret_cast<v4i*>(g.hq + (pos0 + row) * g.I + j * 128 + cc * 16) = (v4i){0, 0, 0, 0};
+    }
+    for (int row = tid; row < rows_avail; row += T::THREADS) *hs_at(g, pos0 + row, j) = kScaleFloor;
+  } else {
+    constexpr int CH = T::GROUPS * 16;
+    for (int ci = tid; ci < rows_avail * CH; ci += T::THREADS) {
+      const int row = ci / CH, cc = ci % CH;
+      const int64_t slot = g.sorted[pos0 + row];
+      if (slot >= g.S) continue;
+      const int grp = cc >> 4;
+      if (grp == 1 && !g1_store) continue;
+      const int64_t n = (grp ? g1 : g0) * 128 + (cc & 15) * 8;
+      *reinterpret_cast<v4i*>(g.C + slot * g.ldc + n) = (v4i){0, 0, 0, 0};
+    }
   }
 }
 
@@ -870,29 +964,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   const int rows_avail = (int)((u < n_short ? base : base + 1) * vb);
 
   if (e < 0 || e >= g.E) {
-    // Expert not local: zero output rows (kernels.py:112-120).
-    if (!FUSED && g.accumulate) return;  // later K chunks leave C as it is (kernels.py:112-120)
-    int64_t g0, g1;
-    bool g1_store;
-    groups_of<FUSED>(g, j, g0, g1, g1_store);
-    if (FUSED) {
-      for (int ci = tid; ci < rows_avail * 8; ci += T::THREADS) {
-        const int row = ci >> 3, cc = ci & 7;
-        *reinterpret_cast<v4i*>(g.hq + (pos0 + row) * g.I + j * 128 + cc * 16) = (v4i){0, 0, 0, 0};
-      }
-      for (int row = tid; row < rows_avail; row += T::THREADS)
-        *hs_at(g, pos0 + row, j) = kScaleFloor;
-    } else {
-      for (int ci = tid; ci < rows_avail * 32; ci += T::THREADS) {
-        const int row = ci >> 5, cc = ci & 31;
-        const int64_t slot = g.sorted[pos0 + row];
-        if (slot >= g.S) continue;
-        const int grp = cc >> 4;
-        if (grp == 1 && !g1_store) continue;
-        const int64_t n = (grp ? g1 : g0) * 128 + (cc & 15) * 8;
-        *reinterpret_cast<v4i*>(g.C + slot * g.ldc + n) = (v4i){0, 0, 0, 0};
-      }
-    }
+    zero_tile<T, FUSED>(g, j, pos0, rows_avail);
     return;
   }
 
@@ -933,9 +1005,9 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
       // rows [0, 128) and then [128, rows_avail), whose valid rows are
       // [128, nvalid); the barrier keeps the second body's first loads out of
       // the LDS the first one's copy-out still reads
-      gemm_tile<128, FUSED, EXACT>(g, j, pos0, 128, e, 128, false);
+      gemm_tile<Tile<128>, FUSED, EXACT>(g, j, pos0, 128, e, 128, false);
       __syncthreads();
-      gemm_tile<128, FUSED, EXACT>(g, j, pos0 + 128, rows_avail - 128, e, nvalid - 128, false);
+      gemm_tile<Tile<128>, FUSED, EXACT>(g, j, pos0 + 128, rows_avail - 128, e, nvalid - 128, false);
       return;
     }
   }
@@ -943,7 +1015,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   // the only readers of their weight tiles: those loads carry the
   // non-temporal hint.  Experts with several row tiles, and taller tiles,
   // share weight tiles through L2 and load them cached.
-  if constexpr (!(EXACT && BM == 256)) gemm_tile<BM, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, BM <= 32 && units == 1);
+  if constexpr (!(EXACT && BM == 256)) gemm_tile<Tile<BM>, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, BM <= 32 && units == 1);
 }
 
 template <int BM, bool FUSED>
@@ -961,8 +1033,79 @@ void w13_exact_kernel(GemmArgs g) {
   grouped_gemm_body<BM, true, true>(g);
 }
 
+// One workgroup of a launch whose tiles all run at once (decode: few blocks).
+// Such a launch waits for memory round trips, so
+//   - the tile is a plain division of the workgroup id, and everything the
+//     tile's first loads depend on (the block's expert and its neighbours', the
+//     slots, the row count) is read in one round trip instead of a chain of three;
+//   - one workgroup has its CU to itself and the whole LDS as its operand ring:
+//     up to six stages in flight instead of one;
+//   - four waves only issue loads and four only compute: where every wave does
+//     both, a step is the time to queue its 37 loads (the CU's address unit takes
+//     64 B a cycle) plus the time to compute;
+//   - a plain launch takes 128 weight rows a tile, twice the workgroups.
+// There is one row tile per block, and row tiles that share weights run at the
+// same time whatever their order.
+template <class T, bool FUSED, bool EXACT>
+__device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
+  const int tid = threadIdx.x;
+  const int64_t b = blockIdx.x / (uint32_t)g.n_tiles, j = blockIdx.x % (uint32_t)g.n_tiles;
+  const int64_t n_blocks = *g.ntpp / T::BM;
+  // within max_padded for every b of the grid (the entries past ntpp are not used)
+  const int64_t blk = g.blk ? (b < n_blocks ? g.blk[b] : 0) : b;
+  const int64_t pos0 = blk * T::BM;
+  const int e = g.eids[b];
+  const int before = b > 0 ? g.eids[b - 1] : -1;
+  const int after = b + 1 < g.max_blocks ? g.eids[b + 1] : -1;
+  bool row_valid = false;
+  if (tid < T::BM && pos0 + tid < g.max_padded) row_valid = g.sorted[pos0 + tid] < g.S;
+  const int nvalid = __syncthreads_count(row_valid);
+  if (b >= n_blocks) return;
+  if (e < 0 || e >= g.E) {
+    zero_tile<T, FUSED>(g, j, pos0, T::BM);
+    return;
+  }
+  const bool single = before != e && !(b + 1 < n_blocks && after == e);  // the expert's only row tile
+  gemm_tile<T, FUSED, EXACT>(g, j, pos0, T::BM, e, nvalid, single);
+}
+
+template <int BM, int GROUPS, bool FUSED, bool EXACT>
+__global__ __launch_bounds__((Tile<BM, GROUPS, true>::THREADS))
+__attribute__((amdgpu_waves_per_eu(2, 2)))
+void flat_gemm_kernel(GemmArgs g) {
+  flat_gemm_body<Tile<BM, GROUPS, true>, FUSED, EXACT>(g);
+}
+
+constexpr int64_t kCus = 256;
+
+template <int BM, int GROUPS, bool FUSED, bool EXACT>
+static int launch_flat(const GemmArgs& args, hipStream_t st) {
+  using T = Tile<BM, GROUPS, true>;
+  const void* fn = (const void*)flat_gemm_kernel<BM, GROUPS, FUSED, EXACT>;
+  static const hipError_t attr_rc =
+      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
+  if (attr_rc != hipSuccess) return kErrLaunch;
+  GemmArgs a = args;
+  if (GROUPS == 1) a.n_tiles = a.N / 128;
+  const int64_t grid = a.max_blocks * a.n_tiles;
+  if (grid <= 0) return kOk;
+  hipLaunchKernelGGL((flat_gemm_kernel<BM, GROUPS, FUSED, EXACT>), dim3((unsigned)grid), dim3(T::THREADS),
+                     T::LDS_BYTES, st, a);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
 template <int BM, bool FUSED, bool EXACT>
 static int launch_gemm(const GemmArgs& args, hipStream_t st) {
+  // Launches whose tiles all find a CU of their own (see flat_gemm_body).
+  if constexpr (BM <= 64) {
+    if (args.bma == BM && args.tile_order == 0 && args.vshift == 0) {
+      if constexpr (!FUSED) {
+        if (args.max_blocks * (args.N / 128) <= kCus) return launch_flat<BM, 1, FUSED, EXACT>(args, st);
+      }
+      if (args.max_blocks * args.n_tiles <= kCus) return launch_flat<BM, 2, FUSED, EXACT>(args, st);
+    }
+  }
+
   using T = Tile<BM>;
   const void* fn;
   if constexpr (EXACT)
@@ -1056,6 +1199,7 @@ int moe::plain_gemm(const void* A, const float* A_scale, const void* B, const fl
   g.K = K;
   g.I = 0;
   g.max_blocks = (max_padded + BM - 1) / BM;
+  g.max_padded = max_padded;
   g.n_tiles = (N / 128 + 1) / 2;
   g.bma = BM;
   g.top_k = top_k;
@@ -1065,6 +1209,7 @@ int moe::plain_gemm(const void* A, const float* A_scale, const void* B, const fl
   dense_strides(g);
   if (scales_by_pos) g.as_pos_ld = max_padded;
   g.blk = local.blocks;
+  if (local.max_blocks > 0 && local.max_blocks < g.max_blocks) g.max_blocks = local.max_blocks;
   return dispatch_gemm<false>(TM, g, (hipStream_t)stream);
 }
 
@@ -1141,6 +1286,7 @@ static int setup_plain(GemmArgs& g, int& TM, const void* A, const float* A_scale
   g.N = N;
   g.K = K;
   g.max_blocks = (max_padded + BM - 1) / BM;
+  g.max_padded = max_padded;
   g.n_tiles = (N / 128 + 1) / 2;
   g.bma = BM;
   g.top_k = top_k;
@@ -1260,6 +1406,7 @@ int moe::w13_gemm(const void* Aq, const float* A_scale, const void* W13, const f
   g.K = H;
   g.I = I;
   g.max_blocks = (max_padded + (BM >> vshift) - 1) / (BM >> vshift);
+  g.max_padded = max_padded;
   g.n_tiles = I / 128;
   g.bma = BM;
   g.vshift = vshift;
@@ -1269,6 +1416,7 @@ int moe::w13_gemm(const void* Aq, const float* A_scale, const void* W13, const f
   dense_strides(g);
   if (scales_by_pos) g.as_pos_ld = g.hs_pos_ld = max_padded;
   g.blk = local.blocks;
+  if (local.max_blocks > 0 && local.max_blocks << vshift < g.max_blocks) g.max_blocks = local.max_blocks << vshift;
   return exact ? dispatch_gemm<true, true>(TM, g, (hipStream_t)stream) : dispatch_gemm<true>(TM, g, (hipStream_t)stream);
 }
 

@@ -5,13 +5,24 @@
 
 namespace moe {
 
-// The list of local blocks that align writes under an expert map (see
-// moe_layer's local_blocks): blocks == null without one.  E_routed: the experts
-// the slots are spread over, for the choice of the tile height (0: E).
+// What the layer knows of its blocks beyond the align outputs.  blocks: the list
+// of local blocks that align writes under an expert map (moe_layer's
+// local_blocks), null without one.  E_routed: the experts the slots are spread
+// over, for the choice of the tile height (0: E).  max_blocks: a bound on the
+// blocks of the launch (0: what fits in max_padded, which with few slots allows
+// for more).
 struct LocalBlocks {
   const int32_t* blocks = nullptr;
   int64_t E_routed = 0;
+  int64_t max_blocks = 0;
 };
+
+// S slots over E experts fill at most this many blocks of BM: m <= min(S, E)
+// experts with c >= 1 slots have ceil(c/BM) <= 1 + (c-1)/BM blocks each.
+inline int64_t blocks_bound(int64_t S, int64_t E, int64_t BM) {
+  const int64_t m = S < E ? S : E;
+  return m + (S - m) / BM;
+}
 
 // local_blocks holds [0] local blocks * BM, then the blocks, then their local
 // expert ids, then a word per token whose bit i says that slot i's expert is local.

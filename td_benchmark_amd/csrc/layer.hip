@@ -19,6 +19,8 @@ static LocalBlocks local_of(const moe_layer* l) {
   LocalBlocks r;
   r.E_routed = l->E_routed;
   if (l->expert_map) r.blocks = local_blk(l->local_blocks);
+  if (block_m_ok(l->block_size_m))
+    r.max_blocks = blocks_bound(l->T * l->top_k, l->expert_map ? l->E : l->E_routed, l->block_size_m);
   return r;
 }
 
