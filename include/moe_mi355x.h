@@ -322,12 +322,15 @@ typedef struct moe_layer {
   int32_t* ntpp;
   void* workspace;
   int32_t* local_blocks;      /* moe_layer_local_blocks_bytes, with expert_map; else NULL */
+  int32_t* runs;              /* moe_layer_runs_bytes, 16-byte aligned: align's notes on the experts' rows for the
+                                 GEMMs' tile order; NULL: without */
   void* hq;                   /* [max_padded, I] e4m3fn */
   float* hs;                  /* [I/128, max_padded] with s1_pos, else [max_padded, I/128] */
   void* D;                    /* [T * top_k, Hp] bf16 */
 } moe_layer;
 
 int64_t moe_layer_local_blocks_bytes(int64_t T, int64_t max_padded, int32_t block_size_m);
+int64_t moe_layer_runs_bytes(int32_t E_routed);
 /* hidden [T, H] bf16 (NULL: align alone), topk_ids [T, top_k]. */
 int moe_layer_quant_align(const moe_layer* layer, const void* hidden, const int32_t* topk_ids, void* stream);
 /* The activation scales by sorted position (nothing where s1_pos is NULL). */

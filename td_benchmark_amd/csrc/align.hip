@@ -216,6 +216,7 @@ struct AlignArgs {
   int32_t* eids;
   int32_t* ntpp;
   int32_t* local;  // the lists of local blocks and slots, or null (see internal.hpp)
+  int32_t* runs;   // the table of runs, or null (see internal.hpp)
   int64_t max_padded;
   int S, E, BM, top_k;
 };
@@ -239,6 +240,7 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   __shared__ int32_t hist[kAlignMaxExperts];
   __shared__ int32_t wave_cnt[kAlignWaves], wave_before[kAlignWaves], wave_total[kAlignWaves];
   __shared__ int32_t wave_lbefore[kAlignWaves], wave_ltotal[kAlignWaves];
+  __shared__ int32_t wave_rank[kAlignWaves], wave_runs[kAlignWaves];
   const int sh = __builtin_ctz(a.BM);  // BM is a power of two
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // wave w takes slots [w*IT*64, (w+1)*IT*64), 64 consecutive ones a step
@@ -258,13 +260,17 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   __syncthreads();
   int before = 0, total = 0;    // padded sizes of the experts before e, and of all
   int lbefore = 0, ltotal = 0;  // and of the local ones among them
+  int place = 0, n_runs = 0;    // experts here with more slots than e (or as many and before it), and with any
+  const int own = hist[e];
   for (int x = tid; x < a.E; x += kAlignThreads) {
     const int p = (hist[x] + a.BM - 1) >> sh << sh;
     total += p;
     if (x < e) before += p;
-    if (a.local && a.expert_map[x] >= 0) {
+    if (!a.expert_map || a.expert_map[x] >= 0) {
       ltotal += p;
       if (x < e) lbefore += p;
+      n_runs += p > 0;
+      place += hist[x] > own || (hist[x] == own && x < e);
     }
   }
 #pragma unroll
@@ -273,15 +279,19 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
     total += __shfl_xor(total, o);
     lbefore += __shfl_xor(lbefore, o);
     ltotal += __shfl_xor(ltotal, o);
+    place += __shfl_xor(place, o);
+    n_runs += __shfl_xor(n_runs, o);
   }
   if (lane == 0) {
     wave_before[wave] = before;
     wave_total[wave] = total;
     wave_lbefore[wave] = lbefore;
     wave_ltotal[wave] = ltotal;
+    wave_rank[wave] = place;
+    wave_runs[wave] = n_runs;
   }
   __syncthreads();
-  before = total = lbefore = ltotal = 0;
+  before = total = lbefore = ltotal = place = n_runs = 0;
   int rank = 0;  // of this wave's first slot of e
 #pragma unroll
   for (int w = 0; w < kAlignWaves; ++w) {
@@ -289,9 +299,11 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
     total += wave_total[w];
     lbefore += wave_lbefore[w];
     ltotal += wave_ltotal[w];
+    place += wave_rank[w];
+    n_runs += wave_runs[w];
     rank += w < wave ? wave_cnt[w] : 0;
   }
-  const int cnt = hist[e];
+  const int cnt = own;
   const int padded = (cnt + a.BM - 1) >> sh << sh;
   const uint64_t lt = lane == 0 ? 0ull : ~0ull >> (64 - lane);
 #pragma unroll
@@ -319,9 +331,12 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
     a.sorted[i] = a.S;
     if ((i & (a.BM - 1)) == 0) a.eids[i >> sh] = -1;
   }
+  if (a.runs && tid == 0 && cnt > 0 && local >= 0)
+    reinterpret_cast<v4i*>(a.runs + 4)[place] = (v4i){before, cnt, local, padded};
   if (e == 0 && tid == 0) {
     *a.ntpp = total;
     if (a.local) *a.local = ltotal;
+    if (a.runs) *a.runs = n_runs;
   }
 }
 
@@ -382,6 +397,7 @@ __global__ __launch_bounds__(kAlignThreads) void quant_align_kernel(AlignArgs a,
 
 // The one-launch form holds up to 32 ids a lane.
 constexpr int64_t kAlignOneLaunchSlots = 32 * kAlignThreads;
+static_assert(kAlignOneLaunchSlots == kRunsMaxSlots, "the one-launch form writes the table of runs");
 // Chunks (16 B of input) up to which the quant runs beside align; larger ones
 // are bound by HBM and take the quant kernel's own block and unroll.
 constexpr int64_t kQuantBesideAlign = (int64_t)1 << 22;
@@ -428,13 +444,14 @@ static void by_slots(int64_t S, F&& f) {
 
 static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
                       int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded,
-                      void* workspace, void* stream, int32_t* local = nullptr, int32_t top_k = 1) {
+                      void* workspace, void* stream, int32_t* local = nullptr, int32_t* runs = nullptr,
+                      int32_t top_k = 1) {
   const int arg_rc = align_args(topk_ids, S, E, BM, sorted_ids, expert_ids, ntpp, max_padded, true, workspace);
   if (arg_rc != kOk) return arg_rc;
   if (!expert_map) local = nullptr;
   hipStream_t st = (hipStream_t)stream;
   if (S <= kAlignOneLaunchSlots) {
-    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local,
+    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs,
                       max_padded, (int)S, (int)E, (int)BM, (int)top_k};
     by_slots(S, [&](auto it) {
       hipLaunchKernelGGL(align_expert_kernel<decltype(it)::value>, dim3((unsigned)E), dim3(kAlignThreads), 0, st, a);
@@ -478,7 +495,7 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
 int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq, float* scales,
                      const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
                      int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded, void* workspace,
-                     int32_t* local, int32_t top_k, void* stream) {
+                     int32_t* local, int32_t* runs, int32_t top_k, void* stream) {
   // both halves' arguments before either is launched
   if (top_k <= 0) return kErrBadTopK;
   if (T < 0 || H < 0 || ldq < (H + 127) / 128 * 128) return kErrBadShape;
@@ -494,10 +511,10 @@ int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int6
     const int qrc = moe_quant_group128_padded(x_bf16, T, H, q_fp8, ldq, scales, stream);
     if (qrc != kOk) return qrc;
     return align_impl(topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp, max_padded, workspace, stream,
-                      local, top_k);
+                      local, runs, top_k);
   }
   if (!expert_map) local = nullptr;
-  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local,
+  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs,
                       max_padded, (int)S, (int)E, (int)BM, (int)top_k};
   const unsigned grid = (unsigned)(E + (q.n_chunks + kAlignThreads - 1) / kAlignThreads);
   by_slots(S, [&](auto it) {
@@ -515,7 +532,7 @@ extern "C" int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q
                                const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp,
                                int64_t max_padded, void* workspace, void* stream) {
   return quant_align(x_bf16, T, H, q_fp8, ldq, scales, topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp,
-                     max_padded, workspace, nullptr, 1, stream);
+                     max_padded, workspace, nullptr, nullptr, 1, stream);
 }
 
 extern "C" int moe_align_block_size(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,

@@ -94,6 +94,7 @@ constexpr int kTailRows = 64;  // row tiles with at most this many valid rows ru
 // every shape and the W2 of DeepSeek-V3 and Qwen3, K <= 7168, lose 1-7 % that
 // way).
 constexpr int64_t kColMajorK = 8192;
+constexpr int kTileGroup = 4;  // n-tiles of a group: 2, 8 and 16 (W13), 2, 3, 7 and 14 (W2) measured slower
 // MFMAs issued between an MFMA and the FMAs that scale its result: the VALU
 // reads a result that is complete, without hazard waits.
 constexpr int kScaleLag = 2;
@@ -102,12 +103,13 @@ constexpr int kScaleLag = 2;
 // launches); DEEP: the form for launches whose tiles all run at once, one
 // workgroup per CU with as deep a ring as the LDS holds, filled by waves that do
 // nothing else (see flat_gemm_body).
-template <int BM_, int GROUPS_ = 2, bool DEEP_ = false>
+template <int BM_, int GROUPS_ = 2, bool DEEP_ = false, bool LOOP_ = false>
 struct Tile {
   static constexpr int BM = BM_;
   static constexpr int GROUPS = GROUPS_;
   static_assert(GROUPS == 2 || (DEEP_ && BM <= 64), "narrow tiles are deep and short");
   static constexpr bool DEEP = DEEP_;
+  static constexpr bool LOOP = LOOP_;  // the workgroup runs several tiles
   static constexpr int NW = DEEP || BM >= 32 ? 8 : 4;  // waves per workgroup (2 per SIMD at 8)
   static constexpr int THREADS = 64 * NW;
   static constexpr int CW = DEEP ? 4 : NW;  // waves that compute: the first ones
@@ -166,6 +168,7 @@ struct GemmArgs {
   // ascending order; eids and ntpp then describe this list, and the other
   // blocks are no part of the launch.
   const int32_t* blk;
+  const int32_t* runs;     // the experts' runs by descending rows (see internal.hpp), or null
   const float* topk_w;     // [S] or null
   uint16_t* C;             // bf16 [S, N]            (plain epilogue)
   uint8_t* hq;             // fp8 [max_padded, I]    (fused epilogue)
@@ -176,6 +179,7 @@ struct GemmArgs {
   int64_t I;
   int64_t max_blocks;      // (virtual) blocks that fit in max_padded
   int64_t max_padded;      // entries of sorted
+  int64_t run_tiles;       // with runs: a bound on the row tiles
   int64_t n_tiles;         // 256-column n-tiles
   int bma;                 // rows per align block (block_size_m); a tile spans BM / bma of them
   // Exact-dot launches only: the tile map counts virtual blocks of bma >> vshift
@@ -185,6 +189,7 @@ struct GemmArgs {
   int top_k;
   int a_by_pos;
   int E;
+  int E_routed;            // with runs: the table's capacity
   int tile_order;          // 0 expert-major (XCD-contiguous), 1 shuffled, 2 half-phase
   // Strides of the (possibly sliced) operands; base pointers are pre-offset.
   int64_t lda;             // A row stride, bytes
@@ -201,6 +206,16 @@ struct GemmArgs {
   // Fused epilogue: hs K-major, hs[j * hs_pos_ld + pos] (0: hs[pos * I/128 + j]).
   int64_t hs_pos_ld;
 };
+
+// The thread's index.  In a workgroup that runs one tile after another (LOOP)
+// it is opaque to the compiler, which would otherwise keep everything derived
+// from it in registers from tile to tile, more than the tall tiles leave free.
+template <class T>
+MOE_DEVICE int thread_id() {
+  int t = threadIdx.x;
+  if constexpr (T::LOOP) asm volatile("" : "+v"(t));
+  return t;
+}
 
 // Element (position pos, group j) of the fused epilogue's scale output.
 MOE_DEVICE float* hs_at(const GemmArgs& g, int64_t pos, int64_t j) {
@@ -295,7 +310,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[T::R
                                               int64_t g1, bool g1_store, uint8_t* staging, float* smRed,
                                               const int32_t* smSlot, const float* smW) {
   constexpr int BM = T::BM, GROUPS = T::GROUPS;
-  const int tid = threadIdx.x;
+  const int tid = thread_id<T>();
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / T::WN;
@@ -461,7 +476,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
   float* smRed = reinterpret_cast<float*>(smem + T::OFF_RED);
   int32_t* smSlot = reinterpret_cast<int32_t*>(smem + T::OFF_ROW);
   float* smW = reinterpret_cast<float*>(smem + T::OFF_W);
-  const int tid = threadIdx.x;
+  const int tid = thread_id<T>();
   const int lane = tid & 63;
   // wave-uniform values live in scalar registers
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -799,38 +814,39 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
   tile_epilogue<T, FUSED>(g, acc, j, pos0, rows_avail, g0, g1, g1_store, smem, smRed, smSlot, smW);
 }
 
+// The fused outputs of the tile's rows [from, to), padding past the body's rows:
+// the zero codes and floor scales an all-zero row quantises to.
+template <class T>
+__device__ __forceinline__ void zero_rows(const GemmArgs& g, int64_t j, int64_t pos0, int from, int to) {
+  const int tid = thread_id<T>();
+  for (int ci = from * 8 + tid; ci < to * 8; ci += T::THREADS) {
+    const int row = ci >> 3, cc = ci & 7;
+    *reinterpret_cast<v4i*>(g.hq + (pos0 + row) * g.I + j * 128 + cc * 16) = (v4i){0, 0, 0, 0};
+  }
+  for (int row = from + tid; row < to; row += T::THREADS) *hs_at(g, pos0 + row, j) = kScaleFloor;
+}
+
 // A tile of a BM-row launch whose valid rows fit SUB rows, run with the
 // SUB-row body.  Positions [SUB, rows_avail) are padding: the fused outputs
 // there are the zero codes and floor scales an all-zero row quantises to.
-template <int SUB, int BM, bool FUSED, bool EXACT>
+template <int SUB, int BM, bool FUSED, bool EXACT, bool LOOP>
 __device__ __forceinline__ void short_tile(const GemmArgs& g, int64_t j, int64_t pos0, int rows_avail, int e,
                                            int nvalid) {
   static_assert(Tile<SUB>::THREADS == Tile<BM>::THREADS, "same workgroup size");
-  gemm_tile<Tile<SUB>, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, false);
-  if (FUSED) {
-    const int tid = threadIdx.x;
-    for (int ci = SUB * 8 + tid; ci < rows_avail * 8; ci += Tile<BM>::THREADS) {
-      const int row = ci >> 3, cc = ci & 7;
-      *reinterpret_cast<v4i*>(g.hq + (pos0 + row) * g.I + j * 128 + cc * 16) = (v4i){0, 0, 0, 0};
-    }
-    for (int row = SUB + tid; row < rows_avail; row += Tile<BM>::THREADS) *hs_at(g, pos0 + row, j) = kScaleFloor;
-  }
+  gemm_tile<Tile<SUB, 2, false, LOOP>, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, false);
+  if (FUSED) zero_rows<Tile<BM, 2, false, LOOP>>(g, j, pos0, SUB, rows_avail);
 }
 
 // Expert not local: zero output rows (kernels.py:112-120).
 template <class T, bool FUSED>
 __device__ __forceinline__ void zero_tile(const GemmArgs& g, int64_t j, int64_t pos0, int rows_avail) {
   if (!FUSED && g.accumulate) return;  // later K chunks leave C as it is (kernels.py:112-120)
-  const int tid = threadIdx.x;
+  const int tid = thread_id<T>();
   int64_t g0, g1;
   bool g1_store;
   groups_of<FUSED, T::GROUPS>(g, j, g0, g1, g1_store);
   if (FUSED) {
-    for (int ci = tid; ci < rows_avail * 8; ci += T::THREADS) {
-      const int row = ci >> 3, cc = ci & 7;
-      *reinterpret_cast<v4i*>(g.hq + (pos0 + row) * g.I + j * 128 + cc * 16) = (v4i){0, 0, 0, 0};
-    }
-    for (int row = tid; row < rows_avail; row += T::THREADS) *hs_at(g, pos0 + row, j) = kScaleFloor;
+    zero_rows<T>(g, j, pos0, 0, rows_avail);
   } else {
     constexpr int CH = T::GROUPS * 16;
     for (int ci = tid; ci < rows_avail * CH; ci += T::THREADS) {
@@ -851,17 +867,64 @@ constexpr int kernel_lds() {
   return BM == 256 && Tile<128>::LDS_BYTES > Tile<256>::LDS_BYTES ? Tile<128>::LDS_BYTES : Tile<BM>::LDS_BYTES;
 }
 
-// One workgroup of a BM-row launch: the tile map below, then the tile's body.
+// The tile with its rows' count known, by the body that fits it.
 // EXACT (fused W13 only) takes the dots on the bf16 matrix core; its 256-row
 // launch runs each tile as two 128-row bodies, since the bf16 fragments of the
 // 256-row body do not fit in the registers.
+template <int BM, bool FUSED, bool EXACT, bool LOOP = false>
+__device__ __forceinline__ void run_tile(const GemmArgs& g, int64_t j, int64_t pos0, int rows_avail, int e,
+                                         int nvalid, bool single) {
+  using T = Tile<BM, 2, false, LOOP>;
+  if constexpr (EXACT) {
+    // The second half of a 256-row align block whose slots all sit in its
+    // first half: padding only, written as the zero codes and floor scales
+    // that the two-body tile writes there.
+    if (nvalid == 0) {
+      zero_rows<T>(g, j, pos0, 0, rows_avail);
+      return;
+    }
+  }
+  // A tile with few valid rows (an expert's last rows, or a one-block tile of
+  // a run split over tiles) runs a shorter body: kTailRows rows, bound by
+  // streaming its weight tile with a three-deep LDS ring; or, in a 256-row
+  // launch, the 128-row body, whose eight waves split the 128 rows into 64 x 64
+  // subtiles instead of leaving half of the 256-row body's MFMAs on padding.
+  if constexpr (BM > kTailRows) {
+    if (nvalid <= kTailRows) {
+      short_tile<kTailRows, BM, FUSED, EXACT, LOOP>(g, j, pos0, rows_avail, e, nvalid);
+      return;
+    }
+  }
+  if constexpr (BM == 256) {
+    if (nvalid <= 128) {
+      short_tile<128, BM, FUSED, EXACT, LOOP>(g, j, pos0, rows_avail, e, nvalid);
+      return;
+    }
+    if constexpr (EXACT) {
+      // rows [0, 128) and then [128, rows_avail), whose valid rows are
+      // [128, nvalid); the barrier keeps the second body's first loads out of
+      // the LDS the first one's copy-out still reads
+      gemm_tile<Tile<128, 2, false, LOOP>, FUSED, EXACT>(g, j, pos0, 128, e, 128, false);
+      __syncthreads();
+      gemm_tile<Tile<128, 2, false, LOOP>, FUSED, EXACT>(g, j, pos0 + 128, rows_avail - 128, e, nvalid - 128, false);
+      return;
+    }
+  }
+  // Weight-streaming tiles (16 and 32 rows) of an expert with one row tile are
+  // the only readers of their weight tiles: those loads carry the
+  // non-temporal hint.  Experts with several row tiles, and taller tiles,
+  // share weight tiles through L2 and load them cached.
+  if constexpr (!(EXACT && BM == 256)) gemm_tile<T, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, BM <= 32 && single);
+}
+
+// One workgroup of a BM-row launch: the tile map below, then the tile's body.
 template <int BM, bool FUSED, bool EXACT>
 __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   using T = Tile<BM>;
   static_assert(FUSED || !EXACT, "the exact-dot form is built for the fused W13 GEMM");
   static_assert(BM <= kTailRows || Tile<kTailRows>::LDS_BYTES <= kernel_lds<BM>(),
                 "the short body must fit in the launch's LDS");
-  const int tid = threadIdx.x;
+  const int tid = thread_id<T>();
 
   // ---- expert-aligned, XCD-aware tile mapping ----------------------------
   // A workgroup computes one row tile by one n-tile.  Tiles are ordered
@@ -908,7 +971,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   int64_t back = 0, fwd = 0;
   int e;
   {
-    const int ln = threadIdx.x & 63;
+    const int ln = thread_id<T>() & 63;
     const int64_t ib = bq - 1 - ln, jf = bq + 1 + ln;
     e = g.eids[bq >> vsh];
     const int xb = ib >= 0 ? g.eids[ib >> vsh] : 0;
@@ -949,7 +1012,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   // Plain launches with a long K (kColMajorK and up: W2 of wide experts, whose
   // weight tiles are large) go column-major within a group instead: the row
   // tiles that share a weight tile start together.
-  constexpr int64_t GG = 4;  // 2, 8 and 16 (W13), 2, 3, 7 and 14 (W2) measured slower
+  constexpr int64_t GG = kTileGroup;
   const int64_t gj0 = in_run / (GG * units) * GG;
   const int64_t gsz = (g.n_tiles - gj0) < GG ? (g.n_tiles - gj0) : GG;
   const int64_t in_grp = in_run - gj0 * units;
@@ -972,50 +1035,137 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   bool row_valid = false;
   if (tid < BM && tid < rows_avail) row_valid = g.sorted[pos0 + tid] < g.S;
   const int nvalid = __syncthreads_count(row_valid);
-  if constexpr (EXACT) {
-    // The second half of a 256-row align block whose slots all sit in its
-    // first half: padding only, written as the zero codes and floor scales
-    // that the two-body tile writes there.
-    if (nvalid == 0) {
-      for (int ci = tid; ci < rows_avail * 8; ci += T::THREADS) {
-        const int row = ci >> 3, cc = ci & 7;
-        *reinterpret_cast<v4i*>(g.hq + (pos0 + row) * g.I + j * 128 + cc * 16) = (v4i){0, 0, 0, 0};
+  run_tile<BM, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, units == 1);
+}
+
+// The tile map of launches with few tiles a CU, from the layer's table of runs.
+// The map above deals every XCD the same number of blocks in expert order,
+// which is even when there are many, but where experts differ (skewed routing)
+// a block costs a whole tile or a fifth of one, and with one or two tiles a CU
+// the last of them decides.  Here the units (a run's row tiles by a group of
+// n-tiles) are dealt out to the XCDs in turn, there and back, by descending
+// rows, so that every XCD gets its share of each size and starts the long ones
+// first; the unit's tiles stay on one XCD and next to each other, as above.
+// When the XCD's last round of tiles would fill at most half of its CUs, those
+// tiles are split into two of half the rows.  One lane looks at one unit, and
+// the row counts come from the table: one round trip to memory.
+//
+// Layer times in expert order and so (us, one box): GroupGEMM shape, 1024
+// tokens, Zipf 237 / 212, uniform 230 / 218; Mixtral, 4096 tokens (W2: 2.3
+// tiles a CU, three rounds) 1660 / 1553, 1000 tokens, Zipf (128-row blocks in
+// 256-row tiles: half of a run's ids idle, on other XCDs than its tiles) 813 /
+// 530; exact dots, 777 tokens, 32 experts (1.1 tiles a CU) 140 / 120; Qwen3, 301
+// tokens 126 / 122.
+constexpr int kXcdCus = 32;
+
+// Workgroup l of XCD x runs its tile; returns how many workgroups the XCD's
+// tiles make (0 where there are none).
+template <int BM, bool FUSED, bool EXACT, bool LOOP>
+__device__ __forceinline__ int planned_run(const GemmArgs& g, int l) {
+  using T = Tile<BM, 2, false, LOOP>;
+  const int x = blockIdx.x % kXcds;
+  const int lane = thread_id<T>() & 63;
+  const int n_tiles = (int)g.n_tiles;
+  const int groups = (n_tiles + kTileGroup - 1) / kTileGroup;  // of n-tiles, as even as possible:
+  const int per_group = (n_tiles + groups - 1) / groups;
+  const int n_units = __builtin_amdgcn_readfirstlane(g.runs[0]) * groups;
+  const v4i* runs = reinterpret_cast<const v4i*>(g.runs + 4);
+  v4i r;
+  int w, n, incl;  // this lane's unit, its tiles, and those up to it
+  auto look = [&](int k) {
+    w = kXcds * k + ((k & 1) ? kXcds - 1 - x : x);
+    r = (v4i){0, 0, 0, 0};
+    n = 0;
+    if (w < g.E_routed * groups) r = runs[w / groups];  // beside the load of the count: one round trip
+    if (w < n_units) {
+      const int left = n_tiles - w % groups * per_group;
+      n = (r[1] + BM - 1) / BM * (left < per_group ? (left < 0 ? 0 : left) : per_group);
+    }
+    incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+  };
+  // this XCD's tiles, and the lane and the unit that tile l falls to
+  auto tiles_of = [&] {
+    int sum = 0;
+    for (int k0 = 0; kXcds * k0 < n_units; k0 += 64) {
+      look(k0 + lane);
+      sum += __builtin_amdgcn_readlane(incl, 63);
+    }
+    return sum;
+  };
+  const int mine = tiles_of();
+  int wgs = mine, half = -1;
+  if constexpr (BM >= 128 && !(EXACT && BM == 256)) {
+    const int rest = mine % kXcdCus;
+    if (rest <= kXcdCus / 2 && mine < 8 * kXcdCus) {
+      wgs += rest;
+      if (l >= mine - rest) {
+        half = (l - (mine - rest)) & 1;
+        l = mine - rest + (l - (mine - rest)) / 2;
       }
-      for (int row = tid; row < rows_avail; row += T::THREADS) *hs_at(g, pos0 + row, j) = kScaleFloor;
-      return;
     }
   }
-  // A tile with few valid rows (an expert's last rows, or a one-block tile of
-  // a run split over tiles) runs a shorter body: kTailRows rows, bound by
-  // streaming its weight tile with a three-deep LDS ring; or, in a 256-row
-  // launch, the 128-row body, whose eight waves split the 128 rows into 64 x 64
-  // subtiles instead of leaving half of the 256-row body's MFMAs on padding.
-  if constexpr (BM > kTailRows) {
-    if (nvalid <= kTailRows) {
-      short_tile<kTailRows, BM, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid);
-      return;
-    }
+  if (l >= mine) return wgs;
+  int before = 0;
+  uint64_t at = 0;
+  for (int k0 = 0;; k0 += 64) {
+    if (n_units > 64 * kXcds) look(k0 + lane);  // else the lanes still hold all of them
+    at = __ballot(before + incl > l);
+    if (at) break;
+    before += __builtin_amdgcn_readlane(incl, 63);
   }
-  if constexpr (BM == 256) {
-    if (nvalid <= 128) {
-      short_tile<128, BM, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid);
-      return;
-    }
-    if constexpr (EXACT) {
-      // rows [0, 128) and then [128, rows_avail), whose valid rows are
-      // [128, nvalid); the barrier keeps the second body's first loads out of
-      // the LDS the first one's copy-out still reads
-      gemm_tile<Tile<128>, FUSED, EXACT>(g, j, pos0, 128, e, 128, false);
-      __syncthreads();
-      gemm_tile<Tile<128>, FUSED, EXACT>(g, j, pos0 + 128, rows_avail - 128, e, nvalid - 128, false);
-      return;
-    }
+  const int src = __ffsll((unsigned long long)at) - 1;
+  const int in = l - before - __builtin_amdgcn_readlane(incl - n, src);  // tile of the unit
+  w = __builtin_amdgcn_readlane(w, src);
+  n = __builtin_amdgcn_readlane(n, src);
+  const int first = __builtin_amdgcn_readlane(r[0], src), cnt = __builtin_amdgcn_readlane(r[1], src);
+  const int padded = __builtin_amdgcn_readlane(r[3], src);
+  const int e = __builtin_amdgcn_readlane(r[2], src);
+  const int units = (cnt + BM - 1) / BM, gsz = n / units;
+  const bool by_col = !FUSED && g.K >= kColMajorK;
+  const int64_t j = w % groups * per_group + (by_col ? in / units : in % gsz);
+  const int r0 = (by_col ? in % units : in / gsz) * BM;
+  int64_t pos0 = first + r0;
+  int nvalid = cnt - r0 < BM ? cnt - r0 : BM;
+  int rows_avail = r0 + BM >= cnt ? padded - r0 : BM;  // the last tile has the run's padding
+  constexpr int H = BM / 2;
+  if (half == 0 && nvalid > H) {
+    nvalid = rows_avail = H;
+  } else if (half == 1) {
+    pos0 += H;
+    rows_avail -= H;
+    nvalid -= H;
+    if (nvalid <= 0) return wgs;  // nothing for the second half
   }
-  // Weight-streaming tiles (16 and 32 rows) of an expert with one row tile are
-  // the only readers of their weight tiles: those loads carry the
-  // non-temporal hint.  Experts with several row tiles, and taller tiles,
-  // share weight tiles through L2 and load them cached.
-  if constexpr (!(EXACT && BM == 256)) gemm_tile<Tile<BM>, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, BM <= 32 && units == 1);
+  if (e >= g.E) {  // a map to an expert that is not here
+    zero_tile<T, FUSED>(g, j, pos0, rows_avail);
+    return wgs;
+  }
+  run_tile<BM, FUSED, EXACT, LOOP>(g, j, pos0, rows_avail, e, nvalid, units == 1);
+  if (FUSED && rows_avail > BM) zero_rows<T>(g, j, pos0, BM, rows_avail);
+  return wgs;
+}
+
+template <int BM, bool FUSED, bool EXACT>
+__global__ __launch_bounds__(Tile<BM>::THREADS)
+__attribute__((amdgpu_waves_per_eu(Tile<BM>::NW / 4 * Tile<BM>::WG_PER_CU, Tile<BM>::NW / 4 * Tile<BM>::WG_PER_CU)))
+void planned_gemm_kernel(GemmArgs args) {
+  const int stride = gridDim.x / kXcds;
+  int l = blockIdx.x / kXcds;
+  const int wgs = planned_run<BM, FUSED, EXACT, false>(args, l);
+  // The grid is an estimate of an XCD's tiles: what is over (a routing more
+  // uneven than it allows for) is taken one tile after another.
+  for (l += stride; l < wgs; l += stride) {
+    __syncthreads();  // the next tile's loads go where the last one's epilogue reads
+    // as thread_id(): the arguments are read again for each tile
+    auto* kernarg = (const __attribute__((address_space(4))) GemmArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kernarg));
+    planned_run<BM, FUSED, EXACT, true>(*(const GemmArgs*)kernarg, l);
+  }
 }
 
 template <int BM, bool FUSED>
@@ -1048,7 +1198,7 @@ void w13_exact_kernel(GemmArgs g) {
 // same time whatever their order.
 template <class T, bool FUSED, bool EXACT>
 __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
-  const int tid = threadIdx.x;
+  const int tid = thread_id<T>();
   const int64_t b = blockIdx.x / (uint32_t)g.n_tiles, j = blockIdx.x % (uint32_t)g.n_tiles;
   const int64_t n_blocks = *g.ntpp / T::BM;
   // within max_padded for every b of the grid (the entries past ntpp are not used)
@@ -1095,6 +1245,23 @@ static int launch_flat(const GemmArgs& args, hipStream_t st) {
 }
 
 template <int BM, bool FUSED, bool EXACT>
+static int launch_planned(const GemmArgs& args, hipStream_t st) {
+  using T = Tile<BM>;
+  const void* fn = (const void*)planned_gemm_kernel<BM, FUSED, EXACT>;
+  static const hipError_t attr_rc =
+      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kernel_lds<BM>());
+  if (attr_rc != hipSuccess) return kErrLaunch;
+  // An even share of the expected tiles -- under an expert map twice the local
+  // experts' share of the slots -- and the halves of a split last round.
+  const int64_t here = 2 * args.E < args.E_routed ? 2 * args.E : args.E_routed;
+  const int64_t row_tiles = blocks_bound((args.S * here + args.E_routed - 1) / args.E_routed, here, BM);
+  const int64_t share = (row_tiles * args.n_tiles + kXcds - 1) / kXcds + kXcdCus / 2;
+  hipLaunchKernelGGL((planned_gemm_kernel<BM, FUSED, EXACT>), dim3((unsigned)(kXcds * share)), dim3(T::THREADS),
+                     kernel_lds<BM>(), st, args);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+template <int BM, bool FUSED, bool EXACT>
 static int launch_gemm(const GemmArgs& args, hipStream_t st) {
   // Launches whose tiles all find a CU of their own (see flat_gemm_body).
   if constexpr (BM <= 64) {
@@ -1104,6 +1271,17 @@ static int launch_gemm(const GemmArgs& args, hipStream_t st) {
       }
       if (args.max_blocks * args.n_tiles <= kCus) return launch_flat<BM, 2, FUSED, EXACT>(args, st);
     }
+  }
+
+  // Few tiles a CU (see planned_run): up to 20 of the tall tiles and 8 of the
+  // weight-streaming ones.  More of those (DeepSeek-V3 at 1000 tokens, 64 rows,
+  // 23 a CU) run 2-3 % slower than in expert order; the tall ones still gain
+  // there (Mixtral at 4096 tokens, 17 a CU, 6 %) or are even.  With at most BM
+  // slots every run is one tile and all are alike.
+  if constexpr (BM >= 32) {
+    constexpr int64_t most = (BM >= 128 ? 20 : 8) * kCus;
+    if (args.runs && args.tile_order == 0 && args.S > BM && args.run_tiles * args.n_tiles <= most)
+      return launch_planned<BM, FUSED, EXACT>(args, st);
   }
 
   using T = Tile<BM>;
@@ -1151,6 +1329,18 @@ static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int64_t E) {
   if (tile_m == 0) return S >= 160 * (int64_t)E ? 256 : BM;
   if (!block_m_ok(tile_m) || tile_m < BM || tile_m % BM != 0) return -1;
   return tile_m;
+}
+
+// What the layer knows of its blocks.
+static void set_blocks(GemmArgs& g, const LocalBlocks& local, int TM, int vshift) {
+  g.blk = local.blocks;
+  g.runs = local.runs;
+  if (local.E_routed > 0) {
+    const int64_t most = blocks_bound(g.S, local.E_routed, g.bma) << vshift;
+    if (most < g.max_blocks) g.max_blocks = most;
+    g.run_tiles = blocks_bound(g.S, local.E_routed, TM);
+    g.E_routed = (int)local.E_routed;
+  }
 }
 
 // 32-bit lane offsets: every A row and every expert's B block must be
@@ -1208,8 +1398,7 @@ int moe::plain_gemm(const void* A, const float* A_scale, const void* B, const fl
   g.tile_order = tile_order;
   dense_strides(g);
   if (scales_by_pos) g.as_pos_ld = max_padded;
-  g.blk = local.blocks;
-  if (local.max_blocks > 0 && local.max_blocks < g.max_blocks) g.max_blocks = local.max_blocks;
+  set_blocks(g, local, TM, 0);
   return dispatch_gemm<false>(TM, g, (hipStream_t)stream);
 }
 
@@ -1415,8 +1604,7 @@ int moe::w13_gemm(const void* Aq, const float* A_scale, const void* W13, const f
   g.E = E;
   dense_strides(g);
   if (scales_by_pos) g.as_pos_ld = g.hs_pos_ld = max_padded;
-  g.blk = local.blocks;
-  if (local.max_blocks > 0 && local.max_blocks << vshift < g.max_blocks) g.max_blocks = local.max_blocks << vshift;
+  set_blocks(g, local, TM, vshift);
   return exact ? dispatch_gemm<true, true>(TM, g, (hipStream_t)stream) : dispatch_gemm<true>(TM, g, (hipStream_t)stream);
 }
 

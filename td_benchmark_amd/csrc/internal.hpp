@@ -7,15 +7,22 @@ namespace moe {
 
 // What the layer knows of its blocks beyond the align outputs.  blocks: the list
 // of local blocks that align writes under an expert map (moe_layer's
-// local_blocks), null without one.  E_routed: the experts the slots are spread
-// over, for the choice of the tile height (0: E).  max_blocks: a bound on the
-// blocks of the launch (0: what fits in max_padded, which with few slots allows
-// for more).
+// local_blocks), null without one.  runs: the table of runs, or null.
+// E_routed: the experts the slots are spread over, for the choice of the tile
+// height and a bound on the blocks (0: E, and what fits in max_padded, which
+// with few slots allows for more).  A map may send several of them to one
+// local expert, so the local ones bound nothing.
 struct LocalBlocks {
   const int32_t* blocks = nullptr;
+  const int32_t* runs = nullptr;
   int64_t E_routed = 0;
-  int64_t max_blocks = 0;
 };
+
+// The table of runs that the one-launch align writes: [0] the experts with
+// slots here, then from [4] four words for each of them by descending rows
+// (equal ones by ascending expert): first position, rows, local expert id,
+// rows with padding.
+constexpr int64_t kRunsMaxSlots = 16384;
 
 // S slots over E experts fill at most this many blocks of BM: m <= min(S, E)
 // experts with c >= 1 slots have ceil(c/BM) <= 1 + (c-1)/BM blocks each.
@@ -46,10 +53,12 @@ int w13_gemm(const void* Aq, const float* A_scale, const void* W13, const float*
              void* stream, LocalBlocks local = {});
 
 // T == 0: align alone.  local: the lists to write under an expert map, or null;
-// top_k: the slots of a token (for its mask).
+// runs: the table of runs to write (S <= kRunsMaxSlots), or null; top_k: the
+// slots of a token (for its mask).
 int quant_align(const void* x, int64_t T, int64_t H, void* q, int64_t ldq, float* scales, const int32_t* topk_ids,
                 int64_t S, int32_t E, int32_t BM, const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids,
-                int32_t* ntpp, int64_t max_padded, void* workspace, int32_t* local, int32_t top_k, void* stream);
+                int32_t* ntpp, int64_t max_padded, void* workspace, int32_t* local, int32_t* runs, int32_t top_k,
+                void* stream);
 
 // The top-k sum of rows of H columns in D (row stride ldd) into y (row stride
 // H); addend rows (row stride lda) or null; with mask (a word per token) the

@@ -19,8 +19,7 @@ static LocalBlocks local_of(const moe_layer* l) {
   LocalBlocks r;
   r.E_routed = l->E_routed;
   if (l->expert_map) r.blocks = local_blk(l->local_blocks);
-  if (block_m_ok(l->block_size_m))
-    r.max_blocks = blocks_bound(l->T * l->top_k, l->expert_map ? l->E : l->E_routed, l->block_size_m);
+  if (l->T * l->top_k <= kRunsMaxSlots) r.runs = l->runs;
   return r;
 }
 
@@ -29,11 +28,14 @@ extern "C" int64_t moe_layer_local_blocks_bytes(int64_t T, int64_t max_padded, i
   return 4 * (1 + 2 * ((max_padded + BM - 1) / BM) + T);
 }
 
+extern "C" int64_t moe_layer_runs_bytes(int32_t E_routed) { return E_routed < 0 ? -1 : 16 * ((int64_t)E_routed + 1); }
+
 extern "C" int moe_layer_quant_align(const moe_layer* l, const void* hidden, const int32_t* topk_ids, void* stream) {
   if (!l || (l->expert_map && !l->local_blocks)) return kErrNullPointer;
   return quant_align(hidden, hidden ? l->T : 0, l->H, l->q1, l->Hp, l->s1, topk_ids, l->T * l->top_k, l->E_routed,
                      l->block_size_m, l->expert_map, l->sorted_ids, l->expert_ids, l->ntpp, l->max_padded,
-                     l->workspace, l->local_blocks, l->top_k, stream);
+                     l->workspace, l->local_blocks,
+                     l->T * l->top_k <= kRunsMaxSlots ? l->runs : nullptr, l->top_k, stream);
 }
 
 extern "C" int moe_layer_scales(const moe_layer* l, void* stream) {

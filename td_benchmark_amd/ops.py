@@ -829,6 +829,7 @@ class FusedExpertsRunner:
             (self.hs_pos if self.scales_by_position else self.hs).fill_(1e-12)
             n = int(lib().moe_layer_local_blocks_bytes(self.T, self.align.max_padded, self.BM))
             self.local_blocks = torch.empty(n // 4, dtype=torch.int32, device=dev)
+        self.runs = torch.empty(int(lib().moe_layer_runs_bytes(n_align)) // 4, dtype=torch.int32, device=dev)
         if out is not None:
             _need(out, "out", torch.bfloat16)
             if tuple(out.shape) != (self.T, H):
@@ -844,7 +845,7 @@ class FusedExpertsRunner:
             w13_scale=_ptr(w13_scale), w2=_ptr(w2), w2_scale=_ptr(w2_scale), expert_map=_ptr(self.expert_map),
             q1=_ptr(self.q1), s1=_ptr(self.s1), s1_pos=_ptr(self.s1_pos) if self.scales_by_position else None,
             sorted_ids=_ptr(a.sorted_ids), expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp),
-            workspace=_ptr(a.workspace), local_blocks=_ptr(self.local_blocks), hq=_ptr(self.hq),
+            workspace=_ptr(a.workspace), local_blocks=_ptr(self.local_blocks), runs=_ptr(self.runs), hq=_ptr(self.hq),
             hs=_ptr(self.hs_pos if self.scales_by_position else self.hs), D=_ptr(self.D))
 
     def _need_hidden(self, hidden: torch.Tensor) -> None:

@@ -43,8 +43,27 @@ def test_mapped_layer_equals_the_local_problem(T, H, E, k, BM, local, shared, ex
     ids2 = torch.from_numpy(np.sort((c.topk_ids + 1) % E, axis=1)[:, ::-1].copy()).cuda()
     off = torch.full_like(ids2, next((e for e in range(E) if e not in local), 0))
     for ids in (g["topk_ids"], ids2, off):
+        for r in (ep, loc):
+            r.D.fill_(3.0)  # a row that is not written shows
         y = ep.run(g["x"], g["topk_w"], ids).clone()
-        loc.D.zero_()
+        loc.D[(em[ids.long()] < 0).view(-1)] = 0
         want = loc.run(g["x"], g["topk_w"], em[ids.long()].contiguous())
         torch.cuda.synchronize()
         assert np.array_equal(bf16_bits(y), bf16_bits(want))
+
+
+def test_map_may_send_several_experts_to_one_local_expert():
+    """Replicated experts: 40 global ids on 2 local experts, more blocks than
+    the local experts could have rows of their own."""
+    from td_benchmark_amd import ops
+    print("case: replicated experts under a map", flush=True)
+    T, E, k = 90, 40, 4
+    c = make_case(T, 256, 256, E, k, 32, seed=3)
+    g = to_gpu(c)
+    w = [g[n][:2].contiguous() for n in ("w13", "w13_s", "w2", "w2_s")]
+    em = torch.from_numpy((np.arange(E) % 2).astype(np.int32)).cuda()
+    y = ops.FusedExpertsRunner(*w, T, k, 32, global_num_experts=E, expert_map=em).run(g["x"], g["topk_w"], g["topk_ids"])
+    loc = ops.FusedExpertsRunner(*w, T, k, 32)
+    want = loc.run(g["x"], g["topk_w"], em[g["topk_ids"].long()].contiguous())
+    torch.cuda.synchronize()
+    assert np.array_equal(bf16_bits(y), bf16_bits(want))
