@@ -342,6 +342,13 @@ int moe_layer_w2(const moe_layer* layer, const float* topk_weights, void* stream
 int moe_layer_reduce(const moe_layer* layer, const void* addend, int64_t addend_ld, int64_t cols, void* y,
                      void* stream);
 
+/* The stages in order, in one call.  shared: NULL, or the shared expert as a
+ * layer of one expert and top_k 1 over the same T and Hp, whose q1, s1 are this
+ * layer's and whose align outputs are prepared (every token to expert 0); its
+ * rows are the addend of the top-k sum. */
+int moe_layer_run(const moe_layer* layer, const moe_layer* shared, const void* hidden, const float* topk_weights,
+                  const int32_t* topk_ids, int64_t cols, void* y, void* stream);
+
 /* FP8 reduce-scatter combine -- the dequantise-and-sum of the FP8 chunks a
  * rank receives in the FP8-compressed reduce-scatter leg, replacing
  * `(fp8.to(float32) * scale.repeat_interleave(128)).sum(dim=0).to(bfloat16)`

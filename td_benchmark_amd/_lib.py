@@ -87,6 +87,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "moe_layer_w13": (ctypes.c_int, [_LAYER, _P]),
     "moe_layer_w2": (ctypes.c_int, [_LAYER, _P, _P]),
     "moe_layer_reduce": (ctypes.c_int, [_LAYER, _P, _i64, _i64, _P, _P]),
+    "moe_layer_run": (ctypes.c_int, [_LAYER, _LAYER, _P, _P, _P, _i64, _P, _P]),
     "moe_silu_and_mul": (ctypes.c_int, [_P, _i64, _i64, _P, _P]),
     "moe_reduce_topk": (ctypes.c_int, [_P, _i64, _i32, _i64, _P, _P]),
 }

@@ -69,3 +69,19 @@ extern "C" int moe_layer_reduce(const moe_layer* l, const void* addend, int64_t 
   return reduce_topk(l->D, l->Hp, addend, addend_ld, l->T, l->top_k, cols,
                      l->expert_map ? local_mask(l->local_blocks, l->max_padded, l->block_size_m) : nullptr, y, stream);
 }
+
+extern "C" int moe_layer_run(const moe_layer* l, const moe_layer* shared, const void* hidden,
+                             const float* topk_weights, const int32_t* topk_ids, int64_t cols, void* y,
+                             void* stream) {
+  if (!l) return kErrNullPointer;
+  if (shared && (shared->T != l->T || shared->Hp != l->Hp || shared->top_k != 1)) return kErrBadShape;
+  if (l->T > 0 && !hidden) return kErrNullPointer;
+  int rc = moe_layer_quant_align(l, hidden, topk_ids, stream);
+  if (rc == kOk) rc = moe_layer_scales(l, stream);
+  if (rc == kOk) rc = moe_layer_w13(l, stream);
+  if (rc == kOk) rc = moe_layer_w2(l, topk_weights, stream);
+  if (rc == kOk && shared) rc = moe_layer_w13(shared, stream);
+  if (rc == kOk && shared) rc = moe_layer_w2(shared, nullptr, stream);
+  if (rc == kOk) rc = moe_layer_reduce(l, shared ? shared->D : nullptr, shared ? shared->Hp : 0, cols, y, stream);
+  return rc;
+}

@@ -35,12 +35,16 @@ _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _CUR_DEVICE = getattr(torch._C, "_cuda_getDevice", None)
 
 
-def _stream(stream: torch.cuda.Stream | None = None) -> ctypes.c_void_p:
+def _stream_handle(stream: torch.cuda.Stream | None = None) -> int:
     if stream is None:
         if _RAW_STREAM is not None and _CUR_DEVICE is not None:
-            return ctypes.c_void_p(_RAW_STREAM(_CUR_DEVICE()))
+            return _RAW_STREAM(_CUR_DEVICE())
         stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    return stream.cuda_stream
+
+
+def _stream(stream: torch.cuda.Stream | None = None) -> ctypes.c_void_p:
+    return ctypes.c_void_p(_stream_handle(stream))
 
 
 def _need(t: torch.Tensor, name: str, dtype: torch.dtype | None = None,
@@ -722,6 +726,39 @@ class SharedExpertRunner:
         return out[:, : self.H]
 
 
+def _need_layer_weights(w13: torch.Tensor, w13_scale: torch.Tensor, w2: torch.Tensor,
+                        w2_scale: torch.Tensor) -> tuple[int, int, int]:
+    """The two weights of a layer and their scales -> (E, H, I)."""
+    E, N2, H = _need_weights(w13, w13_scale, "w13")
+    _need_weights(w2, w2_scale, "w2")
+    if w2.shape != (E, H, N2 // 2):
+        raise ValueError(f"w2 shape {tuple(w2.shape)} does not match w13 {tuple(w13.shape)}")
+    if (N2 // 2) % 128:
+        raise ValueError(f"the intermediate size {N2 // 2} must be a multiple of 128")
+    return E, H, N2 // 2
+
+
+def _routed_experts(E: int, global_num_experts: int | None, expert_map: torch.Tensor | None,
+                    device: torch.device) -> tuple[torch.Tensor | None, int]:
+    """(expert map as int32 on the device or None, the experts the ids select from)."""
+    if expert_map is not None:
+        expert_map = expert_map.to(device=device, dtype=torch.int32).contiguous()
+        n = int(global_num_experts or expert_map.numel())
+        if expert_map.numel() != n:
+            raise ValueError("expert_map must have global_num_experts entries")
+        return expert_map, n
+    if global_num_experts not in (None, -1, E):
+        raise ValueError("global_num_experts != local experts needs an expert_map")
+    return None, E
+
+
+def _layer_block_m(block_size_m: int | None, num_tokens: int, n_experts: int, top_k: int) -> int:
+    bm = block_size_m or get_moe_config(num_tokens, n_experts, top_k)["BLOCK_SIZE_M"]
+    if bm not in SUPPORTED_BLOCK_M:
+        raise ValueError(f"block_size_m must be one of {SUPPORTED_BLOCK_M}")
+    return bm
+
+
 class FusedExpertsRunner:
     """Prebuilt A1->A9 chain for fixed (T, H, I, E, top_k, BM).
 
@@ -769,32 +806,17 @@ class FusedExpertsRunner:
                  shared: SharedExpertRunner | None = None, out: torch.Tensor | None = None,
                  global_num_experts: int | None = None, expert_map: torch.Tensor | None = None,
                  tile_m: int = 0, scales_by_position: bool | None = None, exact_dot: bool = False):
-        E, N2, H = _need_weights(w13, w13_scale, "w13")
-        _need_weights(w2, w2_scale, "w2")
-        if w2.shape != (E, H, N2 // 2):
-            raise ValueError(f"w2 shape {tuple(w2.shape)} does not match w13 {tuple(w13.shape)}")
-        if (N2 // 2) % 128:
-            raise ValueError(f"the intermediate size {N2 // 2} must be a multiple of 128")
-        self.E, self.H, self.I, self.T, self.top_k = E, H, N2 // 2, num_tokens, top_k
+        E, H, I = _need_layer_weights(w13, w13_scale, w2, w2_scale)
+        self.E, self.H, self.I, self.T, self.top_k = E, H, I, num_tokens, top_k
         self.exact_dot = bool(exact_dot)
         self.Hp = Hp = _blocks128(H) * 128
         w13, w2 = _pad_fp8(w13, 2, Hp), _pad_fp8(w2, 1, Hp)
         self.S = num_tokens * top_k
         # Expert parallelism: align over the global experts, GEMMs over the
         # blocks of the local ones.
-        self.expert_map = None
-        n_align = E
-        if expert_map is not None:
-            self.expert_map = expert_map.to(device=w13.device, dtype=torch.int32).contiguous()
-            n_align = int(global_num_experts or self.expert_map.numel())
-            if self.expert_map.numel() != n_align:
-                raise ValueError("expert_map must have global_num_experts entries")
-        elif global_num_experts not in (None, -1, E):
-            raise ValueError("global_num_experts != local experts needs an expert_map")
+        self.expert_map, n_align = _routed_experts(E, global_num_experts, expert_map, w13.device)
         # the slots are spread over all n_align experts, local or not
-        self.BM = block_size_m or get_moe_config(num_tokens, n_align, top_k)["BLOCK_SIZE_M"]
-        if self.BM not in SUPPORTED_BLOCK_M:
-            raise ValueError(f"block_size_m must be one of {SUPPORTED_BLOCK_M}")
+        self.BM = _layer_block_m(block_size_m, num_tokens, n_align, top_k)
         # GEMM workgroup tile rows (0 = automatic; never changes the results)
         self.tile_m = int(tile_m)
         if self.tile_m and (self.tile_m not in SUPPORTED_BLOCK_M or self.tile_m % self.BM):
@@ -847,6 +869,17 @@ class FusedExpertsRunner:
             sorted_ids=_ptr(a.sorted_ids), expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp),
             workspace=_ptr(a.workspace), local_blocks=_ptr(self.local_blocks), runs=_ptr(self.runs), hq=_ptr(self.hq),
             hs=_ptr(self.hs_pos if self.scales_by_position else self.hs), D=_ptr(self.D))
+        # the shared expert as a layer of one expert on this layer's FP8 input
+        self._shared_layer = self._shared_view = None
+        if shared is not None:
+            s = shared._align_for(num_tokens)
+            self._shared_layer = MoeLayer(
+                T=self.T, H=H, Hp=Hp, I=shared.I, max_padded=s.max_padded, top_k=1, E=1, E_routed=1,
+                block_size_m=shared.BM, tile_m=0, exact_dot=0, w13=_ptr(shared.w1), w13_scale=_ptr(shared.w1_scale),
+                w2=_ptr(shared.w2), w2_scale=_ptr(shared.w2_scale), q1=_ptr(self.q1), s1=_ptr(self.s1),
+                sorted_ids=_ptr(s.sorted_ids), expert_ids=_ptr(s.expert_ids), ntpp=_ptr(s.ntpp),
+                workspace=_ptr(s.workspace), hq=_ptr(shared.hq), hs=_ptr(shared.hs), D=_ptr(shared.out))
+            self._shared_view = shared.out[: self.T, :H]
 
     def _need_hidden(self, hidden: torch.Tensor) -> None:
         _need(hidden, "hidden_states", torch.bfloat16)
@@ -866,14 +899,6 @@ class FusedExpertsRunner:
         self.align.need_ids(topk_ids, self.expert_map)
         check(lib().moe_layer_quant_align(self._layer, None, _ptr(topk_ids), _stream()), "moe_layer_quant_align")
 
-    def stage_quant_align(self, hidden: torch.Tensor, topk_ids: torch.Tensor) -> None:
-        """stage_quant and stage_align, which do not depend on each other, in
-        one launch where both are small."""
-        self._need_hidden(hidden)
-        self.align.need_ids(topk_ids, self.expert_map)
-        check(lib().moe_layer_quant_align(self._layer, _ptr(hidden), _ptr(topk_ids), _stream()),
-              "moe_layer_quant_align")
-
     def stage_scales(self) -> None:
         """The activation scales K-major by sorted position for the W13 GEMM
         (nothing to do on the row-major path)."""
@@ -884,10 +909,13 @@ class FusedExpertsRunner:
         self._layer.exact_dot = int(self.exact_dot)
         check(lib().moe_layer_w13(self._layer, _stream()), "moe_layer_w13")
 
-    def stage_w2(self, topk_weights: torch.Tensor) -> None:
+    def _need_weights_of_slots(self, topk_weights: torch.Tensor) -> None:
         _need(topk_weights, "topk_weights", torch.float32)
         if topk_weights.numel() != self.S:
             raise ValueError(f"topk_weights has {topk_weights.numel()} entries for {self.S} slots")
+
+    def stage_w2(self, topk_weights: torch.Tensor) -> None:
+        self._need_weights_of_slots(topk_weights)
         check(lib().moe_layer_w2(self._layer, _ptr(topk_weights), _stream()), "moe_layer_w2")
 
     def stage_shared(self) -> None:
@@ -907,12 +935,19 @@ class FusedExpertsRunner:
             self.y.copy_(self.y_pad[:, : self.H])
 
     def run(self, hidden: torch.Tensor, topk_weights: torch.Tensor, topk_ids: torch.Tensor) -> torch.Tensor:
-        self.stage_quant_align(hidden, topk_ids)
-        self.stage_scales()
-        self.stage_w13()
-        self.stage_w2(topk_weights)
-        self.stage_shared()
-        self.stage_reduce()
+        self._need_hidden(hidden)
+        self.align.need_ids(topk_ids, self.expert_map)
+        self._need_weights_of_slots(topk_weights)
+        layer, shared = self._layer, self._shared_layer
+        layer.exact_dot = int(self.exact_dot)
+        if shared is not None:
+            self.shared.exact_dot = self.exact_dot
+            shared.exact_dot = layer.exact_dot
+            self.shared_out = self._shared_view
+        check(lib().moe_layer_run(layer, shared, hidden.data_ptr(), topk_weights.data_ptr(), topk_ids.data_ptr(),
+                                  self.y_pad.shape[1], self.y_pad.data_ptr(), _stream_handle()), "moe_layer_run")
+        if self.y_pad is not self.y:
+            self.y.copy_(self.y_pad[:, : self.H])
         return self.y
 
     def capture(self, hidden: torch.Tensor, topk_weights: torch.Tensor, topk_ids: torch.Tensor) -> "LayerGraph":
@@ -1106,7 +1141,41 @@ def fused_experts(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tenso
         raise ValueError("fused_experts needs w1_scale and w2_scale")
     T, k = topk_ids.shape
     gne = None if global_num_experts in (-1, None) else global_num_experts
-    runner = FusedExpertsRunner(w1, w1_scale, w2, w2_scale, T, k, block_size_m,
-                                global_num_experts=gne, expert_map=expert_map, exact_dot=exact_dot)
-    return runner.run(hidden_states.contiguous(), topk_weights.contiguous().view(-1),
-                      topk_ids.contiguous().view(-1)).clone()
+    hidden_states, topk_weights, topk_ids = hidden_states.contiguous(), topk_weights.contiguous(), topk_ids.contiguous()
+    if w1.dim() != 3 or w1.shape[2] % 128:  # a ragged hidden size pads the weights, which the runner does
+        runner = FusedExpertsRunner(w1, w1_scale, w2, w2_scale, T, k, block_size_m, global_num_experts=gne,
+                                    expert_map=expert_map, exact_dot=exact_dot)
+        return runner.run(hidden_states, topk_weights.view(-1), topk_ids.view(-1))
+    # What FusedExpertsRunner builds, with all buffers in one allocation.
+    E, H, I = _need_layer_weights(w1, w1_scale, w2, w2_scale)
+    expert_map, n_align = _routed_experts(E, gne, expert_map, w1.device)
+    bm = _layer_block_m(block_size_m, T, n_align, k)
+    S = T * k
+    _need(hidden_states, "hidden_states", torch.bfloat16)
+    if tuple(hidden_states.shape) != (T, H):
+        raise ValueError(f"hidden_states must be [{T}, {H}]")
+    _need(topk_ids, "topk_ids", torch.int32)
+    _need(topk_weights, "topk_weights", torch.float32)
+    if topk_weights.numel() != S:
+        raise ValueError(f"topk_weights has {topk_weights.numel()} entries for {S} slots")
+    L = lib()
+    mp = int(L.moe_align_max_padded(S, n_align, bm))
+    G = H // 128
+    by_pos = gemm_tile_rows(bm, S, n_align) >= 128
+    sizes = {"q1": T * H, "s1": 4 * T * G, "s1_pos": 4 * G * mp if by_pos else 0, "sorted_ids": 4 * mp,
+             "expert_ids": 4 * -(-mp // bm), "ntpp": 4, "workspace": int(L.moe_align_workspace_bytes(S, n_align)),
+             "local_blocks": 0 if expert_map is None else int(L.moe_layer_local_blocks_bytes(T, mp, bm)),
+             "runs": int(L.moe_layer_runs_bytes(n_align)), "hq": mp * I, "hs": 4 * mp * (I // 128), "D": 2 * S * H}
+    block = torch.empty(sum((n + 255 & ~255) + 256 for n in sizes.values()), dtype=torch.uint8, device=w1.device)
+    y = torch.empty((T, H), dtype=torch.bfloat16, device=w1.device)
+    layer = MoeLayer(T=T, H=H, Hp=H, I=I, max_padded=mp, top_k=k, E=E, E_routed=n_align, block_size_m=bm, tile_m=0,
+                     exact_dot=int(exact_dot), w13=w1.data_ptr(), w13_scale=w1_scale.data_ptr(), w2=w2.data_ptr(),
+                     w2_scale=w2_scale.data_ptr(), expert_map=None if expert_map is None else expert_map.data_ptr())
+    at = block.data_ptr()
+    for name, n in sizes.items():
+        if n or name not in ("s1_pos", "local_blocks"):  # those two are absent, not empty
+            setattr(layer, name, at)
+        at += (n + 255 & ~255) + 256
+    check(L.moe_layer_run(layer, None, hidden_states.data_ptr(), topk_weights.data_ptr(), topk_ids.data_ptr(), H,
+                          y.data_ptr(), _stream_handle()), "moe_layer_run")
+    return y

@@ -1,0 +1,62 @@
+"""GPU: fused_experts, whose buffers share one allocation, equals the runner bit
+for bit (one token, both scale layouts, an expert map, exact dots, non-contiguous
+inputs, no tokens), and one call of moe_layer_run equals the stages one by one,
+with a shared expert built for more tokens than the layer's."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from moe_cases import bf16_bits, make_case, to_gpu
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+# (T, H, E, k, BM, mapped, exact)
+CASES = [(1, 256, 8, 2, None, False, False), (300, 384, 6, 3, 128, False, True), (90, 256, 8, 2, 32, True, False),
+         (40, 200, 4, 1, None, False, False), (0, 256, 8, 2, None, False, False)]
+
+
+@pytest.mark.parametrize("T,H,E,k,BM,mapped,exact", CASES)
+def test_call_equals_runner(T, H, E, k, BM, mapped, exact):
+    from td_benchmark_amd import ops
+    print(f"case: call T={T} H={H} E={E} k={k} BM={BM} mapped={mapped} exact={exact}", flush=True)
+    c = make_case(max(T, 1), H, 256, E, k, BM or 32, seed=T + H)
+    g = to_gpu(c)
+    w = [g[n] for n in ("w13", "w13_s", "w2", "w2_s")]
+    em = None
+    if mapped:
+        w = [t[: E // 2].contiguous() for t in w]
+        em = torch.tensor([e // 2 if e % 2 else -1 for e in range(E)], dtype=torch.int64)  # any integer type, any device
+    x, wt, ids = g["x"][:T], g["topk_w"][:T], g["topk_ids"][:T]
+    want = ops.FusedExpertsRunner(*w, T, k, BM, global_num_experts=E if mapped else None, expert_map=em,
+                                  exact_dot=exact).run(x.contiguous(), wt.contiguous(), ids.contiguous())
+    strided = [torch.stack((t, t), dim=1)[:, 0] for t in (x, wt, ids)] if T else [x, wt, ids]
+    y = ops.fused_experts(strided[0], w[0], w[2], strided[1], strided[2], global_num_experts=E if mapped else -1,
+                          w1_scale=w[1], w2_scale=w[3], block_size_m=BM, expert_map=em, exact_dot=exact)
+    torch.cuda.synchronize()
+    assert tuple(y.shape) == (T, H) and np.array_equal(bf16_bits(y), bf16_bits(want))
+
+
+def test_one_call_equals_the_stages():
+    from td_benchmark_amd import ops
+    print("case: stages one by one, shared expert", flush=True)
+    T, E, k = 70, 8, 2
+    c = make_case(T, 256, 256, E, k, 32, seed=4)
+    g = to_gpu(c)
+    w = [g[n] for n in ("w13", "w13_s", "w2", "w2_s")]
+    r = ops.FusedExpertsRunner(*w, T, k, shared=ops.SharedExpertRunner(*[t[1:2].contiguous() for t in w], 200))
+    for exact in (False, True, False):
+        r.exact_dot = exact
+        y = r.run(g["x"], g["topk_w"], g["topk_ids"]).clone()
+        out = r.shared_out.clone()
+        r.stage_quant(g["x"])
+        r.stage_align(g["topk_ids"])
+        r.stage_scales()
+        r.stage_w13()
+        r.stage_w2(g["topk_w"])
+        r.stage_shared()
+        r.stage_reduce()
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(y), bf16_bits(r.y)) and np.array_equal(bf16_bits(out), bf16_bits(r.shared_out))
