@@ -324,6 +324,8 @@ typedef struct moe_layer {
   int32_t* local_blocks;      /* moe_layer_local_blocks_bytes, with expert_map; else NULL */
   int32_t* runs;              /* moe_layer_runs_bytes, 16-byte aligned: align's notes on the experts' rows for the
                                  GEMMs' tile order; NULL: without */
+  int32_t* share;             /* moe_layer_share_bytes, 16-byte aligned, the first 512 bytes zero before the first
+                                 run: lets several workgroups share a W13 tile in small decode; NULL: without */
   void* hq;                   /* [max_padded, I] e4m3fn */
   float* hs;                  /* [I/128, max_padded] with s1_pos, else [max_padded, I/128] */
   void* D;                    /* [T * top_k, Hp] bf16 */
@@ -331,6 +333,7 @@ typedef struct moe_layer {
 
 int64_t moe_layer_local_blocks_bytes(int64_t T, int64_t max_padded, int32_t block_size_m);
 int64_t moe_layer_runs_bytes(int32_t E_routed);
+int64_t moe_layer_share_bytes(void);
 /* hidden [T, H] bf16 (NULL: align alone), topk_ids [T, top_k]. */
 int moe_layer_quant_align(const moe_layer* layer, const void* hidden, const int32_t* topk_ids, void* stream);
 /* The activation scales by sorted position (nothing where s1_pos is NULL). */

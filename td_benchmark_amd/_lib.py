@@ -38,7 +38,7 @@ class MoeLayer(ctypes.Structure):
     _fields_ = ([(n, _i64) for n in ("T", "H", "Hp", "I", "max_padded")]
                 + [(n, _i32) for n in ("top_k", "E", "E_routed", "block_size_m", "tile_m", "exact_dot")]
                 + [(n, _P) for n in ("w13", "w13_scale", "w2", "w2_scale", "expert_map", "q1", "s1", "s1_pos",
-                                     "sorted_ids", "expert_ids", "ntpp", "workspace", "local_blocks", "runs", "hq", "hs", "D")])
+                                     "sorted_ids", "expert_ids", "ntpp", "workspace", "local_blocks", "runs", "share", "hq", "hs", "D")])
 
 
 _LAYER = ctypes.POINTER(MoeLayer)
@@ -82,6 +82,7 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                                      _i64, _i32, _i32, _i64, _i32, _i32, _P, _P, _P]),
     "moe_layer_local_blocks_bytes": (ctypes.c_int64, [_i64, _i64, _i32]),
     "moe_layer_runs_bytes": (ctypes.c_int64, [_i32]),
+    "moe_layer_share_bytes": (ctypes.c_int64, []),
     "moe_layer_quant_align": (ctypes.c_int, [_LAYER, _P, _P, _P]),
     "moe_layer_scales": (ctypes.c_int, [_LAYER, _P]),
     "moe_layer_w13": (ctypes.c_int, [_LAYER, _P]),

@@ -217,6 +217,7 @@ struct AlignArgs {
   int32_t* ntpp;
   int32_t* local;  // the lists of local blocks and slots, or null (see internal.hpp)
   int32_t* runs;   // the table of runs, or null (see internal.hpp)
+  int32_t* share;  // the counters of shared tiles to clear, or null
   int64_t max_padded;
   int S, E, BM, top_k;
 };
@@ -333,6 +334,7 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   }
   if (a.runs && tid == 0 && cnt > 0 && local >= 0)
     reinterpret_cast<v4i*>(a.runs + 4)[place] = (v4i){before, cnt, local, padded};
+  if (a.share && e == 0 && tid < kShareTiles) a.share[tid] = 0;
   if (e == 0 && tid == 0) {
     *a.ntpp = total;
     if (a.local) *a.local = ltotal;
@@ -445,13 +447,13 @@ static void by_slots(int64_t S, F&& f) {
 static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
                       int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded,
                       void* workspace, void* stream, int32_t* local = nullptr, int32_t* runs = nullptr,
-                      int32_t top_k = 1) {
+                      int32_t* share = nullptr, int32_t top_k = 1) {
   const int arg_rc = align_args(topk_ids, S, E, BM, sorted_ids, expert_ids, ntpp, max_padded, true, workspace);
   if (arg_rc != kOk) return arg_rc;
   if (!expert_map) local = nullptr;
   hipStream_t st = (hipStream_t)stream;
   if (S <= kAlignOneLaunchSlots) {
-    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs,
+    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share,
                       max_padded, (int)S, (int)E, (int)BM, (int)top_k};
     by_slots(S, [&](auto it) {
       hipLaunchKernelGGL(align_expert_kernel<decltype(it)::value>, dim3((unsigned)E), dim3(kAlignThreads), 0, st, a);
@@ -495,7 +497,7 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
 int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq, float* scales,
                      const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
                      int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded, void* workspace,
-                     int32_t* local, int32_t* runs, int32_t top_k, void* stream) {
+                     int32_t* local, int32_t* runs, int32_t* share, int32_t top_k, void* stream) {
   // both halves' arguments before either is launched
   if (top_k <= 0) return kErrBadTopK;
   if (T < 0 || H < 0 || ldq < (H + 127) / 128 * 128) return kErrBadShape;
@@ -511,10 +513,10 @@ int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int6
     const int qrc = moe_quant_group128_padded(x_bf16, T, H, q_fp8, ldq, scales, stream);
     if (qrc != kOk) return qrc;
     return align_impl(topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp, max_padded, workspace, stream,
-                      local, runs, top_k);
+                      local, runs, share, top_k);
   }
   if (!expert_map) local = nullptr;
-  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs,
+  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share,
                       max_padded, (int)S, (int)E, (int)BM, (int)top_k};
   const unsigned grid = (unsigned)(E + (q.n_chunks + kAlignThreads - 1) / kAlignThreads);
   by_slots(S, [&](auto it) {
@@ -532,7 +534,7 @@ extern "C" int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q
                                const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp,
                                int64_t max_padded, void* workspace, void* stream) {
   return quant_align(x_bf16, T, H, q_fp8, ldq, scales, topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp,
-                     max_padded, workspace, nullptr, nullptr, 1, stream);
+                     max_padded, workspace, nullptr, nullptr, nullptr, 1, stream);
 }
 
 extern "C" int moe_align_block_size(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,

@@ -103,11 +103,16 @@ constexpr int kScaleLag = 2;
 // launches); DEEP: the form for launches whose tiles all run at once, one
 // workgroup per CU with as deep a ring as the LDS holds, filled by waves that do
 // nothing else (see flat_gemm_body).
-template <int BM_, int GROUPS_ = 2, bool DEEP_ = false, bool LOOP_ = false>
+// W: weight rows of each group (128, or 32 or 64 in the parts of a deep fused
+// tile that several workgroups share, see share_quant).
+template <int BM_, int GROUPS_ = 2, bool DEEP_ = false, bool LOOP_ = false, int W_ = 128>
 struct Tile {
   static constexpr int BM = BM_;
   static constexpr int GROUPS = GROUPS_;
+  static constexpr int W = W_;
+  static constexpr int PARTS = 128 / W;  // workgroups that share a tile
   static_assert(GROUPS == 2 || (DEEP_ && BM <= 64), "narrow tiles are deep and short");
+  static_assert(W == 128 || (DEEP_ && GROUPS == 2 && BM >= 32 && (W == 32 || W == 64)), "parts are of deep tiles");
   static constexpr bool DEEP = DEEP_;
   static constexpr bool LOOP = LOOP_;  // the workgroup runs several tiles
   static constexpr int NW = DEEP || BM >= 32 ? 8 : 4;  // waves per workgroup (2 per SIMD at 8)
@@ -115,23 +120,24 @@ struct Tile {
   static constexpr int CW = DEEP ? 4 : NW;  // waves that compute: the first ones
   static constexpr int PW = DEEP ? 4 : NW;  // waves that issue the loads: the last ones
   // compute waves along M: 4 x 2 waves of 64 x 128 at BM = 256 (fewer LDS bytes per MFMA)
-  static constexpr int WM = BM == 256 ? 4 : ((CW == 8 || BM == 128) ? 2 : 1);
+  static constexpr int WM = BM == 256 ? 4 : ((CW == 8 || BM == 128 || W == 32) ? 2 : 1);
   // LDS ring depth: three 64 KiB stages of the 256-row tile exceed 160 KiB;
   // the 34 KiB stages of the 16-row tile (weight streaming) fit four; the
   // 32-row tile runs two workgroups per CU with two 36 KiB stages each, so one
   // workgroup's pipeline fill and epilogue overlap the other's weight stream
-  static constexpr int KS = GROUPS == 1 ? (BM == 64 ? 6 : 7)
+  static constexpr int KS = W == 32        ? (BM == 64 ? 8 : 10)
+                            : W * GROUPS == 128 ? (BM == 64 ? 6 : 7)
                             : BM == 256 || (BM == 32 && !DEEP_) ? 2
                                                                 : (BM <= 32 ? 4 : 3);
   static constexpr int WG_PER_CU = BM == 32 && !DEEP_ ? 2 : 1;
   static constexpr int WN = CW / WM;              // compute waves along N
   static constexpr int RS = BM / WM / 16;         // 16-row subtiles per wave
-  static constexpr int CS = 8 / WN;               // 16-col subtiles per wave per group
+  static constexpr int CS = W / 16 / WN;          // 16-col subtiles per wave per group
   static constexpr int A_BYTES = BM * 128;
-  static constexpr int B_BYTES = GROUPS * 128 * 128;
+  static constexpr int B_BYTES = GROUPS * W * 128;
   static constexpr int STAGE = A_BYTES + B_BYTES;
   static constexpr int NA = BM / 8;               // 1 KiB A DMA instructions per stage
-  static constexpr int NB = GROUPS * 16;          // 1 KiB B DMA instructions per stage
+  static constexpr int NB = GROUPS * W / 8;       // 1 KiB B DMA instructions per stage
   static constexpr int NS = (BM + 63) / 64;       // 256 B A-scale DMA instructions per stage
   static constexpr int NA_W = (NA + PW - 1) / PW; // A instructions of the busiest loading wave
   static constexpr int NB_W = NB / PW;            // B instructions per loading wave
@@ -169,6 +175,7 @@ struct GemmArgs {
   // blocks are no part of the launch.
   const int32_t* blk;
   const int32_t* runs;     // the experts' runs by descending rows (see internal.hpp), or null
+  int32_t* share;          // fused: counters and rows of tiles that several workgroups share, or null
   const float* topk_w;     // [S] or null
   uint16_t* C;             // bf16 [S, N]            (plain epilogue)
   uint8_t* hq;             // fp8 [max_padded, I]    (fused epilogue)
@@ -447,6 +454,77 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[T::R
   }
 }
 
+// The epilogue of a fused tile whose 128 columns are computed by T::PARTS
+// workgroups, W columns each: a group's scale needs all of them, so every
+// workgroup leaves its h (bf16, as the quant takes it) in global memory and the
+// last one to arrive at the tile's counter quantises the group and puts the
+// counter back to zero.  Nobody waits for anybody.  The rows go through
+// agent-scope atomics (written to and read from beyond the XCDs' L2s); each wave
+// waits for its stores before the workgroup counts itself in.  A release and an
+// acquire fence around plain accesses write back and invalidate an L2 each time:
+// with 192 workgroups they took about 10 us.
+template <class T>
+__device__ __forceinline__ void share_quant(const GemmArgs& g, v4f (&acc)[T::RS][T::GROUPS][T::CS], int64_t j,
+                                            int64_t pos0, int rows_avail, int part, int tile, int32_t* smLast) {
+  constexpr int BM = T::BM;
+  const int tid = thread_id<T>();
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint16_t* hb = reinterpret_cast<uint16_t*>(g.share + kShareTiles) + (int64_t)tile * kShareRows * 128;
+  if (wave < T::CW) {
+    const int row_base = wave / T::WN * T::RS * 16, col_base = part * T::W + wave % T::WN * T::CS * 16;
+    const int fr = lane & 15, kseg = lane >> 4;
+#pragma unroll
+    for (int r = 0; r < T::RS; ++r)
+#pragma unroll
+      for (int c = 0; c < T::CS; ++c) {
+        float h[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const uint32_t gu = pack_bf16x2(acc[r][0][c][v], acc[r][1][c][v]);
+          h[v] = silu_mul_bf16(lo_bf16(gu), hi_bf16(gu));
+        }
+        const uint64_t four = (uint64_t)pack_bf16x2(h[2], h[3]) << 32 | pack_bf16x2(h[0], h[1]);
+        __hip_atomic_store(
+            reinterpret_cast<uint64_t*>(hb + (row_base + r * 16 + fr) * 128 + col_base + c * 16 + 4 * kseg), four,
+            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+  }
+  wait_vmcnt<0>();
+  __syncthreads();  // every wave's stores are complete
+  if (tid == 0)
+    *smLast = __hip_atomic_fetch_add(g.share + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == T::PARTS - 1;
+  __syncthreads();
+  if (!*smLast) return;
+  if (tid == 0) __hip_atomic_store(g.share + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  static_assert(BM * 8 <= T::THREADS, "eight threads a row, sixteen columns a thread");
+  const int row = tid >> 3, cc = tid & 7;
+  if (row >= rows_avail || row >= BM) return;  // whole groups of eight lanes
+  float h[16];
+  float amax = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const uint64_t four = __hip_atomic_load(reinterpret_cast<const uint64_t*>(hb + row * 128 + cc * 16 + q * 4),
+                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t lo = (uint32_t)four, hi = (uint32_t)(four >> 32);
+    h[4 * q] = lo_bf16(lo);
+    h[4 * q + 1] = hi_bf16(lo);
+    h[4 * q + 2] = lo_bf16(hi);
+    h[4 * q + 3] = hi_bf16(hi);
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(h[i]));
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+  const float sc = group_scale(amax);
+  const float inv = 1.0f / sc;
+  v4i codes;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) codes[i] = (int)quant4_e4m3(h[4 * i], h[4 * i + 1], h[4 * i + 2], h[4 * i + 3], sc, inv);
+  *reinterpret_cast<v4i*>(g.hq + (pos0 + row) * g.I + j * 128 + cc * 16) = codes;
+  if (cc == 0) *hs_at(g, pos0 + row, j) = sc;
+}
+
 // Waits until the loads of the oldest of a wave's stages in flight are
 // complete; `younger` stages were issued after it, at most MAX of them still in
 // flight by the ring's depth.
@@ -468,7 +546,7 @@ MOE_DEVICE void wait_stage(int younger) {
 // computes its first BM rows; the caller has checked that the rest are padding.
 template <class T, bool FUSED, bool EXACT = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t pos0, int rows_avail, int e,
-                                          int nvalid, bool b_nt) {
+                                          int nvalid, bool b_nt, int part = 0, int tile = 0) {
   constexpr int BM = T::BM, GROUPS = T::GROUPS;
   static_assert(GROUPS == 2 || !FUSED, "the fused epilogue takes a gate and an up group");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -546,8 +624,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
   groups_of<FUSED, GROUPS>(g, j, g0, g1, g1_store);
   const uint8_t* b_expert = g.B + (int64_t)e * g.b_es;
   const float* bs_expert = g.Bs + (int64_t)e * g.bs_es;
-  const uint8_t* bg0 = b_expert + g0 * 128 * g.ldb;  // the tile's two weight groups
-  const uint8_t* bg1 = b_expert + g1 * 128 * g.ldb;
+  const uint8_t* bg0 = b_expert + (g0 * 128 + part * T::W) * g.ldb;  // the tile's two weight groups
+  const uint8_t* bg1 = b_expert + (g1 * 128 + part * T::W) * g.ldb;
 
   // With the two-stage ring every step waits for all of its loads (vmcnt 0), so
   // the per-wave load count may vary: A rows of 16-row subtiles without a valid
@@ -711,7 +789,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
             (
                 [&] {
                   constexpr int gq = Q / T::CS, cq = Q % T::CS;
-                  const v8i fb = frag_at<(gq * 128 + cq * 16) * 128>(pb0, pb1);
+                  const v8i fb = frag_at<(gq * T::W + cq * 16) * 128>(pb0, pb1);
                   v8bf bbf[4];
 #pragma unroll
                   for (int q = 0; q < 4; ++q) bbf[q] = fp8_quarter_bf16(fb, q);
@@ -745,13 +823,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
           v4f p[LG + 1];
           scale_products();
           bq[0] = frag_at<0>(pb0, pb1);
-          if constexpr (NQ > 1) bq[1] = frag_at<(1 / T::CS * 128 + 1 % T::CS * 16) * 128>(pb0, pb1);
+          if constexpr (NQ > 1) bq[1] = frag_at<(1 / T::CS * T::W + 1 % T::CS * 16) * 128>(pb0, pb1);
           [&]<int... Q>(std::integer_sequence<int, Q...>) {
             (
                 [&] {
                   if constexpr (Q + NBQ - 1 < NQ) {
                     constexpr int gn = (Q + NBQ - 1) / T::CS, cn = (Q + NBQ - 1) % T::CS;
-                    bq[(Q + NBQ - 1) % NBQ] = frag_at<(gn * 128 + cn * 16) * 128>(pb0, pb1);
+                    bq[(Q + NBQ - 1) % NBQ] = frag_at<(gn * T::W + cn * 16) * 128>(pb0, pb1);
                   }
 #pragma unroll
                   for (int r = 0; r < RA; ++r) {
@@ -811,7 +889,10 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t j, int64_t 
   // Every wave is done with the operand ring (the last step waited for all of
   // its loads); the epilogue stages the output at its base.
   block_barrier();
-  tile_epilogue<T, FUSED>(g, acc, j, pos0, rows_avail, g0, g1, g1_store, smem, smRed, smSlot, smW);
+  if constexpr (T::W < 128)
+    share_quant<T>(g, acc, j, pos0, rows_avail, part, tile, reinterpret_cast<int32_t*>(smRed));
+  else
+    tile_epilogue<T, FUSED>(g, acc, j, pos0, rows_avail, g0, g1, g1_store, smem, smRed, smSlot, smW);
 }
 
 // The fused outputs of the tile's rows [from, to), padding past the body's rows:
@@ -1199,7 +1280,8 @@ void w13_exact_kernel(GemmArgs g) {
 template <class T, bool FUSED, bool EXACT>
 __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
   const int tid = thread_id<T>();
-  const int64_t b = blockIdx.x / (uint32_t)g.n_tiles, j = blockIdx.x % (uint32_t)g.n_tiles;
+  const uint32_t tile = blockIdx.x / T::PARTS, part = blockIdx.x % T::PARTS;
+  const int64_t b = tile / (uint32_t)g.n_tiles, j = tile % (uint32_t)g.n_tiles;
   const int64_t n_blocks = *g.ntpp / T::BM;
   // within max_padded for every b of the grid (the entries past ntpp are not used)
   const int64_t blk = g.blk ? (b < n_blocks ? g.blk[b] : 0) : b;
@@ -1212,34 +1294,36 @@ __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
   const int nvalid = __syncthreads_count(row_valid);
   if (b >= n_blocks) return;
   if (e < 0 || e >= g.E) {
-    zero_tile<T, FUSED>(g, j, pos0, T::BM);
+    if (part == 0) zero_tile<T, FUSED>(g, j, pos0, T::BM);
     return;
   }
   const bool single = before != e && !(b + 1 < n_blocks && after == e);  // the expert's only row tile
-  gemm_tile<T, FUSED, EXACT>(g, j, pos0, T::BM, e, nvalid, single);
+  gemm_tile<T, FUSED, EXACT>(g, j, pos0, T::BM, e, nvalid, single, (int)part, (int)tile);
 }
 
-template <int BM, int GROUPS, bool FUSED, bool EXACT>
-__global__ __launch_bounds__((Tile<BM, GROUPS, true>::THREADS))
+template <int BM, int GROUPS, bool FUSED, bool EXACT, int W>
+__global__ __launch_bounds__((Tile<BM, GROUPS, true, false, W>::THREADS))
 __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flat_gemm_kernel(GemmArgs g) {
-  flat_gemm_body<Tile<BM, GROUPS, true>, FUSED, EXACT>(g);
+  flat_gemm_body<Tile<BM, GROUPS, true, false, W>, FUSED, EXACT>(g);
 }
 
 constexpr int64_t kCus = 256;
+constexpr int64_t kShareK = 1024;
+static_assert(kCus / 2 <= kShareTiles, "a counter for each shared tile");
 
-template <int BM, int GROUPS, bool FUSED, bool EXACT>
+template <int BM, int GROUPS, bool FUSED, bool EXACT, int W = 128>
 static int launch_flat(const GemmArgs& args, hipStream_t st) {
-  using T = Tile<BM, GROUPS, true>;
-  const void* fn = (const void*)flat_gemm_kernel<BM, GROUPS, FUSED, EXACT>;
+  using T = Tile<BM, GROUPS, true, false, W>;
+  const void* fn = (const void*)flat_gemm_kernel<BM, GROUPS, FUSED, EXACT, W>;
   static const hipError_t attr_rc =
       hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
   if (attr_rc != hipSuccess) return kErrLaunch;
   GemmArgs a = args;
   if (GROUPS == 1) a.n_tiles = a.N / 128;
-  const int64_t grid = a.max_blocks * a.n_tiles;
+  const int64_t grid = a.max_blocks * a.n_tiles * T::PARTS;
   if (grid <= 0) return kOk;
-  hipLaunchKernelGGL((flat_gemm_kernel<BM, GROUPS, FUSED, EXACT>), dim3((unsigned)grid), dim3(T::THREADS),
+  hipLaunchKernelGGL((flat_gemm_kernel<BM, GROUPS, FUSED, EXACT, W>), dim3((unsigned)grid), dim3(T::THREADS),
                      T::LDS_BYTES, st, a);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
@@ -1268,6 +1352,16 @@ static int launch_gemm(const GemmArgs& args, hipStream_t st) {
     if (args.bma == BM && args.tile_order == 0 && args.vshift == 0) {
       if constexpr (!FUSED) {
         if (args.max_blocks * (args.N / 128) <= kCus) return launch_flat<BM, 1, FUSED, EXACT>(args, st);
+      }
+      // Fewer tiles than half or a quarter of the CUs: each is shared by two or
+      // four of them (see share_quant), which costs about 2 us and saves two
+      // thirds of a K step's time.
+      if constexpr (FUSED && !EXACT && BM >= 32) {
+        if (args.share && args.K >= kShareK) {
+          const int64_t tiles = args.max_blocks * args.n_tiles;
+          if (tiles <= kCus / 4) return launch_flat<BM, 2, FUSED, EXACT, 32>(args, st);
+          if (tiles <= kCus / 2) return launch_flat<BM, 2, FUSED, EXACT, 64>(args, st);
+        }
       }
       if (args.max_blocks * args.n_tiles <= kCus) return launch_flat<BM, 2, FUSED, EXACT>(args, st);
     }
@@ -1335,6 +1429,7 @@ static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int64_t E) {
 static void set_blocks(GemmArgs& g, const LocalBlocks& local, int TM, int vshift) {
   g.blk = local.blocks;
   g.runs = local.runs;
+  g.share = local.share;
   if (local.E_routed > 0) {
     const int64_t most = blocks_bound(g.S, local.E_routed, g.bma) << vshift;
     if (most < g.max_blocks) g.max_blocks = most;

@@ -7,7 +7,8 @@ namespace moe {
 
 // What the layer knows of its blocks beyond the align outputs.  blocks: the list
 // of local blocks that align writes under an expert map (moe_layer's
-// local_blocks), null without one.  runs: the table of runs, or null.
+// local_blocks), null without one.  runs: the table of runs, or null.  share:
+// moe_layer's share buffer, or null.
 // E_routed: the experts the slots are spread over, for the choice of the tile
 // height and a bound on the blocks (0: E, and what fits in max_padded, which
 // with few slots allows for more).  A map may send several of them to one
@@ -15,6 +16,7 @@ namespace moe {
 struct LocalBlocks {
   const int32_t* blocks = nullptr;
   const int32_t* runs = nullptr;
+  int32_t* share = nullptr;
   int64_t E_routed = 0;
 };
 
@@ -30,6 +32,12 @@ inline int64_t blocks_bound(int64_t S, int64_t E, int64_t BM) {
   const int64_t m = S < E ? S : E;
   return m + (S - m) / BM;
 }
+
+// moe_layer's share: a counter for each of kShareTiles tiles that several
+// workgroups compute together, zero between launches, then kShareRows rows of
+// 128 bf16 for each.
+constexpr int kShareTiles = 128;
+constexpr int kShareRows = 64;
 
 // local_blocks holds [0] local blocks * BM, then the blocks, then their local
 // expert ids, then a word per token whose bit i says that slot i's expert is local.
@@ -53,12 +61,12 @@ int w13_gemm(const void* Aq, const float* A_scale, const void* W13, const float*
              void* stream, LocalBlocks local = {});
 
 // T == 0: align alone.  local: the lists to write under an expert map, or null;
-// runs: the table of runs to write (S <= kRunsMaxSlots), or null; top_k: the
-// slots of a token (for its mask).
+// runs: the table of runs to write (S <= kRunsMaxSlots), or null; share: the
+// counters to clear, or null; top_k: the slots of a token (for its mask).
 int quant_align(const void* x, int64_t T, int64_t H, void* q, int64_t ldq, float* scales, const int32_t* topk_ids,
                 int64_t S, int32_t E, int32_t BM, const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids,
-                int32_t* ntpp, int64_t max_padded, void* workspace, int32_t* local, int32_t* runs, int32_t top_k,
-                void* stream);
+                int32_t* ntpp, int64_t max_padded, void* workspace, int32_t* local, int32_t* runs, int32_t* share,
+                int32_t top_k, void* stream);
 
 // The top-k sum of rows of H columns in D (row stride ldd) into y (row stride
 // H); addend rows (row stride lda) or null; with mask (a word per token) the

@@ -20,6 +20,7 @@ static LocalBlocks local_of(const moe_layer* l) {
   r.E_routed = l->E_routed;
   if (l->expert_map) r.blocks = local_blk(l->local_blocks);
   if (l->T * l->top_k <= kRunsMaxSlots) r.runs = l->runs;
+  r.share = l->share;
   return r;
 }
 
@@ -28,6 +29,8 @@ extern "C" int64_t moe_layer_local_blocks_bytes(int64_t T, int64_t max_padded, i
   return 4 * (1 + 2 * ((max_padded + BM - 1) / BM) + T);
 }
 
+extern "C" int64_t moe_layer_share_bytes(void) { return (4 + 2 * 128 * kShareRows) * (int64_t)kShareTiles; }
+
 extern "C" int64_t moe_layer_runs_bytes(int32_t E_routed) { return E_routed < 0 ? -1 : 16 * ((int64_t)E_routed + 1); }
 
 extern "C" int moe_layer_quant_align(const moe_layer* l, const void* hidden, const int32_t* topk_ids, void* stream) {
@@ -35,7 +38,7 @@ extern "C" int moe_layer_quant_align(const moe_layer* l, const void* hidden, con
   return quant_align(hidden, hidden ? l->T : 0, l->H, l->q1, l->Hp, l->s1, topk_ids, l->T * l->top_k, l->E_routed,
                      l->block_size_m, l->expert_map, l->sorted_ids, l->expert_ids, l->ntpp, l->max_padded,
                      l->workspace, l->local_blocks,
-                     l->T * l->top_k <= kRunsMaxSlots ? l->runs : nullptr, l->top_k, stream);
+                     l->T * l->top_k <= kRunsMaxSlots ? l->runs : nullptr, l->share, l->top_k, stream);
 }
 
 extern "C" int moe_layer_scales(const moe_layer* l, void* stream) {

@@ -759,6 +759,18 @@ def _layer_block_m(block_size_m: int | None, num_tokens: int, n_experts: int, to
     return bm
 
 
+# Above this many slots no launch has few enough tiles to share them.
+_SHARE_MAX_SLOTS = 8192
+
+
+def _share_buffer(slots: int, device: torch.device) -> torch.Tensor | None:
+    if slots > _SHARE_MAX_SLOTS:
+        return None
+    buf = torch.empty(int(lib().moe_layer_share_bytes()) // 4, dtype=torch.int32, device=device)
+    buf[:128] = 0  # the counters
+    return buf
+
+
 class FusedExpertsRunner:
     """Prebuilt A1->A9 chain for fixed (T, H, I, E, top_k, BM).
 
@@ -852,6 +864,9 @@ class FusedExpertsRunner:
             n = int(lib().moe_layer_local_blocks_bytes(self.T, self.align.max_padded, self.BM))
             self.local_blocks = torch.empty(n // 4, dtype=torch.int32, device=dev)
         self.runs = torch.empty(int(lib().moe_layer_runs_bytes(n_align)) // 4, dtype=torch.int32, device=dev)
+        # tiles that several workgroups share: small decode, the layer's and the shared expert's
+        self.share = _share_buffer(self.S, dev)
+        self._shared_share = _share_buffer(self.T, dev) if shared is not None else None
         if out is not None:
             _need(out, "out", torch.bfloat16)
             if tuple(out.shape) != (self.T, H):
@@ -867,7 +882,8 @@ class FusedExpertsRunner:
             w13_scale=_ptr(w13_scale), w2=_ptr(w2), w2_scale=_ptr(w2_scale), expert_map=_ptr(self.expert_map),
             q1=_ptr(self.q1), s1=_ptr(self.s1), s1_pos=_ptr(self.s1_pos) if self.scales_by_position else None,
             sorted_ids=_ptr(a.sorted_ids), expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp),
-            workspace=_ptr(a.workspace), local_blocks=_ptr(self.local_blocks), runs=_ptr(self.runs), hq=_ptr(self.hq),
+            workspace=_ptr(a.workspace), local_blocks=_ptr(self.local_blocks), runs=_ptr(self.runs),
+            share=_ptr(self.share), hq=_ptr(self.hq),
             hs=_ptr(self.hs_pos if self.scales_by_position else self.hs), D=_ptr(self.D))
         # the shared expert as a layer of one expert on this layer's FP8 input
         self._shared_layer = self._shared_view = None
@@ -878,7 +894,7 @@ class FusedExpertsRunner:
                 block_size_m=shared.BM, tile_m=0, exact_dot=0, w13=_ptr(shared.w1), w13_scale=_ptr(shared.w1_scale),
                 w2=_ptr(shared.w2), w2_scale=_ptr(shared.w2_scale), q1=_ptr(self.q1), s1=_ptr(self.s1),
                 sorted_ids=_ptr(s.sorted_ids), expert_ids=_ptr(s.expert_ids), ntpp=_ptr(s.ntpp),
-                workspace=_ptr(s.workspace), hq=_ptr(shared.hq), hs=_ptr(shared.hs), D=_ptr(shared.out))
+                workspace=_ptr(s.workspace), share=_ptr(self._shared_share), hq=_ptr(shared.hq), hs=_ptr(shared.hs), D=_ptr(shared.out))
             self._shared_view = shared.out[: self.T, :H]
 
     def _need_hidden(self, hidden: torch.Tensor) -> None:
@@ -1165,7 +1181,8 @@ def fused_experts(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tenso
     sizes = {"q1": T * H, "s1": 4 * T * G, "s1_pos": 4 * G * mp if by_pos else 0, "sorted_ids": 4 * mp,
              "expert_ids": 4 * -(-mp // bm), "ntpp": 4, "workspace": int(L.moe_align_workspace_bytes(S, n_align)),
              "local_blocks": 0 if expert_map is None else int(L.moe_layer_local_blocks_bytes(T, mp, bm)),
-             "runs": int(L.moe_layer_runs_bytes(n_align)), "hq": mp * I, "hs": 4 * mp * (I // 128), "D": 2 * S * H}
+             "runs": int(L.moe_layer_runs_bytes(n_align)),
+             "share": int(L.moe_layer_share_bytes()) if 0 < S <= _SHARE_MAX_SLOTS else 0, "hq": mp * I, "hs": 4 * mp * (I // 128), "D": 2 * S * H}
     block = torch.empty(sum((n + 255 & ~255) + 256 for n in sizes.values()), dtype=torch.uint8, device=w1.device)
     y = torch.empty((T, H), dtype=torch.bfloat16, device=w1.device)
     layer = MoeLayer(T=T, H=H, Hp=H, I=I, max_padded=mp, top_k=k, E=E, E_routed=n_align, block_size_m=bm, tile_m=0,
@@ -1173,7 +1190,7 @@ def fused_experts(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tenso
                      w2_scale=w2_scale.data_ptr(), expert_map=None if expert_map is None else expert_map.data_ptr())
     at = block.data_ptr()
     for name, n in sizes.items():
-        if n or name not in ("s1_pos", "local_blocks"):  # those two are absent, not empty
+        if n or name not in ("s1_pos", "local_blocks", "share"):  # those are absent, not empty
             setattr(layer, name, at)
         at += (n + 255 & ~255) + 256
     check(L.moe_layer_run(layer, None, hidden_states.data_ptr(), topk_weights.data_ptr(), topk_ids.data_ptr(), H,

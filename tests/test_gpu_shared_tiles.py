@@ -1,0 +1,58 @@
+"""GPU: W13 tiles that two or four workgroups share (small decode with a long K)
+give the unshared launch's codes, scales and output bit for bit, run after run
+on the same counters, with a shared expert, under an expert map and from
+fused_experts."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from moe_cases import bf16_bits, make_case, to_gpu, u8_bits
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+# (T, H, I, E, k, BM): tiles = min(S, E) and more blocks by I/128; four workgroups a tile up to 64, two up to 128
+CASES = [(1, 1024, 384, 16, 8, 32), (1, 2048, 2048, 8, 4, 32), (5, 1024, 1024, 4, 2, 32), (16, 1152, 256, 8, 4, 64),
+         (40, 1024, 640, 4, 2, 32), (33, 1024, 1024, 16, 1, 64), (3, 1024, 1408, 16, 3, 16)]
+
+
+@pytest.mark.parametrize("T,H,I,E,k,BM", CASES)
+def test_shared_tiles_equal_whole_ones(T, H, I, E, k, BM):
+    from td_benchmark_amd import ops
+    print(f"case: shared tiles T={T} H={H} I={I} E={E} k={k} BM={BM}", flush=True)
+    c = make_case(T, H, I, E, k, BM, seed=T + I)
+    g = to_gpu(c)
+    w = [g[n] for n in ("w13", "w13_s", "w2", "w2_s")]
+    r = ops.FusedExpertsRunner(*w, T, k, BM, shared=ops.SharedExpertRunner(*[t[:1].contiguous() for t in w], T, BM))
+
+    def outputs():
+        r.hq.view(torch.uint8).fill_(0x55)
+        r.hs.fill_(-1.0)
+        y = r.run(g["x"], g["topk_w"], g["topk_ids"])
+        torch.cuda.synchronize()
+        n = int(r.align.ntpp.item())
+        return u8_bits(r.hq)[:n], r.hs.cpu().numpy()[:n].view(np.uint32), bf16_bits(y)
+
+    layers = (r._layer, r._shared_layer)
+    got = [outputs() for _ in range(3)]
+    kept = [m.share for m in layers]
+    for m in layers:
+        m.share = None
+    want = outputs()
+    for m, s in zip(layers, kept):
+        m.share = s
+    for o in got + [outputs()]:
+        for a, b in zip(o, want):
+            assert np.array_equal(a, b)
+    assert int(r.share[:128].abs().sum()) == 0 and int(r._shared_share[:128].abs().sum()) == 0
+    local = [t[: E // 2].contiguous() for t in w]
+    em = torch.tensor([e if e < E // 2 else -1 for e in range(E)], dtype=torch.int32, device="cuda")
+    ep = ops.FusedExpertsRunner(*local, T, k, BM, global_num_experts=E, expert_map=em)
+    y = ep.run(g["x"], g["topk_w"], g["topk_ids"]).clone()
+    ep._layer.share = None
+    assert torch.equal(y, ep.run(g["x"], g["topk_w"], g["topk_ids"]))
+    one = ops.FusedExpertsRunner(*w, T, k, BM)
+    one._layer.share = None
+    y = ops.fused_experts(g["x"], w[0], w[2], g["topk_w"], g["topk_ids"], w1_scale=w[1], w2_scale=w[3], block_size_m=BM)
+    assert torch.equal(y, one.run(g["x"], g["topk_w"], g["topk_ids"]))
