@@ -225,9 +225,14 @@ struct AlignArgs {
 // Bit i: the expert of token t's slot i is local.
 MOE_DEVICE int32_t local_slots(const int32_t* ids, const int32_t* expert_map, int E, int top_k, int t) {
   uint32_t m = 0;
-  for (int i = 0; i < top_k && i < 32; ++i) {
-    const int x = ids[(int64_t)t * top_k + i];
-    if ((unsigned)x < (unsigned)E && expert_map[x] >= 0) m |= 1u << i;
+  for (int i0 = 0; i0 < top_k && i0 < 32; i0 += 8) {  // eight at a time: two round trips, not sixteen
+    int x[8], here[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = i0 + i < top_k ? ids[(int64_t)t * top_k + i0 + i] : -1;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) here[i] = (unsigned)x[i] < (unsigned)E ? expert_map[x[i]] : -1;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) m |= here[i] >= 0 ? 1u << (i0 + i) : 0u;
   }
   return (int32_t)m;
 }

@@ -187,6 +187,8 @@ struct GemmArgs {
   int64_t max_blocks;      // (virtual) blocks that fit in max_padded
   int64_t max_padded;      // entries of sorted
   int64_t run_tiles;       // with runs: a bound on the row tiles
+  int64_t share_tiles;     // with runs: the row tiles a launch is sized for
+  int unit_tiles;          // with runs: a third of an XCD's expected tiles
   int64_t n_tiles;         // 256-column n-tiles
   int bma;                 // rows per align block (block_size_m); a tile spans BM / bma of them
   // Exact-dot launches only: the tile map counts virtual blocks of bma >> vshift
@@ -196,7 +198,6 @@ struct GemmArgs {
   int top_k;
   int a_by_pos;
   int E;
-  int E_routed;            // with runs: the table's capacity
   int tile_order;          // 0 expert-major (XCD-contiguous), 1 shuffled, 2 half-phase
   // Strides of the (possibly sliced) operands; base pointers are pre-offset.
   int64_t lda;             // A row stride, bytes
@@ -1128,8 +1129,10 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
 // rows, so that every XCD gets its share of each size and starts the long ones
 // first; the unit's tiles stay on one XCD and next to each other, as above.
 // When the XCD's last round of tiles would fill at most half of its CUs, those
-// tiles are split into two of half the rows.  One lane looks at one unit, and
-// the row counts come from the table: one round trip to memory.
+// tiles are split into two of half the rows.  A unit has up to four n-tiles, and
+// fewer where the longest run's would be over a third of an XCD's share (16
+// experts, Zipf, 5103 tokens: a run of 8 row tiles, 105 us a layer with four,
+// 89 in expert order).  One lane looks at one unit.
 //
 // Layer times in expert order and so (us, one box): GroupGEMM shape, 1024
 // tokens, Zipf 237 / 212, uniform 230 / 218; Mixtral, 4096 tokens (W2: 2.3
@@ -1147,9 +1150,14 @@ __device__ __forceinline__ int planned_run(const GemmArgs& g, int l) {
   const int x = blockIdx.x % kXcds;
   const int lane = thread_id<T>() & 63;
   const int n_tiles = (int)g.n_tiles;
-  const int groups = (n_tiles + kTileGroup - 1) / kTileGroup;  // of n-tiles, as even as possible:
+  const int n_runs = __builtin_amdgcn_readfirstlane(g.runs[0]);
+  if (n_runs <= 0) return 0;
+  const int longest = (__builtin_amdgcn_readfirstlane(g.runs[5]) + BM - 1) / BM;  // row tiles of the first run
+  int group = g.unit_tiles / longest;
+  group = group < 1 ? 1 : (group > kTileGroup ? kTileGroup : group);
+  const int groups = (n_tiles + group - 1) / group;  // of n-tiles, as even as possible:
   const int per_group = (n_tiles + groups - 1) / groups;
-  const int n_units = __builtin_amdgcn_readfirstlane(g.runs[0]) * groups;
+  const int n_units = n_runs * groups;
   const v4i* runs = reinterpret_cast<const v4i*>(g.runs + 4);
   v4i r;
   int w, n, incl;  // this lane's unit, its tiles, and those up to it
@@ -1157,8 +1165,8 @@ __device__ __forceinline__ int planned_run(const GemmArgs& g, int l) {
     w = kXcds * k + ((k & 1) ? kXcds - 1 - x : x);
     r = (v4i){0, 0, 0, 0};
     n = 0;
-    if (w < g.E_routed * groups) r = runs[w / groups];  // beside the load of the count: one round trip
     if (w < n_units) {
+      r = runs[w / groups];
       const int left = n_tiles - w % groups * per_group;
       n = (r[1] + BM - 1) / BM * (left < per_group ? (left < 0 ? 0 : left) : per_group);
     }
@@ -1335,11 +1343,8 @@ static int launch_planned(const GemmArgs& args, hipStream_t st) {
   static const hipError_t attr_rc =
       hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kernel_lds<BM>());
   if (attr_rc != hipSuccess) return kErrLaunch;
-  // An even share of the expected tiles -- under an expert map twice the local
-  // experts' share of the slots -- and the halves of a split last round.
-  const int64_t here = 2 * args.E < args.E_routed ? 2 * args.E : args.E_routed;
-  const int64_t row_tiles = blocks_bound((args.S * here + args.E_routed - 1) / args.E_routed, here, BM);
-  const int64_t share = (row_tiles * args.n_tiles + kXcds - 1) / kXcds + kXcdCus / 2;
+  // an even share of the expected tiles, and the halves of a split last round
+  const int64_t share = (args.share_tiles * args.n_tiles + kXcds - 1) / kXcds + kXcdCus / 2;
   hipLaunchKernelGGL((planned_gemm_kernel<BM, FUSED, EXACT>), dim3((unsigned)(kXcds * share)), dim3(T::THREADS),
                      kernel_lds<BM>(), st, args);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
@@ -1434,7 +1439,11 @@ static void set_blocks(GemmArgs& g, const LocalBlocks& local, int TM, int vshift
     const int64_t most = blocks_bound(g.S, local.E_routed, g.bma) << vshift;
     if (most < g.max_blocks) g.max_blocks = most;
     g.run_tiles = blocks_bound(g.S, local.E_routed, TM);
-    g.E_routed = (int)local.E_routed;
+    // Under an expert map up to twice the local experts' share of the slots is expected.
+    const int64_t here = 2 * (int64_t)g.E < local.E_routed ? 2 * (int64_t)g.E : local.E_routed;
+    const int64_t slots = (g.S * here + local.E_routed - 1) / local.E_routed;
+    g.share_tiles = blocks_bound(slots, here, TM);
+    g.unit_tiles = (int)((slots / TM + here / 2) * g.n_tiles / (3 * kXcds));
   }
 }
 

@@ -45,6 +45,7 @@ CASES = [
     (640, 256, 1152, 4, 2, 256, 0, "zipf", True),          # 128-row exact tiles, padding past the last tile
     (515, 256, 640, 2, 2, 128, 256, "one_expert", False),  # every token in both runs
     (257, 256, 256, 3, 1, 256, 256, "softmax", True),
+    (2600, 256, 640, 5, 1, 128, 256, "zipf", False),       # a run of many row tiles: units of one n-tile
 ]
 
 
