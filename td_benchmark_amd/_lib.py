@@ -38,7 +38,8 @@ class MoeLayer(ctypes.Structure):
     _fields_ = ([(n, _i64) for n in ("T", "H", "Hp", "I", "max_padded")]
                 + [(n, _i32) for n in ("top_k", "E", "E_routed", "block_size_m", "tile_m", "exact_dot")]
                 + [(n, _P) for n in ("w13", "w13_scale", "w2", "w2_scale", "expert_map", "q1", "s1", "s1_pos",
-                                     "sorted_ids", "expert_ids", "ntpp", "workspace", "local_blocks", "runs", "share", "hq", "hs", "D")])
+                                     "sorted_ids", "expert_ids", "ntpp", "workspace", "local_blocks", "runs",
+                                     "share", "hq", "hs", "D")])
 
 
 _LAYER = ctypes.POINTER(MoeLayer)

@@ -23,8 +23,9 @@
 // split evenly over the expert's tiles, so a weight tile is fetched once per
 // up to 256 rows.  8 waves (2 per SIMD, so one wave's MFMAs run while the other
 // waits on LDS or the barrier) for TM >= 32, 4 for TM = 16; at TM = 256 they
-// are 4 x 2 waves of 64 x 128.  TM = 32 runs two workgroups per CU.  The K step is 128 = one scale block, and every
-// K step is exactly one 16x16x128 MFMA per 16x16 output subtile started from
+// are 4 x 2 waves of 64 x 128.  TM = 32 runs two workgroups per CU.  (Launches
+// whose tiles all run at once take other forms, see Launch.)  The K step is
+// 128 = one scale block, and every K step is exactly one 16x16x128 MFMA per 16x16 output subtile started from
 // zero, so the per-block scales are applied as acc = fma(partial,
 // a_s[row]*b_s[group], acc) (kScaleLag MFMAs later) with no second
 // accumulator.  The fp32 promotion at every 128-K block also bounds the matrix
@@ -71,11 +72,16 @@
 // the contraction does not depend on how the hardware orders K inside the
 // instruction.
 //
-// Launch: workgroup ids are dealt round-robin to the 8 XCDs; the id -> tile map
-// gives each XCD a contiguous range of an expert-major tile order, so all row
-// tiles of one expert that read the same weight tile run together on one
-// XCD (weights leave HBM once) and a row tile's A rows are shared by its
-// n-tiles in that XCD's L2.
+// Launch: workgroup ids are dealt round-robin to the 8 XCDs.  The same tiles are
+// dealt out in one of three ways, by how many there are:
+//   many (grouped_gemm_body): the id -> tile map gives each XCD a contiguous
+//     range of an expert-major tile order, so all row tiles of one expert that
+//     read the same weight tile run together on one XCD (weights leave HBM once)
+//     and a row tile's A rows are shared by its n-tiles in that XCD's L2;
+//   a few a CU (planned_run): units of a run's row tiles, dealt out by size;
+//   at most one a CU (flat_gemm_body): no map, a deep ring, loading waves, and
+//     for the fewest tiles several workgroups a tile (share_quant).
+// Every form computes each output with the same operations in the same order.
 #include <type_traits>
 
 #include "common.hpp"
@@ -463,7 +469,11 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs& g, v4f (&acc)[T::R
 // agent-scope atomics (written to and read from beyond the XCDs' L2s); each wave
 // waits for its stores before the workgroup counts itself in.  A release and an
 // acquire fence around plain accesses write back and invalidate an L2 each time:
-// with 192 workgroups they took about 10 us.
+// with 192 workgroups they took about 10 us.  A CU loads 50-60 GB/s of weights
+// that are in no cache, whatever the ring, so a tile's time is its bytes over the
+// CUs that stream it: W13 of Qwen3 at one token (48 tiles, K 2048) 15.3 us with
+// one workgroup a tile, 11.3 with four; of DeepSeek-V3's shared expert at 16
+// tokens (16 tiles, K 7168) 42.8 and 18.0.
 template <class T>
 __device__ __forceinline__ void share_quant(const GemmArgs& g, v4f (&acc)[T::RS][T::GROUPS][T::CS], int64_t j,
                                             int64_t pos0, int rows_avail, int part, int tile, int32_t* smLast) {
@@ -1134,7 +1144,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
 // experts, Zipf, 5103 tokens: a run of 8 row tiles, 105 us a layer with four,
 // 89 in expert order).  One lane looks at one unit.
 //
-// Layer times in expert order and so (us, one box): GroupGEMM shape, 1024
+// Layer times in expert order and so (us): GroupGEMM shape, 1024
 // tokens, Zipf 237 / 212, uniform 230 / 218; Mixtral, 4096 tokens (W2: 2.3
 // tiles a CU, three rounds) 1660 / 1553, 1000 tokens, Zipf (128-row blocks in
 // 256-row tiles: half of a run's ids idle, on other XCDs than its tiles) 813 /
@@ -1284,7 +1294,11 @@ void w13_exact_kernel(GemmArgs g) {
 //     64 B a cycle) plus the time to compute;
 //   - a plain launch takes 128 weight rows a tile, twice the workgroups.
 // There is one row tile per block, and row tiles that share weights run at the
-// same time whatever their order.
+// same time whatever their order.  Kernel times with the map, ring and tile of
+// the many-tile launches, and so (us): Mixtral, 7 tokens, W2 (K 14336, 8 blocks
+// by 16 tiles of 256: half the CUs) 146 / 73; Qwen3, one token, W13 21.8 / 15.3
+// (11.3 shared, below), W2 11.4 / 6.8.  Over one tile a CU the second tile of a CU
+// waits for the whole first: there the launches below are faster.
 template <class T, bool FUSED, bool EXACT>
 __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
   const int tid = thread_id<T>();
@@ -1360,7 +1374,11 @@ static int launch_gemm(const GemmArgs& args, hipStream_t st) {
       }
       // Fewer tiles than half or a quarter of the CUs: each is shared by two or
       // four of them (see share_quant), which costs about 2 us and saves two
-      // thirds of a K step's time.
+      // thirds of a K step's time.  Layer times whole / shared (us, 64 experts,
+      // top-8): 48 tiles, by four, K 512 20.5 / 21.1, K 1024 23.3 / 21.9, K 2048
+      // 27.8 / 24.0, K 4096 39.6 / 29.7; 128 tiles, by two, K 1024 25.1 / 26.0,
+      // K 2048 32.1 / 31.0, K 4096 51.4 / 50.5.  Over 128 tiles two parts of a
+      // tile no longer all find a CU.
       if constexpr (FUSED && !EXACT && BM >= 32) {
         if (args.share && args.K >= kShareK) {
           const int64_t tiles = args.max_blocks * args.n_tiles;
