@@ -856,17 +856,10 @@ class FusedExpertsRunner:
         else:
             self.hs = torch.empty((mp, self.I // 128), dtype=torch.float32, device=dev)
         self.D = torch.empty((max(self.S, 1), Hp), dtype=torch.bfloat16, device=dev)
-        self.local_blocks = None
-        if self.expert_map is not None:
-            # written at the positions of local experts only: elsewhere what a run of zero rows leaves
-            self.hq.view(torch.uint8).zero_()
-            (self.hs_pos if self.scales_by_position else self.hs).fill_(1e-12)
-            n = int(lib().moe_layer_local_blocks_bytes(self.T, self.align.max_padded, self.BM))
-            self.local_blocks = torch.empty(n // 4, dtype=torch.int32, device=dev)
+        self.local_blocks = self._local_list() if self.expert_map is not None else None
         self.runs = torch.empty(int(lib().moe_layer_runs_bytes(n_align)) // 4, dtype=torch.int32, device=dev)
-        # tiles that several workgroups share: small decode, the layer's and the shared expert's
+        # tiles that several workgroups share: small decode
         self.share = _share_buffer(self.S, dev)
-        self._shared_share = _share_buffer(self.T, dev) if shared is not None else None
         if out is not None:
             _need(out, "out", torch.bfloat16)
             if tuple(out.shape) != (self.T, H):
@@ -875,27 +868,69 @@ class FusedExpertsRunner:
         # An H or an output the sum cannot write in place: the sum at the padded width, whose first H columns are y.
         in_place = Hp == H or (H % 8 == 0 and self.y.data_ptr() % 16 == 0)
         self.y_pad = self.y if in_place else torch.empty((self.T, Hp), dtype=torch.bfloat16, device=dev)
+        self._bind()
+
+    def _local_list(self) -> torch.Tensor:
+        """Room for the list of the local experts' blocks.  Under an expert map
+        hq and hs are written at their positions only: elsewhere they hold what
+        a run of zero rows leaves."""
+        self.hq.view(torch.uint8).zero_()
+        (self.hs_pos if self.scales_by_position else self.hs).fill_(1e-12)
+        n = int(lib().moe_layer_local_blocks_bytes(self.T, self.align.max_padded, self.BM))
+        return torch.empty(n // 4, dtype=torch.int32, device=self.hq.device)
+
+    def _bind(self) -> None:
+        """The native layer over the runner's own buffers; what a program may set is filled in at each run."""
         a = self.align
         self._layer = MoeLayer(
-            T=self.T, H=H, Hp=Hp, I=self.I, max_padded=a.max_padded, top_k=top_k, E=E, E_routed=n_align,
-            block_size_m=self.BM, tile_m=self.tile_m, exact_dot=int(self.exact_dot), w13=_ptr(w13),
-            w13_scale=_ptr(w13_scale), w2=_ptr(w2), w2_scale=_ptr(w2_scale), expert_map=_ptr(self.expert_map),
-            q1=_ptr(self.q1), s1=_ptr(self.s1), s1_pos=_ptr(self.s1_pos) if self.scales_by_position else None,
-            sorted_ids=_ptr(a.sorted_ids), expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp),
-            workspace=_ptr(a.workspace), local_blocks=_ptr(self.local_blocks), runs=_ptr(self.runs),
-            share=_ptr(self.share), hq=_ptr(self.hq),
+            T=self.T, H=self.H, Hp=self.Hp, I=self.I, max_padded=a.max_padded, top_k=self.top_k, E=self.E,
+            E_routed=a.E, block_size_m=self.BM, q1=_ptr(self.q1), s1=_ptr(self.s1),
+            s1_pos=_ptr(self.s1_pos) if self.scales_by_position else None, sorted_ids=_ptr(a.sorted_ids),
+            expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp), workspace=_ptr(a.workspace),
+            local_blocks=_ptr(self.local_blocks), runs=_ptr(self.runs), share=_ptr(self.share), hq=_ptr(self.hq),
             hs=_ptr(self.hs_pos if self.scales_by_position else self.hs), D=_ptr(self.D))
-        # the shared expert as a layer of one expert on this layer's FP8 input
-        self._shared_layer = self._shared_view = None
-        if shared is not None:
-            s = shared._align_for(num_tokens)
-            self._shared_layer = MoeLayer(
-                T=self.T, H=H, Hp=Hp, I=shared.I, max_padded=s.max_padded, top_k=1, E=1, E_routed=1,
-                block_size_m=shared.BM, tile_m=0, exact_dot=0, w13=_ptr(shared.w1), w13_scale=_ptr(shared.w1_scale),
-                w2=_ptr(shared.w2), w2_scale=_ptr(shared.w2_scale), q1=_ptr(self.q1), s1=_ptr(self.s1),
-                sorted_ids=_ptr(s.sorted_ids), expert_ids=_ptr(s.expert_ids), ntpp=_ptr(s.ntpp),
-                workspace=_ptr(s.workspace), share=_ptr(self._shared_share), hq=_ptr(shared.hq), hs=_ptr(shared.hs), D=_ptr(shared.out))
-            self._shared_view = shared.out[: self.T, :H]
+        self._shared_layer = self._shared_of = None
+        self._fill()
+
+    def _fill(self) -> tuple[MoeLayer, MoeLayer | None]:
+        """The native layers with what a program may have set since the last
+        run: the mode, the weights, the expert map, the shared expert."""
+        layer, shared, s = self._layer, None, self.shared
+        layer.exact_dot, layer.tile_m = int(self.exact_dot), self.tile_m
+        layer.w13, layer.w13_scale = self.w13.data_ptr(), self.w13_scale.data_ptr()
+        layer.w2, layer.w2_scale = self.w2.data_ptr(), self.w2_scale.data_ptr()
+        layer.expert_map = None if self.expert_map is None else self.expert_map.data_ptr()
+        if layer.expert_map and not layer.local_blocks:  # the first map of a runner built without one
+            self.local_blocks = self._local_list()
+            layer.local_blocks = self.local_blocks.data_ptr()
+        if s is not None:
+            if s is not self._shared_of:
+                self._bind_shared(s)
+            shared = self._shared_layer
+            shared.exact_dot = layer.exact_dot
+            shared.w13, shared.w13_scale = s.w1.data_ptr(), s.w1_scale.data_ptr()
+            shared.w2, shared.w2_scale = s.w2.data_ptr(), s.w2_scale.data_ptr()
+        return layer, shared
+
+    def _bind_shared(self, s: SharedExpertRunner) -> None:
+        """The shared expert as a layer of one expert on this layer's FP8 input."""
+        a = s._align_for(self.T)
+        self._shared_share = _share_buffer(self.T, self.q1.device)
+        self._shared_layer = MoeLayer(
+            T=self.T, H=self.H, Hp=self.Hp, I=s.I, max_padded=a.max_padded, top_k=1, E=1, E_routed=1,
+            block_size_m=s.BM, q1=_ptr(self.q1), s1=_ptr(self.s1), sorted_ids=_ptr(a.sorted_ids),
+            expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp), workspace=_ptr(a.workspace),
+            share=_ptr(self._shared_share), hq=_ptr(s.hq), hs=_ptr(s.hs), D=_ptr(s.out))
+        self._shared_view = s.out[: self.T, : self.H]
+        self._shared_of = s
+
+    def __getstate__(self) -> dict:
+        """The runner's state without its addresses (a copy has its own buffers)."""
+        return {k: v for k, v in self.__dict__.items() if k not in ("_layer", "_shared_layer", "_shared_of")}
+
+    def __setstate__(self, state: dict) -> None:
+        self.__dict__.update(state)
+        self._bind()
 
     def _need_hidden(self, hidden: torch.Tensor) -> None:
         _need(hidden, "hidden_states", torch.bfloat16)
@@ -922,8 +957,7 @@ class FusedExpertsRunner:
             check(lib().moe_layer_scales(self._layer, _stream()), "moe_layer_scales")
 
     def stage_w13(self) -> None:
-        self._layer.exact_dot = int(self.exact_dot)
-        check(lib().moe_layer_w13(self._layer, _stream()), "moe_layer_w13")
+        check(lib().moe_layer_w13(self._fill()[0], _stream()), "moe_layer_w13")
 
     def _need_weights_of_slots(self, topk_weights: torch.Tensor) -> None:
         _need(topk_weights, "topk_weights", torch.float32)
@@ -932,7 +966,7 @@ class FusedExpertsRunner:
 
     def stage_w2(self, topk_weights: torch.Tensor) -> None:
         self._need_weights_of_slots(topk_weights)
-        check(lib().moe_layer_w2(self._layer, _ptr(topk_weights), _stream()), "moe_layer_w2")
+        check(lib().moe_layer_w2(self._fill()[0], _ptr(topk_weights), _stream()), "moe_layer_w2")
 
     def stage_shared(self) -> None:
         """The shared expert on the layer's own FP8 input (no second quant),
@@ -954,11 +988,9 @@ class FusedExpertsRunner:
         self._need_hidden(hidden)
         self.align.need_ids(topk_ids, self.expert_map)
         self._need_weights_of_slots(topk_weights)
-        layer, shared = self._layer, self._shared_layer
-        layer.exact_dot = int(self.exact_dot)
+        layer, shared = self._fill()
         if shared is not None:
             self.shared.exact_dot = self.exact_dot
-            shared.exact_dot = layer.exact_dot
             self.shared_out = self._shared_view
         check(lib().moe_layer_run(layer, shared, hidden.data_ptr(), topk_weights.data_ptr(), topk_ids.data_ptr(),
                                   self.y_pad.shape[1], self.y_pad.data_ptr(), _stream_handle()), "moe_layer_run")

@@ -60,3 +60,52 @@ def test_one_call_equals_the_stages():
         r.stage_reduce()
         torch.cuda.synchronize()
         assert np.array_equal(bf16_bits(y), bf16_bits(r.y)) and np.array_equal(bf16_bits(out), bf16_bits(r.shared_out))
+
+
+def test_runner_follows_its_attributes_and_copies():
+    """Weights, expert map and shared expert set on a runner after it is built
+    are the ones a run takes, and a copy of a runner runs on its own buffers."""
+    import copy
+    import io
+
+    from td_benchmark_amd import ops
+    print("case: weights, map and shared expert set between runs; copies", flush=True)
+    T, E, k = 40, 8, 2
+    g, g2 = (to_gpu(make_case(T, 256, 256, E, k, 32, seed=s)) for s in (5, 6))
+    names = ("w13", "w13_s", "w2", "w2_s")
+    args = g["x"], g["topk_w"], g["topk_ids"]
+
+    def fresh(gg, shared=None, em=None):
+        w = [gg[n] for n in names]
+        r = ops.FusedExpertsRunner(*w, T, k, 32, expert_map=em, global_num_experts=E if em is not None else None,
+                                   shared=ops.SharedExpertRunner(*[t[shared:shared + 1].contiguous() for t in w], T)
+                                   if shared is not None else None)
+        return r, bf16_bits(r.run(*args).clone())
+
+    r, first = fresh(g, shared=1)
+    r.w13, r.w13_scale, r.w2, r.w2_scale = (g2[n].clone() for n in names)
+    r.shared = fresh(g2, shared=2)[0].shared
+    want = fresh(g2, shared=2)[1]
+    assert np.array_equal(bf16_bits(r.run(*args)), want) and not np.array_equal(first, want)
+    r.shared = None
+    assert np.array_equal(bf16_bits(r.run(*args)), fresh(g2)[1])
+
+    maps = [torch.tensor([e if e % 2 == odd else -1 for e in range(E)], dtype=torch.int32, device="cuda")
+            for odd in (0, 1)]
+    r, _ = fresh(g, em=maps[0])
+    r.expert_map = maps[1]
+    want = fresh(g, em=maps[1])[1]
+    assert np.array_equal(bf16_bits(r.run(*args)), want)
+    r, whole = fresh(g)
+    for em, y in ((maps[1], want), (None, whole)):
+        r.expert_map = em
+        assert np.array_equal(bf16_bits(r.run(*args)), y)
+
+    r, want = fresh(g, shared=1)
+    file = io.BytesIO()
+    torch.save(r, file)
+    file.seek(0)
+    for c in (copy.deepcopy(r), torch.load(file, weights_only=False)):
+        r.y.zero_()
+        assert c.q1.data_ptr() != r.q1.data_ptr() and c._layer.q1 == c.q1.data_ptr()
+        assert np.array_equal(bf16_bits(c.run(*args)), want) and not bf16_bits(r.y).any()
