@@ -325,6 +325,7 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
     for (int i = tid; i < padded >> sh; i += kAlignThreads) {
       local_blk(a.local)[(lbefore >> sh) + i] = (before >> sh) + i;
       local_eid(a.local, a.max_padded, a.BM)[(lbefore >> sh) + i] = local;
+      local_rid(a.local, a.max_padded, a.BM)[(lbefore >> sh) + i] = e;
     }
   }
   // the tokens' local slots, and the positions and blocks past ntpp, shared out over the workgroups
@@ -353,10 +354,12 @@ __global__ __launch_bounds__(kAlignThreads) void align_expert_kernel(AlignArgs a
 }
 
 // The same lists after the three launches: the first workgroup compacts the
-// blocks whose (local) expert id is not -1, 1024 at a time, the others mark the
-// tokens' local slots.
+// blocks whose (local) expert id is not -1, 1024 at a time (a block's first
+// position always holds a slot, whose id is the expert before the map), the
+// others mark the tokens' local slots.
 __global__ __launch_bounds__(1024) void local_blocks_kernel(const int32_t* __restrict__ ids, int64_t S, int E,
                                                             int top_k, const int32_t* __restrict__ expert_map,
+                                                            const int32_t* __restrict__ sorted,
                                                             const int32_t* __restrict__ eids,
                                                             const int32_t* __restrict__ ntpp, int BM,
                                                             int64_t max_padded, int32_t* __restrict__ local) {
@@ -385,6 +388,7 @@ __global__ __launch_bounds__(1024) void local_blocks_kernel(const int32_t* __res
     if (e >= 0) {
       local_blk(local)[at + __popcll(m & lt)] = b;
       local_eid(local, max_padded, BM)[at + __popcll(m & lt)] = e;
+      local_rid(local, max_padded, BM)[at + __popcll(m & lt)] = ids[sorted[(int64_t)b * BM]];
     }
     __syncthreads();
   }
@@ -495,7 +499,7 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
   }
   if (local)
     hipLaunchKernelGGL(local_blocks_kernel, dim3((unsigned)(1 + (S / top_k + 1023) / 1024)), dim3(1024), 0, st,
-                       topk_ids, S, (int)E, (int)top_k, expert_map, expert_ids, ntpp, (int)BM, max_padded, local);
+                       topk_ids, S, (int)E, (int)top_k, expert_map, sorted_ids, expert_ids, ntpp, (int)BM, max_padded, local);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 

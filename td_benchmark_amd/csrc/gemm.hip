@@ -180,6 +180,9 @@ struct GemmArgs {
   // ascending order; eids and ntpp then describe this list, and the other
   // blocks are no part of the launch.
   const int32_t* blk;
+  // What tells runs of blocks apart: eids, or with blk the experts before the
+  // map (two of them may share a local one, see local_blocks).
+  const int32_t* rid;
   const int32_t* runs;     // the experts' runs by descending rows (see internal.hpp), or null
   int32_t* share;          // fused: counters and rows of tiles that several workgroups share, or null
   const float* topk_w;     // [S] or null
@@ -1057,29 +1060,29 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   }
   if (t >= total) return;
   const int64_t bq = t / g.n_tiles;  // a block of the tile's run
-  // The run of blocks with bq's expert: the expert ids of bq and of the 64
+  // The run of blocks with bq's expert: the run ids of bq and of the 64
   // blocks on either side are loaded together (one memory round trip for runs
   // of up to 65 blocks), longer runs continue 64 blocks at a time.
   int64_t back = 0, fwd = 0;
-  int e;
+  const int e = g.eids[bq >> vsh];
   {
     const int ln = thread_id<T>() & 63;
     const int64_t ib = bq - 1 - ln, jf = bq + 1 + ln;
-    e = g.eids[bq >> vsh];
-    const int xb = ib >= 0 ? g.eids[ib >> vsh] : 0;
-    const int xf = jf < n_blocks ? g.eids[jf >> vsh] : 0;
-    uint64_t end = __ballot(!(ib >= 0 && xb == e));  // blocks before bq with the same expert
+    const int id = g.rid[bq >> vsh];
+    const int xb = ib >= 0 ? g.rid[ib >> vsh] : 0;
+    const int xf = jf < n_blocks ? g.rid[jf >> vsh] : 0;
+    uint64_t end = __ballot(!(ib >= 0 && xb == id));  // blocks before bq with the same expert
     for (int64_t base = bq - 1 - 64; !end; base -= 64) {
       back += 64;
       const int64_t idx = base - ln;
-      end = __ballot(!(idx >= 0 && g.eids[idx >> vsh] == e));
+      end = __ballot(!(idx >= 0 && g.rid[idx >> vsh] == id));
     }
     back += __ffsll((unsigned long long)end) - 1;
-    end = __ballot(!(jf < n_blocks && xf == e));      // and after it
+    end = __ballot(!(jf < n_blocks && xf == id));      // and after it
     for (int64_t base = bq + 1 + 64; !end; base += 64) {
       fwd += 64;
       const int64_t idx = base + ln;
-      end = __ballot(!(idx < n_blocks && g.eids[idx >> vsh] == e));
+      end = __ballot(!(idx < n_blocks && g.rid[idx >> vsh] == id));
     }
     fwd += __ffsll((unsigned long long)end) - 1;
   }
@@ -1113,7 +1116,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   const int64_t u = by_col ? in_grp % units : in_grp / gsz;  // row tile of the run
   const int64_t base = run / units, n_short = units - run % units;  // n_short tiles of `base` blocks
   const int64_t b = b0 + (u < n_short ? u * base : n_short * base + (u - n_short) * (base + 1));
-  // sorted position of tile row 0 (a run's blocks are consecutive in the listed order too)
+  // sorted position of tile row 0 (the blocks of one run id are consecutive in the sorted order too)
   const int64_t pos0 = (g.blk ? ((int64_t)g.blk[b >> vsh] << vsh) + (b & ((1 << vsh) - 1)) : b) * vb;
   // tile rows that belong to this run (the rest are not read or written)
   const int rows_avail = (int)((u < n_short ? base : base + 1) * vb);
@@ -1451,6 +1454,7 @@ static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int64_t E) {
 // What the layer knows of its blocks.
 static void set_blocks(GemmArgs& g, const LocalBlocks& local, int TM, int vshift) {
   g.blk = local.blocks;
+  if (local.rids) g.rid = local.rids;
   g.runs = local.runs;
   g.share = local.share;
   if (local.E_routed > 0) {
@@ -1502,7 +1506,7 @@ int moe::plain_gemm(const void* A, const float* A_scale, const void* B, const fl
   g.B = (const uint8_t*)B;
   g.Bs = B_scale;
   g.sorted = sorted_ids;
-  g.eids = expert_ids;
+  g.eids = g.rid = expert_ids;
   g.ntpp = ntpp;
   g.topk_w = topk_weights;
   g.C = (uint16_t*)C;
@@ -1589,7 +1593,7 @@ static int setup_plain(GemmArgs& g, int& TM, const void* A, const float* A_scale
   g.B = (const uint8_t*)B;
   g.Bs = B_scale;
   g.sorted = sorted_ids;
-  g.eids = expert_ids;
+  g.eids = g.rid = expert_ids;
   g.ntpp = ntpp;
   g.topk_w = topk_weights;
   g.C = (uint16_t*)C;
@@ -1707,7 +1711,7 @@ int moe::w13_gemm(const void* Aq, const float* A_scale, const void* W13, const f
   g.B = (const uint8_t*)W13;
   g.Bs = W13_scale;
   g.sorted = sorted_ids;
-  g.eids = expert_ids;
+  g.eids = g.rid = expert_ids;
   g.ntpp = ntpp;
   g.topk_w = nullptr;
   g.hq = (uint8_t*)hq;

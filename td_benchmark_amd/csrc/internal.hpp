@@ -15,6 +15,7 @@ namespace moe {
 // local expert, so the local ones bound nothing.
 struct LocalBlocks {
   const int32_t* blocks = nullptr;
+  const int32_t* rids = nullptr;  // with blocks: what tells the listed blocks' runs apart
   const int32_t* runs = nullptr;
   int32_t* share = nullptr;
   int64_t E_routed = 0;
@@ -40,7 +41,10 @@ constexpr int kShareTiles = 128;
 constexpr int kShareRows = 64;
 
 // local_blocks holds [0] local blocks * BM, then the blocks, then their local
-// expert ids, then a word per token whose bit i says that slot i's expert is local.
+// expert ids, then the experts that the ids select (a map may send several of
+// them to one local expert: listed one after another they are two runs, with
+// other blocks or padding between their slots), then a word per token whose bit
+// i says that slot i's expert is local.
 inline const int32_t* local_rows(const int32_t* l) { return l; }
 template <class T>
 MOE_HOST_DEVICE T* local_blk(T* l) { return l + 1; }
@@ -48,7 +52,9 @@ template <class T>
 MOE_HOST_DEVICE T* local_eid(T* l, int64_t max_padded, int32_t BM) { return l + 1 + (max_padded + BM - 1) / BM; }
 
 template <class T>
-MOE_HOST_DEVICE T* local_mask(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 2 * ((max_padded + BM - 1) / BM); }
+MOE_HOST_DEVICE T* local_rid(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 2 * ((max_padded + BM - 1) / BM); }
+template <class T>
+MOE_HOST_DEVICE T* local_mask(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 3 * ((max_padded + BM - 1) / BM); }
 
 int plain_gemm(const void* A, const float* A_scale, const void* B, const float* B_scale, const int32_t* sorted_ids,
                const int32_t* expert_ids, const int32_t* ntpp, const float* topk_weights, int64_t S, int32_t top_k,

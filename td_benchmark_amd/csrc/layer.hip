@@ -18,7 +18,10 @@ using namespace moe;
 static LocalBlocks local_of(const moe_layer* l) {
   LocalBlocks r;
   r.E_routed = l->E_routed;
-  if (l->expert_map) r.blocks = local_blk(l->local_blocks);
+  if (l->expert_map) {
+    r.blocks = local_blk(l->local_blocks);
+    r.rids = local_rid(l->local_blocks, l->max_padded, l->block_size_m);
+  }
   if (l->T * l->top_k <= kRunsMaxSlots) r.runs = l->runs;
   r.share = l->share;
   return r;
@@ -26,7 +29,7 @@ static LocalBlocks local_of(const moe_layer* l) {
 
 extern "C" int64_t moe_layer_local_blocks_bytes(int64_t T, int64_t max_padded, int32_t BM) {
   if (T < 0 || max_padded < 0 || !block_m_ok(BM)) return -1;
-  return 4 * (1 + 2 * ((max_padded + BM - 1) / BM) + T);
+  return 4 * (1 + 3 * ((max_padded + BM - 1) / BM) + T);
 }
 
 extern "C" int64_t moe_layer_share_bytes(void) { return (4 + 2 * 128 * kShareRows) * (int64_t)kShareTiles; }

@@ -67,3 +67,38 @@ def test_map_may_send_several_experts_to_one_local_expert():
     want = loc.run(g["x"], g["topk_w"], em[g["topk_ids"].long()].contiguous())
     torch.cuda.synchronize()
     assert np.array_equal(bf16_bits(y), bf16_bits(want))
+
+
+# (T, E, k, BM, tile_m, exact): row tiles of several align blocks, from the one-launch and the three-launch align
+REPLICATED = [(2100, 64, 8, None, 0, False), (2100, 64, 8, 64, 256, False), (2100, 64, 8, 128, 256, True),
+              (700, 24, 8, 64, 256, False), (500, 12, 4, 32, 128, False)]
+
+
+@pytest.mark.parametrize("kind", ["apart", "adjacent", "both"])
+@pytest.mark.parametrize("T,E,k,BM,tile_m,exact", REPLICATED)
+def test_replicated_experts_keep_their_own_runs(T, E, k, BM, tile_m, exact, kind):
+    """Two experts of the ids on one local expert, with experts of other
+    devices between them (apart), none between them (adjacent), or both: their
+    blocks stay two runs with the padding at each end, in the expert-ordered
+    tile map (which runs without align's table of runs) and the other one."""
+    from td_benchmark_amd import ops
+    print(f"case: replicated T={T} E={E} k={k} BM={BM} tile_m={tile_m} exact={exact} {kind}", flush=True)
+    e = np.arange(E)
+    emap = {"apart": np.where(e % 2 == 0, e // 4, -1), "adjacent": e // 2,
+            "both": np.where(e % 4 == 2, -1, e // 4)}[kind].astype(np.int32)
+    n = int(emap.max()) + 1
+    c = make_case(T, 256, 256, E, k, BM or 128, seed=T + E)
+    g = to_gpu(c)
+    w = [g[name][:n].contiguous() for name in ("w13", "w13_s", "w2", "w2_s")]
+    em = torch.from_numpy(emap).cuda()
+    ids = em[g["topk_ids"].long()].contiguous()
+    loc = ops.FusedExpertsRunner(*w, T, k, 32, tile_m=32, exact_dot=exact)
+    loc.D[(ids < 0).view(-1)] = 0
+    want = bf16_bits(loc.run(g["x"], g["topk_w"], ids))
+    ep = ops.FusedExpertsRunner(*w, T, k, BM, tile_m=tile_m, global_num_experts=E, expert_map=em, exact_dot=exact)
+    for runs in (ep._layer.runs, None):
+        ep._layer.runs = runs
+        ep.D.fill_(3.0)
+        y = ep.run(g["x"], g["topk_w"], g["topk_ids"])
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(y), want)
