@@ -914,6 +914,9 @@ class FusedExpertsRunner:
 
     def _bind_shared(self, s: SharedExpertRunner) -> None:
         """The shared expert as a layer of one expert on this layer's FP8 input."""
+        # the native layer takes the width of its weights and rows from here
+        if s.Hp != self.Hp or (self.Hp == self.H and s.H != self.H):
+            raise ValueError(f"shared expert of hidden size {s.H} does not match the layer's {self.H}")
         a = s._align_for(self.T)
         self._shared_share = _share_buffer(self.T, self.q1.device)
         self._shared_layer = MoeLayer(
@@ -921,7 +924,7 @@ class FusedExpertsRunner:
             block_size_m=s.BM, q1=_ptr(self.q1), s1=_ptr(self.s1), sorted_ids=_ptr(a.sorted_ids),
             expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp), workspace=_ptr(a.workspace),
             share=_ptr(self._shared_share), hq=_ptr(s.hq), hs=_ptr(s.hs), D=_ptr(s.out))
-        self._shared_view = s.out[: self.T, : self.H]
+        self._shared_view = s.out[: self.T, : s.H]
         self._shared_of = s
 
     def __getstate__(self) -> dict:

@@ -109,3 +109,38 @@ def test_runner_follows_its_attributes_and_copies():
         r.y.zero_()
         assert c.q1.data_ptr() != r.q1.data_ptr() and c._layer.q1 == c.q1.data_ptr()
         assert np.array_equal(bf16_bits(c.run(*args)), want) and not bf16_bits(r.y).any()
+
+
+def test_shared_expert_set_later_has_to_fit():
+    """A shared expert set on a built runner is refused where its rows are of
+    another width than the layer's, or too few, and taken where both run at
+    one padded width."""
+    from td_benchmark_amd import ops
+    print("case: shared experts of other sizes set on a runner", flush=True)
+    T, E, k = 24, 4, 2
+    names = ("w13", "w13_s", "w2", "w2_s")
+    g = {H: to_gpu(make_case(T, H, 256, E, k, 32, seed=H)) for H in (128, 200, 256, 384)}
+
+    def shared(H, rows=T):
+        return ops.SharedExpertRunner(*[g[H][n][:1].contiguous() for n in names], rows)
+
+    def layer(H):
+        return ops.FusedExpertsRunner(*[g[H][n] for n in names], T, k, 32)
+
+    def args(H):
+        return g[H]["x"], g[H]["topk_w"], g[H]["topk_ids"]
+
+    for H, bad in ((256, shared(128)), (256, shared(384)), (256, shared(200)), (200, shared(384)),
+                   (256, shared(256, T - 1))):
+        r = layer(H)
+        want = bf16_bits(r.run(*args(H)))
+        r.shared = bad
+        with pytest.raises(ValueError):
+            r.run(*args(H))
+        r.shared = None
+        assert np.array_equal(bf16_bits(r.run(*args(H))), want)
+    r = layer(200)
+    y = r.run(*args(200)).clone()
+    r.shared = shared(256)
+    got = r.run(*args(200))
+    assert np.array_equal(bf16_bits(got), bf16_bits((y.float() + r.shared_out[:, :200].float()).bfloat16()))
