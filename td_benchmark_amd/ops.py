@@ -857,6 +857,7 @@ class FusedExpertsRunner:
             self.hs = torch.empty((mp, self.I // 128), dtype=torch.float32, device=dev)
         self.D = torch.empty((max(self.S, 1), Hp), dtype=torch.bfloat16, device=dev)
         self.local_blocks = self._local_list() if self.expert_map is not None else None
+        self._aligned_map = self.expert_map  # the map of the last align, whose list the later stages run over
         self.runs = torch.empty(int(lib().moe_layer_runs_bytes(n_align)) // 4, dtype=torch.int32, device=dev)
         # tiles that several workgroups share: small decode
         self.share = _share_buffer(self.S, dev)
@@ -880,37 +881,49 @@ class FusedExpertsRunner:
         return torch.empty(n // 4, dtype=torch.int32, device=self.hq.device)
 
     def _bind(self) -> None:
-        """The native layer over the runner's own buffers; what a program may set is filled in at each run."""
+        """The native layer over the runner's own buffers; what a program may set is filled in by each stage."""
         a = self.align
         self._layer = MoeLayer(
             T=self.T, H=self.H, Hp=self.Hp, I=self.I, max_padded=a.max_padded, top_k=self.top_k, E=self.E,
-            E_routed=a.E, block_size_m=self.BM, q1=_ptr(self.q1), s1=_ptr(self.s1),
+            E_routed=a.E, block_size_m=self.BM, expert_map=_ptr(self._aligned_map), q1=_ptr(self.q1), s1=_ptr(self.s1),
             s1_pos=_ptr(self.s1_pos) if self.scales_by_position else None, sorted_ids=_ptr(a.sorted_ids),
             expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp), workspace=_ptr(a.workspace),
             local_blocks=_ptr(self.local_blocks), runs=_ptr(self.runs), share=_ptr(self.share), hq=_ptr(self.hq),
             hs=_ptr(self.hs_pos if self.scales_by_position else self.hs), D=_ptr(self.D))
         self._shared_layer = self._shared_of = None
-        self._fill()
+        if self.shared is not None:
+            self._fill_shared()
 
-    def _fill(self) -> tuple[MoeLayer, MoeLayer | None]:
-        """The native layers with what a program may have set since the last
-        run: the mode, the weights, the expert map, the shared expert."""
-        layer, shared, s = self._layer, None, self.shared
+    def _fill(self) -> MoeLayer:
+        """The native layer with the mode and weights that a program may have set since the last stage."""
+        layer = self._layer
         layer.exact_dot, layer.tile_m = int(self.exact_dot), self.tile_m
         layer.w13, layer.w13_scale = self.w13.data_ptr(), self.w13_scale.data_ptr()
         layer.w2, layer.w2_scale = self.w2.data_ptr(), self.w2_scale.data_ptr()
-        layer.expert_map = None if self.expert_map is None else self.expert_map.data_ptr()
-        if layer.expert_map and not layer.local_blocks:  # the first map of a runner built without one
+        return layer
+
+    def _fill_map(self) -> MoeLayer:
+        """The native layer for an align under the expert map that the runner
+        has now.  The stages after it run over the list that this align writes,
+        so a map set in between waits for the next align."""
+        layer, m = self._layer, self.expert_map
+        self._aligned_map = m
+        layer.expert_map = None if m is None else m.data_ptr()
+        if m is not None and not layer.local_blocks:  # the first map of a runner built without one
             self.local_blocks = self._local_list()
             layer.local_blocks = self.local_blocks.data_ptr()
-        if s is not None:
-            if s is not self._shared_of:
-                self._bind_shared(s)
-            shared = self._shared_layer
-            shared.exact_dot = layer.exact_dot
-            shared.w13, shared.w13_scale = s.w1.data_ptr(), s.w1_scale.data_ptr()
-            shared.w2, shared.w2_scale = s.w2.data_ptr(), s.w2_scale.data_ptr()
-        return layer, shared
+        return layer
+
+    def _fill_shared(self) -> MoeLayer:
+        """The shared expert's native layer with the mode and weights it has now."""
+        s = self.shared
+        if s is not self._shared_of:
+            self._bind_shared(s)
+        shared = self._shared_layer
+        shared.exact_dot = int(self.exact_dot)
+        shared.w13, shared.w13_scale = s.w1.data_ptr(), s.w1_scale.data_ptr()
+        shared.w2, shared.w2_scale = s.w2.data_ptr(), s.w2_scale.data_ptr()
+        return shared
 
     def _bind_shared(self, s: SharedExpertRunner) -> None:
         """The shared expert as a layer of one expert on this layer's FP8 input."""
@@ -951,7 +964,7 @@ class FusedExpertsRunner:
 
     def stage_align(self, topk_ids: torch.Tensor) -> None:
         self.align.need_ids(topk_ids, self.expert_map)
-        check(lib().moe_layer_quant_align(self._layer, None, _ptr(topk_ids), _stream()), "moe_layer_quant_align")
+        check(lib().moe_layer_quant_align(self._fill_map(), None, _ptr(topk_ids), _stream()), "moe_layer_quant_align")
 
     def stage_scales(self) -> None:
         """The activation scales K-major by sorted position for the W13 GEMM
@@ -960,7 +973,7 @@ class FusedExpertsRunner:
             check(lib().moe_layer_scales(self._layer, _stream()), "moe_layer_scales")
 
     def stage_w13(self) -> None:
-        check(lib().moe_layer_w13(self._fill()[0], _stream()), "moe_layer_w13")
+        check(lib().moe_layer_w13(self._fill(), _stream()), "moe_layer_w13")
 
     def _need_weights_of_slots(self, topk_weights: torch.Tensor) -> None:
         _need(topk_weights, "topk_weights", torch.float32)
@@ -969,7 +982,7 @@ class FusedExpertsRunner:
 
     def stage_w2(self, topk_weights: torch.Tensor) -> None:
         self._need_weights_of_slots(topk_weights)
-        check(lib().moe_layer_w2(self._fill()[0], _ptr(topk_weights), _stream()), "moe_layer_w2")
+        check(lib().moe_layer_w2(self._fill(), _ptr(topk_weights), _stream()), "moe_layer_w2")
 
     def stage_shared(self) -> None:
         """The shared expert on the layer's own FP8 input (no second quant),
@@ -991,8 +1004,10 @@ class FusedExpertsRunner:
         self._need_hidden(hidden)
         self.align.need_ids(topk_ids, self.expert_map)
         self._need_weights_of_slots(topk_weights)
-        layer, shared = self._fill()
-        if shared is not None:
+        layer, shared = self._fill(), None
+        self._fill_map()
+        if self.shared is not None:
+            shared = self._fill_shared()
             self.shared.exact_dot = self.exact_dot
             self.shared_out = self._shared_view
         check(lib().moe_layer_run(layer, shared, hidden.data_ptr(), topk_weights.data_ptr(), topk_ids.data_ptr(),

@@ -144,3 +144,40 @@ def test_shared_expert_set_later_has_to_fit():
     r.shared = shared(256)
     got = r.run(*args(200))
     assert np.array_equal(bf16_bits(got), bf16_bits((y.float() + r.shared_out[:, :200].float()).bfloat16()))
+
+
+@pytest.mark.parametrize("T,BM", [(40, 32), (2100, 64)])  # the one-launch and the three-launch align
+def test_stages_follow_the_map_their_align_had(T, BM):
+    """Stage by stage: an expert map set on a runner counts from the next align
+    on (the first map of a runner built without one, another map, none again),
+    and one set between the stages waits for it."""
+    from td_benchmark_amd import ops
+    print(f"case: maps set between stages, T={T} BM={BM}", flush=True)
+    E, k = 16, 8
+    g = to_gpu(make_case(T, 256, 256, E, k, BM, seed=T))
+    w = [g[n] for n in ("w13", "w13_s", "w2", "w2_s")]
+    args = g["x"], g["topk_w"], g["topk_ids"]
+    maps = [None] + [torch.tensor([e if e % 3 == m else -1 for e in range(E)], dtype=torch.int32, device="cuda")
+                     for m in (0, 1)]
+
+    def fresh(em):
+        r = ops.FusedExpertsRunner(*w, T, k, BM, expert_map=em)
+        return bf16_bits(r.run(*args).clone())
+
+    want = [fresh(em) for em in maps]
+    r = ops.FusedExpertsRunner(*w, T, k, BM)
+    for now, then in ((0, 1), (1, 2), (2, 0), (0, 0), (2, 2)):
+        r.expert_map = maps[now]
+        r.D.fill_(3.0)
+        r.stage_quant(g["x"])
+        r.stage_align(g["topk_ids"])
+        r.expert_map = maps[then]
+        r.stage_scales()
+        r.stage_w13()
+        r.stage_w2(g["topk_w"])
+        r.stage_shared()
+        r.stage_reduce()
+        torch.cuda.synchronize()
+        assert np.array_equal(bf16_bits(r.y), want[now])
+    r.expert_map = maps[1]
+    assert np.array_equal(bf16_bits(r.run(*args)), want[1])
