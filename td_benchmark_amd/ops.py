@@ -992,11 +992,13 @@ class FusedExpertsRunner:
             self.shared_out = self.shared(self.q1, self.s1)
 
     def stage_reduce(self) -> None:
-        addend, ld = None, 0
+        addend = None
         if self.shared is not None:  # the shared expert's rows at the padded width
-            addend, ld = self.shared.out, self.Hp
-        check(lib().moe_layer_reduce(self._layer, _ptr(addend), ld, self.y_pad.shape[1], _ptr(self.y_pad), _stream()),
-              "moe_layer_reduce")
+            addend = self.shared.out[: self.T] if self.Hp != self.H else self.shared_out
+        if addend is not None:
+            _need(addend, "shared expert rows", torch.bfloat16, (self.T, self.Hp))
+        check(lib().moe_layer_reduce(self._layer, _ptr(addend), self.Hp, self.y_pad.shape[1], _ptr(self.y_pad),
+                                     _stream()), "moe_layer_reduce")
         if self.y_pad is not self.y:
             self.y.copy_(self.y_pad[:, : self.H])
 

@@ -181,3 +181,30 @@ def test_stages_follow_the_map_their_align_had(T, BM):
         assert np.array_equal(bf16_bits(r.y), want[now])
     r.expert_map = maps[1]
     assert np.array_equal(bf16_bits(r.run(*args)), want[1])
+
+
+def test_reduce_takes_the_shared_rows_that_were_computed():
+    """The top-k sum adds no shared expert's rows before its stage has run, and
+    refuses rows that are not the layer's."""
+    from td_benchmark_amd import ops
+    print("case: reduce before and after the shared stage", flush=True)
+    T, E, k = 24, 4, 2
+    g = to_gpu(make_case(T, 256, 256, E, k, 32, seed=1))
+    w = [g[n] for n in ("w13", "w13_s", "w2", "w2_s")]
+    plain = bf16_bits(ops.FusedExpertsRunner(*w, T, k, 32).run(g["x"], g["topk_w"], g["topk_ids"]))
+    r = ops.FusedExpertsRunner(*w, T, k, 32, shared=ops.SharedExpertRunner(*[t[:1].contiguous() for t in w], T))
+    r.shared.out.fill_(7.0)
+    r.stage_quant(g["x"])
+    r.stage_align(g["topk_ids"])
+    r.stage_scales()
+    r.stage_w13()
+    r.stage_w2(g["topk_w"])
+    r.stage_reduce()
+    assert np.array_equal(bf16_bits(r.y), plain)
+    r.stage_shared()
+    r.stage_reduce()
+    both = bf16_bits(r.y.clone())
+    assert np.array_equal(both, bf16_bits(r.run(g["x"], g["topk_w"], g["topk_ids"]))) and not np.array_equal(both, plain)
+    r.shared_out = r.shared_out[: T - 1]
+    with pytest.raises(ValueError):
+        r.stage_reduce()
