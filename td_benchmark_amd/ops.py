@@ -813,6 +813,16 @@ class FusedExpertsRunner:
     the local experts' blocks only: ``hq``, ``hs`` and ``D`` are written for
     the slots of local experts, and the top-k sum takes the others as zero."""
 
+    # What the native layer holds the addresses and sizes of: setting one of
+    # them binds it anew.
+    _BOUND = frozenset(("T", "H", "Hp", "I", "E", "top_k", "BM", "align", "q1", "s1", "s1_pos", "scales_by_position",
+                        "hq", "hs", "hs_pos", "D", "local_blocks", "runs", "share"))
+
+    def __setattr__(self, name: str, value: Any) -> None:
+        object.__setattr__(self, name, value)
+        if name in self._BOUND:
+            self.__dict__["_layer"] = None
+
     def __init__(self, w13: torch.Tensor, w13_scale: torch.Tensor, w2: torch.Tensor,
                  w2_scale: torch.Tensor, num_tokens: int, top_k: int, block_size_m: int | None = None,
                  shared: SharedExpertRunner | None = None, out: torch.Tensor | None = None,
@@ -869,7 +879,9 @@ class FusedExpertsRunner:
         # An H or an output the sum cannot write in place: the sum at the padded width, whose first H columns are y.
         in_place = Hp == H or (H % 8 == 0 and self.y.data_ptr() % 16 == 0)
         self.y_pad = self.y if in_place else torch.empty((self.T, Hp), dtype=torch.bfloat16, device=dev)
-        self._bind()
+        self._native()
+        if shared is not None:
+            self._fill_shared()
 
     def _local_list(self) -> torch.Tensor:
         """Room for the list of the local experts' blocks.  Under an expert map
@@ -880,9 +892,12 @@ class FusedExpertsRunner:
         n = int(lib().moe_layer_local_blocks_bytes(self.T, self.align.max_padded, self.BM))
         return torch.empty(n // 4, dtype=torch.int32, device=self.hq.device)
 
-    def _bind(self) -> None:
-        """The native layer over the runner's own buffers; what a program may set is filled in by each stage."""
+    def _native(self) -> MoeLayer:
+        """The native layer over the runner's buffers; the rest of what a program may set is filled in by each stage."""
+        if self._layer is not None:
+            return self._layer
         a = self.align
+        self._shared_bound = None  # the shared expert's layer reads q1 and s1
         self._layer = MoeLayer(
             T=self.T, H=self.H, Hp=self.Hp, I=self.I, max_padded=a.max_padded, top_k=self.top_k, E=self.E,
             E_routed=a.E, block_size_m=self.BM, expert_map=_ptr(self._aligned_map), q1=_ptr(self.q1), s1=_ptr(self.s1),
@@ -890,13 +905,11 @@ class FusedExpertsRunner:
             expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp), workspace=_ptr(a.workspace),
             local_blocks=_ptr(self.local_blocks), runs=_ptr(self.runs), share=_ptr(self.share), hq=_ptr(self.hq),
             hs=_ptr(self.hs_pos if self.scales_by_position else self.hs), D=_ptr(self.D))
-        self._shared_layer = self._shared_of = None
-        if self.shared is not None:
-            self._fill_shared()
+        return self._layer
 
     def _fill(self) -> MoeLayer:
         """The native layer with the mode and weights that a program may have set since the last stage."""
-        layer = self._layer
+        layer = self._native()
         layer.exact_dot, layer.tile_m = int(self.exact_dot), self.tile_m
         layer.w13, layer.w13_scale = self.w13.data_ptr(), self.w13_scale.data_ptr()
         layer.w2, layer.w2_scale = self.w2.data_ptr(), self.w2_scale.data_ptr()
@@ -906,31 +919,31 @@ class FusedExpertsRunner:
         """The native layer for an align under the expert map that the runner
         has now.  The stages after it run over the list that this align writes,
         so a map set in between waits for the next align."""
-        layer, m = self._layer, self.expert_map
-        self._aligned_map = m
-        layer.expert_map = None if m is None else m.data_ptr()
-        if m is not None and not layer.local_blocks:  # the first map of a runner built without one
+        m = self.expert_map
+        if m is not None and self.local_blocks is None:  # the first map of a runner built without one
             self.local_blocks = self._local_list()
-            layer.local_blocks = self.local_blocks.data_ptr()
+        self._aligned_map = m
+        layer = self._native()
+        layer.expert_map = None if m is None else m.data_ptr()
         return layer
 
     def _fill_shared(self) -> MoeLayer:
-        """The shared expert's native layer with the mode and weights it has now."""
+        """The shared expert's native layer with the mode, weights and buffers it has now."""
         s = self.shared
-        if s is not self._shared_of:
-            self._bind_shared(s)
+        a, b = s._align_for(self.T), self._shared_bound
+        if b is None or b[0] is not s or b[1] is not a or b[2] is not s.hq or b[3] is not s.hs or b[4] is not s.out:
+            self._bind_shared(s, a)
         shared = self._shared_layer
         shared.exact_dot = int(self.exact_dot)
         shared.w13, shared.w13_scale = s.w1.data_ptr(), s.w1_scale.data_ptr()
         shared.w2, shared.w2_scale = s.w2.data_ptr(), s.w2_scale.data_ptr()
         return shared
 
-    def _bind_shared(self, s: SharedExpertRunner) -> None:
+    def _bind_shared(self, s: SharedExpertRunner, a: AlignBuffers) -> None:
         """The shared expert as a layer of one expert on this layer's FP8 input."""
         # the native layer takes the width of its weights and rows from here
         if s.Hp != self.Hp or (self.Hp == self.H and s.H != self.H):
             raise ValueError(f"shared expert of hidden size {s.H} does not match the layer's {self.H}")
-        a = s._align_for(self.T)
         self._shared_share = _share_buffer(self.T, self.q1.device)
         self._shared_layer = MoeLayer(
             T=self.T, H=self.H, Hp=self.Hp, I=s.I, max_padded=a.max_padded, top_k=1, E=1, E_routed=1,
@@ -938,15 +951,15 @@ class FusedExpertsRunner:
             expert_ids=_ptr(a.expert_ids), ntpp=_ptr(a.ntpp), workspace=_ptr(a.workspace),
             share=_ptr(self._shared_share), hq=_ptr(s.hq), hs=_ptr(s.hs), D=_ptr(s.out))
         self._shared_view = s.out[: self.T, : s.H]
-        self._shared_of = s
+        self._shared_bound = (s, a, s.hq, s.hs, s.out)
 
     def __getstate__(self) -> dict:
         """The runner's state without its addresses (a copy has its own buffers)."""
-        return {k: v for k, v in self.__dict__.items() if k not in ("_layer", "_shared_layer", "_shared_of")}
+        return {k: v for k, v in self.__dict__.items() if k not in ("_layer", "_shared_layer", "_shared_bound")}
 
     def __setstate__(self, state: dict) -> None:
-        self.__dict__.update(state)
-        self._bind()
+        self.__dict__.update(state, _layer=None)
+        self._native()
 
     def _need_hidden(self, hidden: torch.Tensor) -> None:
         _need(hidden, "hidden_states", torch.bfloat16)
@@ -970,7 +983,7 @@ class FusedExpertsRunner:
         """The activation scales K-major by sorted position for the W13 GEMM
         (nothing to do on the row-major path)."""
         if self.scales_by_position:
-            check(lib().moe_layer_scales(self._layer, _stream()), "moe_layer_scales")
+            check(lib().moe_layer_scales(self._native(), _stream()), "moe_layer_scales")
 
     def stage_w13(self) -> None:
         check(lib().moe_layer_w13(self._fill(), _stream()), "moe_layer_w13")
@@ -997,7 +1010,7 @@ class FusedExpertsRunner:
             addend = self.shared.out[: self.T] if self.Hp != self.H else self.shared_out
         if addend is not None:
             _need(addend, "shared expert rows", torch.bfloat16, (self.T, self.Hp))
-        check(lib().moe_layer_reduce(self._layer, _ptr(addend), self.Hp, self.y_pad.shape[1], _ptr(self.y_pad),
+        check(lib().moe_layer_reduce(self._native(), _ptr(addend), self.Hp, self.y_pad.shape[1], _ptr(self.y_pad),
                                      _stream()), "moe_layer_reduce")
         if self.y_pad is not self.y:
             self.y.copy_(self.y_pad[:, : self.H])
@@ -1006,8 +1019,8 @@ class FusedExpertsRunner:
         self._need_hidden(hidden)
         self.align.need_ids(topk_ids, self.expert_map)
         self._need_weights_of_slots(topk_weights)
-        layer, shared = self._fill(), None
         self._fill_map()
+        layer, shared = self._fill(), None
         if self.shared is not None:
             shared = self._fill_shared()
             self.shared.exact_dot = self.exact_dot

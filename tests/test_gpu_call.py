@@ -208,3 +208,50 @@ def test_reduce_takes_the_shared_rows_that_were_computed():
     r.shared_out = r.shared_out[: T - 1]
     with pytest.raises(ValueError):
         r.stage_reduce()
+
+
+def test_runner_follows_its_buffers():
+    """Buffers set on a runner or its shared expert after they are built are
+    the ones that run and the stages read and write; the former ones are left
+    alone."""
+    from td_benchmark_amd import ops
+    print("case: buffers set between runs", flush=True)
+    T, E, k = 70, 8, 2
+    g = to_gpu(make_case(T, 256, 256, E, k, 32, seed=8))
+    w = [g[n] for n in ("w13", "w13_s", "w2", "w2_s")]
+    args = g["x"], g["topk_w"], g["topk_ids"]
+
+    def filled(t):
+        old = t.view(torch.uint8) if t.is_contiguous() else t.t().view(torch.uint8)
+        old.fill_(0x33)
+        return old
+
+    for by_pos in (False, True):
+        r = ops.FusedExpertsRunner(*w, T, k, 32, tile_m=128, scales_by_position=by_pos,
+                                   shared=ops.SharedExpertRunner(*[t[:1].contiguous() for t in w], T))
+        want = bf16_bits(r.run(*args).clone())
+        kept = []
+        for obj, names in ((r, ["q1", "s1", "hq", "D", "hs_pos" if by_pos else "hs"] + ["s1_pos"] * by_pos),
+                           (r.shared, ["hq", "hs", "out"])):
+            for name in names:
+                old = getattr(obj, name)
+                setattr(obj, name, torch.empty_like(old))
+                kept.append(filled(old))
+        old = r.align
+        r.align = ops.AlignBuffers(old.S, old.E, old.BM, old.sorted_ids.device)
+        kept += [filled(t) for t in (old.sorted_ids, old.expert_ids, old.ntpp)]
+        assert np.array_equal(bf16_bits(r.run(*args)), want)
+        r.D.fill_(3.0)
+        r.stage_quant(args[0])
+        r.stage_align(args[2])
+        r.D = torch.empty_like(r.D)  # between the stages
+        r.stage_scales()
+        r.stage_w13()
+        r.stage_w2(args[1])
+        r.stage_shared()
+        r.stage_reduce()
+        assert np.array_equal(bf16_bits(r.y), want)
+        assert all(bool((t == 0x33).all()) for t in kept)
+        if by_pos:
+            r.scales_by_position = False
+            assert np.array_equal(bf16_bits(r.run(*args)), want)
