@@ -324,8 +324,10 @@ typedef struct moe_layer {
   int32_t* local_blocks;      /* moe_layer_local_blocks_bytes, with expert_map; else NULL */
   int32_t* runs;              /* moe_layer_runs_bytes, 16-byte aligned: align's notes on the experts' rows for the
                                  GEMMs' tile order; NULL: without */
-  int32_t* share;             /* moe_layer_share_bytes, 16-byte aligned, the first 512 bytes zero before the first
-                                 run: lets several workgroups share a W13 tile in small decode; NULL: without */
+  int32_t* share;             /* moe_layer_share_bytes, 16-byte aligned: lets several workgroups share a W13 tile in
+                                 small decode; NULL: without.  Its first 512 bytes are zero before a W13 stage, which
+                                 leaves them so; moe_layer_quant_align clears them, and moe_layer_run the shared
+                                 layer's too. */
   void* hq;                   /* [max_padded, I] e4m3fn */
   float* hs;                  /* [I/128, max_padded] with s1_pos, else [max_padded, I/128] */
   void* D;                    /* [T * top_k, Hp] bf16 */

@@ -86,11 +86,14 @@ __global__ __launch_bounds__(kAlignChunk) void align_count_kernel(
 // kernel.
 __global__ __launch_bounds__(kAlignMaxExperts) void align_scan_kernel(
     int32_t* __restrict__ chunk_count, int64_t n_chunks, int E, int BM, int use_lds,
-    int32_t* __restrict__ off_out, int32_t* __restrict__ cnt_out, int32_t* __restrict__ ntpp_out) {
+    int32_t* __restrict__ off_out, int32_t* __restrict__ cnt_out, int32_t* __restrict__ ntpp_out, int32_t* share,
+    int32_t* share2) {
   extern __shared__ int32_t staged[];  // [n_chunks][E] when use_lds
   __shared__ int32_t wave_tot[kAlignMaxExperts / 64];
   const int tid = threadIdx.x;
   const int e = tid;
+  if (share && tid < kShareTiles) share[tid] = 0;
+  if (share2 && tid < kShareTiles) share2[tid] = 0;
   if (use_lds) {
     for (int64_t i = tid; i < n_chunks * E; i += kAlignMaxExperts) staged[i] = chunk_count[i];
     __syncthreads();
@@ -217,7 +220,8 @@ struct AlignArgs {
   int32_t* ntpp;
   int32_t* local;  // the lists of local blocks and slots, or null (see internal.hpp)
   int32_t* runs;   // the table of runs, or null (see internal.hpp)
-  int32_t* share;  // the counters of shared tiles to clear, or null
+  int32_t* share;  // the counters of shared tiles to clear, of two layers, or null
+  int32_t* share2;
   int64_t max_padded;
   int S, E, BM, top_k;
 };
@@ -341,6 +345,7 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   if (a.runs && tid == 0 && cnt > 0 && local >= 0)
     reinterpret_cast<v4i*>(a.runs + 4)[place] = (v4i){before, cnt, local, padded};
   if (a.share && e == 0 && tid < kShareTiles) a.share[tid] = 0;
+  if (a.share2 && e == 0 && tid < kShareTiles) a.share2[tid] = 0;
   if (e == 0 && tid == 0) {
     *a.ntpp = total;
     if (a.local) *a.local = ltotal;
@@ -456,13 +461,13 @@ static void by_slots(int64_t S, F&& f) {
 static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
                       int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded,
                       void* workspace, void* stream, int32_t* local = nullptr, int32_t* runs = nullptr,
-                      int32_t* share = nullptr, int32_t top_k = 1) {
+                      int32_t* share = nullptr, int32_t* share2 = nullptr, int32_t top_k = 1) {
   const int arg_rc = align_args(topk_ids, S, E, BM, sorted_ids, expert_ids, ntpp, max_padded, true, workspace);
   if (arg_rc != kOk) return arg_rc;
   if (!expert_map) local = nullptr;
   hipStream_t st = (hipStream_t)stream;
   if (S <= kAlignOneLaunchSlots) {
-    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share,
+    const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share, share2,
                       max_padded, (int)S, (int)E, (int)BM, (int)top_k};
     by_slots(S, [&](auto it) {
       hipLaunchKernelGGL(align_expert_kernel<decltype(it)::value>, dim3((unsigned)E), dim3(kAlignThreads), 0, st, a);
@@ -490,7 +495,7 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
   const int use_lds = n_chunks * E <= kAlignStageLimit ? 1 : 0;
   hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(kAlignMaxExperts),
                      use_lds ? (size_t)(n_chunks * E * sizeof(int32_t)) : 0, st, chunk_count, n_chunks,
-                     (int)E, (int)BM, use_lds, off, cnt, ntpp);
+                     (int)E, (int)BM, use_lds, off, cnt, ntpp, share, share2);
   const int64_t wide = S > max_padded ? S : max_padded;
   if (wide > 0) {
     hipLaunchKernelGGL(align_place_kernel, dim3((unsigned)((wide + 255) / 256)), dim3(256), 0, st,
@@ -506,7 +511,7 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
 int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq, float* scales,
                      const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM, const int32_t* expert_map,
                      int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp, int64_t max_padded, void* workspace,
-                     int32_t* local, int32_t* runs, int32_t* share, int32_t top_k, void* stream) {
+                     int32_t* local, int32_t* runs, int32_t* share, int32_t* share2, int32_t top_k, void* stream) {
   // both halves' arguments before either is launched
   if (top_k <= 0) return kErrBadTopK;
   if (T < 0 || H < 0 || ldq < (H + 127) / 128 * 128) return kErrBadShape;
@@ -522,10 +527,10 @@ int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int6
     const int qrc = moe_quant_group128_padded(x_bf16, T, H, q_fp8, ldq, scales, stream);
     if (qrc != kOk) return qrc;
     return align_impl(topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp, max_padded, workspace, stream,
-                      local, runs, share, top_k);
+                      local, runs, share, share2, top_k);
   }
   if (!expert_map) local = nullptr;
-  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share,
+  const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share, share2,
                       max_padded, (int)S, (int)E, (int)BM, (int)top_k};
   const unsigned grid = (unsigned)(E + (q.n_chunks + kAlignThreads - 1) / kAlignThreads);
   by_slots(S, [&](auto it) {
@@ -543,7 +548,7 @@ extern "C" int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q
                                const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp,
                                int64_t max_padded, void* workspace, void* stream) {
   return quant_align(x_bf16, T, H, q_fp8, ldq, scales, topk_ids, S, E, BM, expert_map, sorted_ids, expert_ids, ntpp,
-                     max_padded, workspace, nullptr, nullptr, nullptr, 1, stream);
+                     max_padded, workspace, nullptr, nullptr, nullptr, nullptr, 1, stream);
 }
 
 extern "C" int moe_align_block_size(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,

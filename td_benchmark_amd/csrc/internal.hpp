@@ -35,8 +35,9 @@ inline int64_t blocks_bound(int64_t S, int64_t E, int64_t BM) {
 }
 
 // moe_layer's share: a counter for each of kShareTiles tiles that several
-// workgroups compute together, zero between launches, then kShareRows rows of
-// 128 bf16 for each.
+// workgroups compute together, zero between launches (align clears them, which
+// runs on the layer's stream before the GEMMs), then kShareRows rows of 128 bf16
+// for each.
 constexpr int kShareTiles = 128;
 constexpr int kShareRows = 64;
 
@@ -67,12 +68,13 @@ int w13_gemm(const void* Aq, const float* A_scale, const void* W13, const float*
              void* stream, LocalBlocks local = {});
 
 // T == 0: align alone.  local: the lists to write under an expert map, or null;
-// runs: the table of runs to write (S <= kRunsMaxSlots), or null; share: the
-// counters to clear, or null; top_k: the slots of a token (for its mask).
+// runs: the table of runs to write (S <= kRunsMaxSlots), or null; share, share2:
+// the counters to clear (the layer's and its shared expert's), or null; top_k:
+// the slots of a token (for its mask).
 int quant_align(const void* x, int64_t T, int64_t H, void* q, int64_t ldq, float* scales, const int32_t* topk_ids,
                 int64_t S, int32_t E, int32_t BM, const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids,
                 int32_t* ntpp, int64_t max_padded, void* workspace, int32_t* local, int32_t* runs, int32_t* share,
-                int32_t top_k, void* stream);
+                int32_t* share2, int32_t top_k, void* stream);
 
 // The top-k sum of rows of H columns in D (row stride ldd) into y (row stride
 // H); addend rows (row stride lda) or null; with mask (a word per token) the

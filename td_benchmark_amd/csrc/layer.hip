@@ -36,12 +36,18 @@ extern "C" int64_t moe_layer_share_bytes(void) { return (4 + 2 * 128 * kShareRow
 
 extern "C" int64_t moe_layer_runs_bytes(int32_t E_routed) { return E_routed < 0 ? -1 : 16 * ((int64_t)E_routed + 1); }
 
-extern "C" int moe_layer_quant_align(const moe_layer* l, const void* hidden, const int32_t* topk_ids, void* stream) {
+static int layer_quant_align(const moe_layer* l, const moe_layer* shared, const void* hidden, const int32_t* topk_ids,
+                             void* stream) {
   if (!l || (l->expert_map && !l->local_blocks)) return kErrNullPointer;
   return quant_align(hidden, hidden ? l->T : 0, l->H, l->q1, l->Hp, l->s1, topk_ids, l->T * l->top_k, l->E_routed,
                      l->block_size_m, l->expert_map, l->sorted_ids, l->expert_ids, l->ntpp, l->max_padded,
                      l->workspace, l->local_blocks,
-                     l->T * l->top_k <= kRunsMaxSlots ? l->runs : nullptr, l->share, l->top_k, stream);
+                     l->T * l->top_k <= kRunsMaxSlots ? l->runs : nullptr, l->share,
+                     shared ? shared->share : nullptr, l->top_k, stream);
+}
+
+extern "C" int moe_layer_quant_align(const moe_layer* l, const void* hidden, const int32_t* topk_ids, void* stream) {
+  return layer_quant_align(l, nullptr, hidden, topk_ids, stream);
 }
 
 extern "C" int moe_layer_scales(const moe_layer* l, void* stream) {
@@ -82,7 +88,7 @@ extern "C" int moe_layer_run(const moe_layer* l, const moe_layer* shared, const 
   if (!l) return kErrNullPointer;
   if (shared && (shared->T != l->T || shared->Hp != l->Hp || shared->top_k != 1)) return kErrBadShape;
   if (l->T > 0 && !hidden) return kErrNullPointer;
-  int rc = moe_layer_quant_align(l, hidden, topk_ids, stream);
+  int rc = layer_quant_align(l, shared, hidden, topk_ids, stream);
   if (rc == kOk) rc = moe_layer_scales(l, stream);
   if (rc == kOk) rc = moe_layer_w13(l, stream);
   if (rc == kOk) rc = moe_layer_w2(l, topk_weights, stream);

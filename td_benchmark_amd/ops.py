@@ -766,9 +766,7 @@ _SHARE_MAX_SLOTS = 8192
 def _share_buffer(slots: int, device: torch.device) -> torch.Tensor | None:
     if slots > _SHARE_MAX_SLOTS:
         return None
-    buf = torch.empty(int(lib().moe_layer_share_bytes()) // 4, dtype=torch.int32, device=device)
-    buf[:128] = 0  # the counters
-    return buf
+    return torch.empty(int(lib().moe_layer_share_bytes()) // 4, dtype=torch.int32, device=device)
 
 
 class FusedExpertsRunner:
@@ -811,7 +809,8 @@ class FusedExpertsRunner:
 
     With ``expert_map`` (global -> local expert id or -1) the GEMMs run over
     the local experts' blocks only: ``hq``, ``hs`` and ``D`` are written for
-    the slots of local experts, and the top-k sum takes the others as zero."""
+    the slots of local experts and hold anything elsewhere, and the top-k sum
+    takes the other slots as zero."""
 
     # What the native layer holds the addresses and sizes of: setting one of
     # them binds it anew.
@@ -884,11 +883,7 @@ class FusedExpertsRunner:
             self._fill_shared()
 
     def _local_list(self) -> torch.Tensor:
-        """Room for the list of the local experts' blocks.  Under an expert map
-        hq and hs are written at their positions only: elsewhere they hold what
-        a run of zero rows leaves."""
-        self.hq.view(torch.uint8).zero_()
-        (self.hs_pos if self.scales_by_position else self.hs).fill_(1e-12)
+        """Room for the list of the local experts' blocks, which align writes."""
         n = int(lib().moe_layer_local_blocks_bytes(self.T, self.align.max_padded, self.BM))
         return torch.empty(n // 4, dtype=torch.int32, device=self.hq.device)
 
