@@ -809,8 +809,9 @@ class FusedExpertsRunner:
 
     With ``expert_map`` (global -> local expert id or -1) the GEMMs run over
     the local experts' blocks only: ``hq``, ``hs`` and ``D`` are written for
-    the slots of local experts and hold anything elsewhere, and the top-k sum
-    takes the other slots as zero."""
+    the slots of local experts and left as they are elsewhere (hq and hs start
+    as zero rows, D as anything), and the top-k sum takes the other slots as
+    zero."""
 
     # What the native layer holds the addresses and sizes of: setting one of
     # them binds it anew.
@@ -883,7 +884,12 @@ class FusedExpertsRunner:
             self._fill_shared()
 
     def _local_list(self) -> torch.Tensor:
-        """Room for the list of the local experts' blocks, which align writes."""
+        """Room for the list of the local experts' blocks, which align writes.
+        hq and hs, which the runs write at those blocks' positions only, start
+        as what zero rows quantise to (a run leaves the other positions as it
+        finds them, also where an earlier run had local blocks)."""
+        self.hq.view(torch.uint8).zero_()
+        (self.hs_pos if self.scales_by_position else self.hs).fill_(1e-12)
         n = int(lib().moe_layer_local_blocks_bytes(self.T, self.align.max_padded, self.BM))
         return torch.empty(n // 4, dtype=torch.int32, device=self.hq.device)
 
