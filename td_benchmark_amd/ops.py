@@ -921,9 +921,10 @@ class FusedExpertsRunner:
         has now.  The stages after it run over the list that this align writes,
         so a map set in between waits for the next align."""
         m = self.expert_map
-        if m is not None and self.local_blocks is None:  # the first map of a runner built without one
-            self.local_blocks = self._local_list()
-        self._aligned_map = m
+        if m is not self._aligned_map:
+            if self.local_blocks is None:  # the first map of a runner built without one
+                self.local_blocks = self._local_list()
+            self._aligned_map = m
         layer = self._native()
         layer.expert_map = None if m is None else m.data_ptr()
         return layer
