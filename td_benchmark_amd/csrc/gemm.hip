@@ -224,6 +224,7 @@ struct GemmArgs {
   // fields above it moves those that small launches read first into other cache
   // lines of the arguments (Qwen3, one token: 22.1 us a layer, 22.8 so).
   const int32_t* rid;
+  int merged;              // eids may join runs of several experts before a map
 };
 
 // The thread's index.  In a workgroup that runs one tile after another (LOOP)
@@ -1097,8 +1098,8 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   // a run of three blocks in 2-block tiles becomes 1 + 2 blocks, two tiles
   // that stream the same weight tiles at the same pace, rather than 2 + 1,
   // a full tile and a tile of a few padded rows.  Only the last align block
-  // of a run holds padding, so a tile's valid rows are still a prefix (with
-  // virtual blocks, the run's last one may hold no valid row at all).
+  // of an expert holds padding (with virtual blocks, the last one may hold no
+  // valid row at all).
   const int64_t ub = BM / vb;
   const int64_t units = (run + ub - 1) / ub;
   const int64_t in_run = t - b0 * g.n_tiles;
@@ -1128,10 +1129,22 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
     return;
   }
 
-  // Rows of the tile that hold real slots (a prefix: padding follows them).
+  // The rows up to the tile's last one with a slot.  They all hold slots, except
+  // where the block experts come from a map that sends neighbouring experts to
+  // one: their blocks are one run here, with padding between the slots.
   bool row_valid = false;
   if (tid < BM && tid < rows_avail) row_valid = g.sorted[pos0 + tid] < g.S;
-  const int nvalid = __syncthreads_count(row_valid);
+  int nvalid = __syncthreads_count(row_valid);
+  if (g.merged && __syncthreads_or(row_valid && tid >= nvalid)) {
+    for (int r0 = (BM - 1) / 64 * 64; r0 >= 0; r0 -= 64) {
+      const int row = r0 + (tid & 63);
+      const uint64_t slots = __ballot(row < rows_avail && g.sorted[pos0 + row] < g.S);
+      if (slots) {
+        nvalid = r0 + 64 - __clzll((long long)slots);
+        break;
+      }
+    }
+  }
   run_tile<BM, FUSED, EXACT>(g, j, pos0, rows_avail, e, nvalid, units == 1);
 }
 
@@ -1456,6 +1469,7 @@ static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int64_t E) {
 // What the layer knows of its blocks.
 static void set_blocks(GemmArgs& g, const LocalBlocks& local, int TM, int vshift) {
   g.blk = local.blocks;
+  g.merged = local.E_routed == 0 && TM > (g.bma >> vshift);
   if (local.rids) g.rid = local.rids;
   g.runs = local.runs;
   g.share = local.share;
@@ -1590,6 +1604,7 @@ static int setup_plain(GemmArgs& g, int& TM, const void* A, const float* A_scale
   if (!A || !A_scale || !B || !B_scale || !sorted_ids || !expert_ids || !ntpp || !C)
     return kErrNullPointer;
   g = GemmArgs{};
+  g.merged = TM > BM;
   g.A = (const uint8_t*)A;
   g.As = A_scale;
   g.B = (const uint8_t*)B;

@@ -9,7 +9,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from moe_cases import bf16_bits, make_case, to_gpu
+from moe_cases import bf16_bits, make_case, to_gpu, u8_bits
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -102,3 +102,41 @@ def test_replicated_experts_keep_their_own_runs(T, E, k, BM, tile_m, exact, kind
         y = ep.run(g["x"], g["topk_w"], g["topk_ids"])
         torch.cuda.synchronize()
         assert np.array_equal(bf16_bits(y), want)
+
+
+@pytest.mark.parametrize("E,BM,tile_m,exact", [(16, 64, 256, False), (10, 128, 256, False), (10, 128, 256, True),
+                                               (50, 16, 64, False)])
+def test_padding_inside_a_run(E, BM, tile_m, exact):
+    """The align and GEMM calls one by one, under a map that sends neighbours
+    to one local expert: their blocks are one run of the block experts, with
+    padding between the slots of a tile, and every slot is computed."""
+    from td_benchmark_amd import ops
+    print(f"case: padding inside a run E={E} BM={BM} tile_m={tile_m} exact={exact}", flush=True)
+    T, k, I, H = 333, 3, 256, 256
+    c = make_case(T, H, I, E, k, BM, seed=E + BM)
+    g = to_gpu(c)
+    n = E // 2
+    w = [g[name][:n].contiguous() for name in ("w13", "w13_s", "w2", "w2_s")]
+    em = torch.arange(E, dtype=torch.int32, device="cuda") // 2
+    q, s = ops.per_token_group_quant_fp8(g["x"])
+    out = []
+    for tm in (BM, tile_m):
+        srt, eids, ntpp = ops.moe_align_block_size(g["topk_ids"], BM, E, em)
+        hq, hs = ops.gemm_w13_silu_quant(q, s, w[0], w[1], srt, eids, ntpp, T * k, k, BM, tile_m=tm, exact_dot=exact)
+        D = torch.full((T * k, 1, H), 3.0, dtype=torch.bfloat16, device="cuda")
+        ops.dispatch_fused_moe_kernel(hq, w[2], D, hs, w[3], None, g["topk_w"], srt, eids, ntpp, True, 1,
+                                      {"BLOCK_SIZE_M": BM}, a_by_pos=True, tile_m=tm)
+        torch.cuda.synchronize()
+        at = (srt[: int(ntpp)] < T * k).nonzero()[:, 0].cpu().numpy()
+        out.append((u8_bits(hq)[at], hs.cpu().numpy()[at].view(np.uint32), bf16_bits(D)))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    # the N- and K-split calls choose the tile rows by themselves (256 from 160 slots an expert on)
+    for mul, call, kw in ((True, ops.invoke_moe_kernel_n_split, {"N_offset": 0, "N_chunk": H}),
+                          (False, ops.invoke_moe_kernel_k_split, {"K_offset": 0, "K_chunk": I, "is_first_chunk": True})):
+        C, D = (torch.full((T * k, 1, H), 3.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        head = (hs, w[3], None) + ((g["topk_w"],) if mul else ()) + (srt, eids, ntpp, mul, 1, {"BLOCK_SIZE_M": BM})
+        call(hq, w[2], C, *head, **kw, a_by_pos=True)
+        ops.dispatch_fused_moe_kernel(hq, w[2], D, hs, w[3], None, g["topk_w"], srt, eids, ntpp, mul, 1,
+                                      {"BLOCK_SIZE_M": BM}, a_by_pos=True, tile_m=BM)
+        assert np.array_equal(bf16_bits(C), bf16_bits(D))
