@@ -222,8 +222,8 @@ struct AlignArgs {
   int32_t* runs;   // the table of runs, or null (see internal.hpp)
   int32_t* share;  // the counters of shared tiles to clear, of two layers, or null
   int32_t* share2;
-  int64_t max_padded;
-  int S, E, BM, top_k;
+  int max_padded, S, top_k;
+  uint16_t E, BM;  // at most 1024 and 256
 };
 
 // Bit i: the expert of token t's slot i is local.
@@ -468,7 +468,7 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
   hipStream_t st = (hipStream_t)stream;
   if (S <= kAlignOneLaunchSlots) {
     const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share, share2,
-                      max_padded, (int)S, (int)E, (int)BM, (int)top_k};
+                      (int)max_padded, (int)S, (int)top_k, (uint16_t)E, (uint16_t)BM};
     by_slots(S, [&](auto it) {
       hipLaunchKernelGGL(align_expert_kernel<decltype(it)::value>, dim3((unsigned)E), dim3(kAlignThreads), 0, st, a);
     });
@@ -531,7 +531,7 @@ int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int6
   }
   if (!expert_map) local = nullptr;
   const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share, share2,
-                      max_padded, (int)S, (int)E, (int)BM, (int)top_k};
+                      (int)max_padded, (int)S, (int)top_k, (uint16_t)E, (uint16_t)BM};
   const unsigned grid = (unsigned)(E + (q.n_chunks + kAlignThreads - 1) / kAlignThreads);
   by_slots(S, [&](auto it) {
     constexpr int IT = decltype(it)::value;

@@ -195,6 +195,7 @@ struct GemmArgs {
   int64_t run_tiles;       // with runs: a bound on the row tiles
   int64_t share_tiles;     // with runs: the row tiles a launch is sized for
   int unit_tiles;          // with runs: a third of an XCD's expected tiles
+  int merged;              // eids may join runs of several experts before a map
   int64_t n_tiles;         // 256-column n-tiles
   int bma;                 // rows per align block (block_size_m); a tile spans BM / bma of them
   // Exact-dot launches only: the tile map counts virtual blocks of bma >> vshift
@@ -219,12 +220,6 @@ struct GemmArgs {
   int64_t as_pos_ld;
   // Fused epilogue: hs K-major, hs[j * hs_pos_ld + pos] (0: hs[pos * I/128 + j]).
   int64_t hs_pos_ld;
-  // What tells runs of blocks apart: eids, or with blk the experts before the
-  // map (two of them may share a local one, see local_blocks).  Last: among the
-  // fields above it moves those that small launches read first into other cache
-  // lines of the arguments (Qwen3, one token: 22.1 us a layer, 22.8 so).
-  const int32_t* rid;
-  int merged;              // eids may join runs of several experts before a map
 };
 
 // The thread's index.  In a workgroup that runs one tile after another (LOOP)
@@ -1068,24 +1063,25 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   // of up to 65 blocks), longer runs continue 64 blocks at a time.
   int64_t back = 0, fwd = 0;
   const int e = g.eids[bq >> vsh];
+  const int32_t* rid = g.blk ? listed_rid(g.blk, g.eids) : g.eids;
   {
     const int ln = thread_id<T>() & 63;
     const int64_t ib = bq - 1 - ln, jf = bq + 1 + ln;
-    const int id = g.rid[bq >> vsh];
-    const int xb = ib >= 0 ? g.rid[ib >> vsh] : 0;
-    const int xf = jf < n_blocks ? g.rid[jf >> vsh] : 0;
+    const int id = rid[bq >> vsh];
+    const int xb = ib >= 0 ? rid[ib >> vsh] : 0;
+    const int xf = jf < n_blocks ? rid[jf >> vsh] : 0;
     uint64_t end = __ballot(!(ib >= 0 && xb == id));  // blocks before bq with the same expert
     for (int64_t base = bq - 1 - 64; !end; base -= 64) {
       back += 64;
       const int64_t idx = base - ln;
-      end = __ballot(!(idx >= 0 && g.rid[idx >> vsh] == id));
+      end = __ballot(!(idx >= 0 && rid[idx >> vsh] == id));
     }
     back += __ffsll((unsigned long long)end) - 1;
     end = __ballot(!(jf < n_blocks && xf == id));      // and after it
     for (int64_t base = bq + 1 + 64; !end; base += 64) {
       fwd += 64;
       const int64_t idx = base + ln;
-      end = __ballot(!(idx < n_blocks && g.rid[idx >> vsh] == id));
+      end = __ballot(!(idx < n_blocks && rid[idx >> vsh] == id));
     }
     fwd += __ffsll((unsigned long long)end) - 1;
   }
@@ -1470,7 +1466,6 @@ static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int64_t E) {
 static void set_blocks(GemmArgs& g, const LocalBlocks& local, int TM, int vshift) {
   g.blk = local.blocks;
   g.merged = local.E_routed == 0 && TM > (g.bma >> vshift);
-  if (local.rids) g.rid = local.rids;
   g.runs = local.runs;
   g.share = local.share;
   if (local.E_routed > 0) {
@@ -1522,7 +1517,7 @@ int moe::plain_gemm(const void* A, const float* A_scale, const void* B, const fl
   g.B = (const uint8_t*)B;
   g.Bs = B_scale;
   g.sorted = sorted_ids;
-  g.eids = g.rid = expert_ids;
+  g.eids = expert_ids;
   g.ntpp = ntpp;
   g.topk_w = topk_weights;
   g.C = (uint16_t*)C;
@@ -1610,7 +1605,7 @@ static int setup_plain(GemmArgs& g, int& TM, const void* A, const float* A_scale
   g.B = (const uint8_t*)B;
   g.Bs = B_scale;
   g.sorted = sorted_ids;
-  g.eids = g.rid = expert_ids;
+  g.eids = expert_ids;
   g.ntpp = ntpp;
   g.topk_w = topk_weights;
   g.C = (uint16_t*)C;
@@ -1728,7 +1723,7 @@ int moe::w13_gemm(const void* Aq, const float* A_scale, const void* W13, const f
   g.B = (const uint8_t*)W13;
   g.Bs = W13_scale;
   g.sorted = sorted_ids;
-  g.eids = g.rid = expert_ids;
+  g.eids = expert_ids;
   g.ntpp = ntpp;
   g.topk_w = nullptr;
   g.hq = (uint8_t*)hq;

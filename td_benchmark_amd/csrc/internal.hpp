@@ -15,7 +15,6 @@ namespace moe {
 // local expert, so the local ones bound nothing.
 struct LocalBlocks {
   const int32_t* blocks = nullptr;
-  const int32_t* rids = nullptr;  // with blocks: what tells the listed blocks' runs apart
   const int32_t* runs = nullptr;
   int32_t* share = nullptr;
   int64_t E_routed = 0;
@@ -54,6 +53,8 @@ MOE_HOST_DEVICE T* local_eid(T* l, int64_t max_padded, int32_t BM) { return l + 
 
 template <class T>
 MOE_HOST_DEVICE T* local_rid(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 2 * ((max_padded + BM - 1) / BM); }
+// The same from the first two parts of the list, for a kernel that has them.
+MOE_HOST_DEVICE const int32_t* listed_rid(const int32_t* blk, const int32_t* eid) { return eid + (eid - blk); }
 template <class T>
 MOE_HOST_DEVICE T* local_mask(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 3 * ((max_padded + BM - 1) / BM); }
 

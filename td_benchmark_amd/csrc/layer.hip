@@ -18,10 +18,7 @@ using namespace moe;
 static LocalBlocks local_of(const moe_layer* l) {
   LocalBlocks r;
   r.E_routed = l->E_routed;
-  if (l->expert_map) {
-    r.blocks = local_blk(l->local_blocks);
-    r.rids = local_rid(l->local_blocks, l->max_padded, l->block_size_m);
-  }
+  if (l->expert_map) r.blocks = local_blk(l->local_blocks);
   if (l->T * l->top_k <= kRunsMaxSlots) r.runs = l->runs;
   r.share = l->share;
   return r;
