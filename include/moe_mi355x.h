@@ -104,8 +104,8 @@ int moe_align_block_size_mapped(const int32_t* topk_ids, int64_t S, int32_t E, i
 /* A1 + A3 in one call -- the layer's two first stages, which do not depend on
  * each other: moe_quant_group128_padded(x, T, H, q, ldq, scales) and
  * moe_align_block_size[_mapped] (expert_map NULL = unmapped), with the same
- * outputs and argument checks.  One launch where both are small (S <= 16384),
- * the separate kernels otherwise. */
+ * outputs and argument checks.  One launch where both are small (S <= 16384
+ * and S * E <= 12 * 2^20), the separate kernels otherwise. */
 int moe_quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int64_t ldq, float* scales,
                     const int32_t* topk_ids, int64_t S, int32_t E, int32_t block_size_m,
                     const int32_t* expert_map, int32_t* sorted_ids, int32_t* expert_ids, int32_t* ntpp,

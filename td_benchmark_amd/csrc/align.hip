@@ -12,10 +12,10 @@
 // The within-expert order is the stable (ascending slot) order, so the result
 // is deterministic and bit-exact against the CPU restatement.
 //
-// Up to 16384 slots one launch with a workgroup per expert (align_expert)
-// computes everything, alone or beside the activation quant in the same launch
-// (the two do not depend on each other); above that three launches, none of
-// which waits on another workgroup:
+// Up to 16384 slots (fewer from 768 experts on, but for a layer) one launch with
+// a workgroup per expert (align_expert) computes everything, alone or beside the
+// activation quant in the same launch (the two do not depend on each other);
+// above that three launches, none of which waits on another workgroup:
 //   1. count:  1024 slots per workgroup.  Slots with equal expert inside a wave
 //      are found with log2(E) ballots (a match-any built from per-bit ballots),
 //      giving each slot its rank among equal-expert slots of its wave; per-wave
@@ -241,13 +241,30 @@ MOE_DEVICE int32_t local_slots(const int32_t* ids, const int32_t* expert_map, in
   return (int32_t)m;
 }
 
+// Each expert's count is kept in COPIES words, by lane: a wave's slots of one
+// expert add to eight words at a time, where 64 adds to one word follow each
+// other.  A call of align alone with every slot on one expert took, with one
+// word, with eight, and in three launches (us; the smallest launch takes 6 to 7
+// so): S = 8192, E = 64: 12.8, 7.0, 13.0; S = 16384, E = 64: 19.0, 7.3, 13.0;
+// S = 16384, E = 256, Zipf: 9.1, 7.2, 13.0.  Up to 1024 slots the few adds cost
+// less than the longer sums (0.15 us).
 constexpr int kAlignThreads = 512;
 constexpr int kAlignWaves = kAlignThreads / 64;
 
 // IT: ids a lane holds (IT * 512 >= S).
 template <int IT>
 MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
-  __shared__ int32_t hist[kAlignMaxExperts];
+  constexpr int COPIES = IT > 2 ? 8 : 1;
+  __shared__ __attribute__((aligned(16))) int32_t hist[kAlignMaxExperts * COPIES];
+  auto count_of = [&](int x) {
+    if constexpr (COPIES == 1) {
+      return hist[x];
+    } else {
+      const v4i* c = reinterpret_cast<const v4i*>(hist + x * COPIES);
+      const v4i s = c[0] + c[1];
+      return s[0] + s[1] + s[2] + s[3];
+    }
+  };
   __shared__ int32_t wave_cnt[kAlignWaves], wave_before[kAlignWaves], wave_total[kAlignWaves];
   __shared__ int32_t wave_lbefore[kAlignWaves], wave_ltotal[kAlignWaves];
   __shared__ int32_t wave_rank[kAlignWaves], wave_runs[kAlignWaves];
@@ -258,12 +275,12 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   int id[IT];
 #pragma unroll
   for (int i = 0; i < IT; ++i) id[i] = first + 64 * i < a.S ? a.ids[first + 64 * i] : -1;
-  for (int i = tid; i < a.E; i += kAlignThreads) hist[i] = 0;
+  for (int i = tid; i < a.E * COPIES; i += kAlignThreads) hist[i] = 0;
   __syncthreads();
   int mine = 0;  // this wave's slots of expert e
 #pragma unroll
   for (int i = 0; i < IT; ++i) {
-    if ((unsigned)id[i] < (unsigned)a.E) atomicAdd(&hist[id[i]], 1);
+    if ((unsigned)id[i] < (unsigned)a.E) atomicAdd(&hist[id[i] * COPIES + lane % COPIES], 1);
     mine += __popcll(__ballot(id[i] == e));
   }
   if (lane == 0) wave_cnt[wave] = mine;
@@ -271,16 +288,17 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   int before = 0, total = 0;    // padded sizes of the experts before e, and of all
   int lbefore = 0, ltotal = 0;  // and of the local ones among them
   int place = 0, n_runs = 0;    // experts here with more slots than e (or as many and before it), and with any
-  const int own = hist[e];
+  const int own = count_of(e);
   for (int x = tid; x < a.E; x += kAlignThreads) {
-    const int p = (hist[x] + a.BM - 1) >> sh << sh;
+    const int c = count_of(x);
+    const int p = (c + a.BM - 1) >> sh << sh;
     total += p;
     if (x < e) before += p;
     if (!a.expert_map || a.expert_map[x] >= 0) {
       ltotal += p;
       if (x < e) lbefore += p;
       n_runs += p > 0;
-      place += hist[x] > own || (hist[x] == own && x < e);
+      place += c > own || (c == own && x < e);
     }
   }
 #pragma unroll
@@ -411,7 +429,11 @@ __global__ __launch_bounds__(kAlignThreads) void quant_align_kernel(AlignArgs a,
     quant_chunks<kAlignThreads, 1, false, WHOLE>(q, (int64_t)blockIdx.x - a.E);
 }
 
-// The one-launch form holds up to 32 ids a lane.
+// The one-launch form holds up to 32 ids a lane.  Every workgroup reads every
+// slot: with near 1024 experts and all 16384 slots align alone takes 16.5 to
+// 18.6 us so and 16 in three launches (1024 experts, 8192 slots: 11.2 to 12.4
+// and 14; 256, 16384: 7.2 and 13), which only the layer's table of runs outweighs.
+constexpr int64_t kAlignOneLaunchReads = (int64_t)12 << 20;
 constexpr int64_t kAlignOneLaunchSlots = 32 * kAlignThreads;
 static_assert(kAlignOneLaunchSlots == kRunsMaxSlots, "the one-launch form writes the table of runs");
 // Chunks (16 B of input) up to which the quant runs beside align; larger ones
@@ -450,11 +472,16 @@ static int align_args(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
   return kOk;
 }
 
+static bool align_one_launch(int64_t S, int32_t E, const int32_t* runs) {
+  return S <= kAlignOneLaunchSlots && (runs || S * E <= kAlignOneLaunchReads);
+}
+
 // f(ids a lane holds) for the one-launch form.
 template <class F>
 static void by_slots(int64_t S, F&& f) {
   if (S <= 2 * kAlignThreads) f(std::integral_constant<int, 2>{});
   else if (S <= 8 * kAlignThreads) f(std::integral_constant<int, 8>{});
+  else if (S <= 16 * kAlignThreads) f(std::integral_constant<int, 16>{});
   else f(std::integral_constant<int, 32>{});
 }
 
@@ -466,7 +493,7 @@ static int align_impl(const int32_t* topk_ids, int64_t S, int32_t E, int32_t BM,
   if (arg_rc != kOk) return arg_rc;
   if (!expert_map) local = nullptr;
   hipStream_t st = (hipStream_t)stream;
-  if (S <= kAlignOneLaunchSlots) {
+  if (align_one_launch(S, E, runs)) {
     const AlignArgs a{topk_ids, expert_map, sorted_ids, expert_ids, ntpp, local, runs, share, share2,
                       (int)max_padded, (int)S, (int)top_k, (uint16_t)E, (uint16_t)BM};
     by_slots(S, [&](auto it) {
@@ -522,7 +549,7 @@ int moe::quant_align(const void* x_bf16, int64_t T, int64_t H, void* q_fp8, int6
   const int rc = align_args(topk_ids, S, E, BM, sorted_ids, expert_ids, ntpp, max_padded, true, workspace);
   if (rc != kOk) return rc;
   const QuantArgs q = quant_args(x_bf16, T, H, q_fp8, ldq, scales);
-  if (S > kAlignOneLaunchSlots || q.n_chunks == 0 || q.n_chunks > kQuantBesideAlign ||
+  if (!align_one_launch(S, E, runs) || q.n_chunks == 0 || q.n_chunks > kQuantBesideAlign ||
       !quant_vectorised(x_bf16, H, q_fp8, ldq)) {
     const int qrc = moe_quant_group128_padded(x_bf16, T, H, q_fp8, ldq, scales, stream);
     if (qrc != kOk) return qrc;

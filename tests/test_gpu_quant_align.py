@@ -25,6 +25,10 @@ CASES = [
     (4097, 1, 1000, 32, 100, "skewed"),    # S = 4097, general quant
     (2048, 8, 256, 128, 1160, "mapped"),   # S = 16384
     (16385, 1, 64, 16, 128, "mapped"),     # three launches
+    (8192, 1, 96, 32, 128, "skewed"),      # 16 ids a lane
+    (8193, 1, 300, 16, 128, "one"),        # 32 ids a lane, all to one count
+    (12288, 1, 1024, 16, 128, "skewed"),   # the most reads of one launch
+    (12289, 1, 1024, 16, 128, "uniform"),  # past them: three launches
 ]
 
 
