@@ -109,8 +109,10 @@ MOE_DEVICE void quant_chunks(const QuantArgs& a, int64_t blk) {
       hi = pad ? 0u : pack4_e4m3(v[4], v[5], v[6], v[7]);
     }
     if (ch < a.n_chunks) {
-      if (WHOLE || SWIGLU || col[i] < a.ldq)
-        __builtin_nontemporal_store((v2u){lo, hi}, reinterpret_cast<v2u*>(a.q + row[i] * a.ldq + col[i]));
+      // dense rows: chunk ch of the codes too, and no row and column kept through the codes' registers
+      if (WHOLE || col[i] < a.ldq)
+        __builtin_nontemporal_store((v2u){lo, hi},
+                                    reinterpret_cast<v2u*>(a.q + (WHOLE ? ch * 8 : row[i] * a.ldq + col[i])));
       if ((tid & 15) == 0) a.s[ch >> 4] = sc;
     }
   }
