@@ -12,15 +12,30 @@ from moe_cases import bf16_bits, make_case, to_gpu, u8_bits
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
-# (T, H, I, E, k, BM): tiles = min(S, E) and more blocks by I/128; four workgroups a tile up to 64, two up to 128
-CASES = [(1, 1024, 384, 16, 8, 32), (1, 2048, 2048, 8, 4, 32), (5, 1024, 1024, 4, 2, 32), (16, 1152, 256, 8, 4, 64),
-         (40, 1024, 640, 4, 2, 32), (33, 1024, 1024, 16, 1, 64), (3, 1024, 1408, 16, 3, 16)]
+# (T, H, I, E, k, BM, workgroups that share a W13 tile of the routed layer)
+CASES = [(1, 1024, 384, 16, 8, 32, 4), (1, 2048, 2048, 8, 4, 32, 4), (5, 1024, 1024, 4, 2, 32, 4),
+         (16, 1152, 256, 8, 4, 64, 4), (40, 1024, 640, 4, 2, 32, 4), (33, 1024, 1024, 16, 1, 64, 2),
+         (1, 1024, 2048, 16, 8, 32, 2),   # 128 tiles of 32 rows
+         (5, 1024, 1664, 16, 1, 32, 2),   # 65
+         (4, 1024, 1024, 16, 2, 32, 4),   # 64
+         (90, 1024, 1024, 8, 2, 32, 2),   # several blocks an expert
+         (3, 1024, 5504, 4, 1, 32, 1),    # 129: whole tiles
+         (3, 1024, 1408, 16, 3, 16, 1)]   # 16-row tiles are whole (the shared expert's, of 16 rows too)
 
 
-@pytest.mark.parametrize("T,H,I,E,k,BM", CASES)
-def test_shared_tiles_equal_whole_ones(T, H, I, E, k, BM):
+def _parts(T, H, I, E, k, BM):
+    """Workgroups a tile, from the tiles that the slots can make at most."""
+    S = T * k
+    m = min(S, E)
+    tiles = (m + (S - m) // BM) * (I // 128)
+    return 1 if BM < 32 or H < 1024 or tiles > 128 else 4 if tiles <= 64 else 2
+
+
+@pytest.mark.parametrize("T,H,I,E,k,BM,parts", CASES)
+def test_shared_tiles_equal_whole_ones(T, H, I, E, k, BM, parts):
     from td_benchmark_amd import ops
-    print(f"case: shared tiles T={T} H={H} I={I} E={E} k={k} BM={BM}", flush=True)
+    print(f"case: shared tiles T={T} H={H} I={I} E={E} k={k} BM={BM} parts={parts}", flush=True)
+    assert _parts(T, H, I, E, k, BM) == parts
     c = make_case(T, H, I, E, k, BM, seed=T + I)
     g = to_gpu(c)
     w = [g[n] for n in ("w13", "w13_s", "w2", "w2_s")]
