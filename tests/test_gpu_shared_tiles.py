@@ -134,3 +134,29 @@ def test_shared_tiles_in_graphs_and_on_streams(T, H, I, E, k, BM):
         last = s
         torch.cuda.current_stream().wait_stream(s)
         assert torch.equal(got, want[n % 2])
+
+
+@pytest.mark.parametrize("T,H,I,E,k,BM,parts", [(5, 1024, 1024, 4, 2, 32, 4), (33, 1024, 1024, 16, 1, 64, 2)])
+def test_shared_tiles_with_infinities_and_nans(T, H, I, E, k, BM, parts):
+    """Rows with infinities, NaNs of both signs and values that overflow in the
+    dots give the whole tiles' bits too."""
+    print(f"case: shared tiles, infinities and NaNs, T={T} H={H} I={I} E={E} k={k} BM={BM}", flush=True)
+    assert _parts(T, H, I, E, k, BM) == parts
+    g, r = _layer(T, H, I, E, k, BM)
+    x = g["x"]
+    x[0, 3] = float("nan")
+    x[1, 5] = -float("nan")
+    x[2, 7] = float("inf")
+    x[3, 9] = -float("inf")
+    x[4] *= 3e38
+    out = []
+    for share in (True, False):
+        if not share:
+            r._layer.share = r._shared_layer.share = None
+        r.hq.view(torch.uint8).fill_(0x55)
+        y = r.run(x, g["topk_w"], g["topk_ids"]).clone()
+        torch.cuda.synchronize()
+        at = (r.align.sorted_ids[: int(r.align.ntpp)] < T * k).nonzero()[:, 0].cpu().numpy()
+        out.append((u8_bits(r.hq)[at], r.hs.cpu().numpy()[at].view(np.uint32), bf16_bits(y), bf16_bits(r.shared_out)))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
