@@ -346,8 +346,7 @@ MOE_DEVICE void align_expert(const AlignArgs& a, int e) {
   if (a.local && local >= 0) {
     for (int i = tid; i < padded >> sh; i += kAlignThreads) {
       local_blk(a.local)[(lbefore >> sh) + i] = (before >> sh) + i;
-      local_eid(a.local, a.max_padded, a.BM)[(lbefore >> sh) + i] = local;
-      local_rid(a.local, a.max_padded, a.BM)[(lbefore >> sh) + i] = e;
+      local_eid(a.local, a.max_padded, a.BM)[(lbefore >> sh) + i] = block_word(e, local);
     }
   }
   // the tokens' local slots, and the positions and blocks past ntpp, shared out over the workgroups
@@ -410,8 +409,7 @@ __global__ __launch_bounds__(1024) void local_blocks_kernel(const int32_t* __res
     }
     if (e >= 0) {
       local_blk(local)[at + __popcll(m & lt)] = b;
-      local_eid(local, max_padded, BM)[at + __popcll(m & lt)] = e;
-      local_rid(local, max_padded, BM)[at + __popcll(m & lt)] = ids[sorted[(int64_t)b * BM]];
+      local_eid(local, max_padded, BM)[at + __popcll(m & lt)] = block_word(ids[sorted[(int64_t)b * BM]], e);
     }
     __syncthreads();
   }
@@ -594,13 +592,14 @@ extern "C" int moe_align_block_size_mapped(const int32_t* topk_ids, int64_t S, i
 }
 
 // ---------------------------------------------------------------------------
-// Allocation-free align: the same three kernels with their workspace in a
-// file-scope device array instead of caller memory, for callers that cannot
-// allocate (code under graph capture, tight serving loops).  Each GPU holds
-// its own copy of the array until the process ends; every call on a GPU
-// shares it, so calls that overlap on one GPU race.  Nothing in the workspace
-// needs clearing: every call writes each chunk count, rank, offset and count
-// that it later reads.
+// Allocation-free align: the same kernels, the three launches with their
+// workspace in a file-scope device array instead of caller memory, for callers
+// that cannot allocate (code under graph capture, tight serving loops).  Each
+// GPU holds its own copy of the array until the process ends; every call on a
+// GPU that takes three launches shares it, so such calls race where they
+// overlap.  Nothing in the workspace needs clearing: every call writes each
+// chunk count, rank, offset and count that it later reads.  (The one launch
+// uses no workspace.)
 
 namespace moe {
 

@@ -168,6 +168,8 @@ struct Tile {
   static_assert(VM * (KS - 2) < 64, "vmcnt immediate");
 };
 
+constexpr int kMergedRuns = 1 << 16;  // added to GemmArgs::bma
+
 struct GemmArgs {
   const uint8_t* A;        // fp8 [rows, K]
   const float* As;         // [rows, K/128]
@@ -177,8 +179,8 @@ struct GemmArgs {
   const int32_t* eids;     // [max_blocks]
   const int32_t* ntpp;     // [1]
   // Expert parallelism (else null): the align blocks of local experts in
-  // ascending order; eids and ntpp then describe this list, and the other
-  // blocks are no part of the launch.
+  // ascending order; eids (as words, see block_word) and ntpp then describe this
+  // list, and the other blocks are no part of the launch.
   const int32_t* blk;
   const int32_t* runs;     // the experts' runs by descending rows (see internal.hpp), or null
   int32_t* share;          // fused: counters and rows of tiles that several workgroups share, or null
@@ -195,9 +197,11 @@ struct GemmArgs {
   int64_t run_tiles;       // with runs: a bound on the row tiles
   int64_t share_tiles;     // with runs: the row tiles a launch is sized for
   int unit_tiles;          // with runs: a third of an XCD's expected tiles
-  int merged;              // eids may join runs of several experts before a map
   int64_t n_tiles;         // 256-column n-tiles
-  int bma;                 // rows per align block (block_size_m); a tile spans BM / bma of them
+  // Rows per align block (block_size_m); a tile spans BM / bma of them.  With
+  // kMergedRuns added where a run of eids may hold several experts before a map
+  // (a field of its own, read late, cost an expert-parallel rank's layer 0.3 %).
+  int bma;
   // Exact-dot launches only: the tile map counts virtual blocks of bma >> vshift
   // rows (align block b is virtual blocks b << vshift ..), so 128-row tiles can
   // run over 256-row align blocks.  0 everywhere else.
@@ -1030,7 +1034,8 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   // fetch the weight tile from HBM once.
   const int ntpp = *g.ntpp;
   const int vsh = EXACT ? g.vshift : 0;
-  const int64_t vb = (int64_t)g.bma >> vsh;  // rows of a (virtual) block
+  const int bma = g.bma & (kMergedRuns - 1);
+  const int64_t vb = (int64_t)bma >> vsh;  // rows of a (virtual) block
   const int64_t n_blocks = ntpp / vb;
   const int64_t total = n_blocks * g.n_tiles;
   const int64_t per_xcd = (total + kXcds - 1) / kXcds;
@@ -1058,33 +1063,33 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   }
   if (t >= total) return;
   const int64_t bq = t / g.n_tiles;  // a block of the tile's run
-  // The run of blocks with bq's expert: the run ids of bq and of the 64
+  // The run of blocks with bq's expert: the expert ids (or words) of bq and of the 64
   // blocks on either side are loaded together (one memory round trip for runs
   // of up to 65 blocks), longer runs continue 64 blocks at a time.
   int64_t back = 0, fwd = 0;
-  const int e = g.eids[bq >> vsh];
-  const int32_t* rid = g.blk ? listed_rid(g.blk, g.eids) : g.eids;
+  int word;  // of bq
   {
     const int ln = thread_id<T>() & 63;
     const int64_t ib = bq - 1 - ln, jf = bq + 1 + ln;
-    const int id = rid[bq >> vsh];
-    const int xb = ib >= 0 ? rid[ib >> vsh] : 0;
-    const int xf = jf < n_blocks ? rid[jf >> vsh] : 0;
-    uint64_t end = __ballot(!(ib >= 0 && xb == id));  // blocks before bq with the same expert
+    word = g.eids[bq >> vsh];
+    const int xb = ib >= 0 ? g.eids[ib >> vsh] : 0;
+    const int xf = jf < n_blocks ? g.eids[jf >> vsh] : 0;
+    uint64_t end = __ballot(!(ib >= 0 && xb == word));  // blocks before bq with the same expert
     for (int64_t base = bq - 1 - 64; !end; base -= 64) {
       back += 64;
       const int64_t idx = base - ln;
-      end = __ballot(!(idx >= 0 && rid[idx >> vsh] == id));
+      end = __ballot(!(idx >= 0 && g.eids[idx >> vsh] == word));
     }
     back += __ffsll((unsigned long long)end) - 1;
-    end = __ballot(!(jf < n_blocks && xf == id));      // and after it
+    end = __ballot(!(jf < n_blocks && xf == word));      // and after it
     for (int64_t base = bq + 1 + 64; !end; base += 64) {
       fwd += 64;
       const int64_t idx = base + ln;
-      end = __ballot(!(idx < n_blocks && rid[idx >> vsh] == id));
+      end = __ballot(!(idx < n_blocks && g.eids[idx >> vsh] == word));
     }
     fwd += __ffsll((unsigned long long)end) - 1;
   }
+  const int e = g.blk ? local_of_word(word) : word;
   const int64_t b0 = bq - back;
   const int64_t run = back + 1 + fwd;
   // A row tile spans up to ub consecutive align blocks of the run (one when BM
@@ -1115,7 +1120,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   const int64_t u = by_col ? in_grp % units : in_grp / gsz;  // row tile of the run
   const int64_t base = run / units, n_short = units - run % units;  // n_short tiles of `base` blocks
   const int64_t b = b0 + (u < n_short ? u * base : n_short * base + (u - n_short) * (base + 1));
-  // sorted position of tile row 0 (the blocks of one run id are consecutive in the sorted order too)
+  // sorted position of tile row 0 (the listed blocks of one word are consecutive in the sorted order too)
   const int64_t pos0 = (g.blk ? ((int64_t)g.blk[b >> vsh] << vsh) + (b & ((1 << vsh) - 1)) : b) * vb;
   // tile rows that belong to this run (the rest are not read or written)
   const int rows_avail = (int)((u < n_short ? base : base + 1) * vb);
@@ -1131,7 +1136,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GemmArgs& g) {
   bool row_valid = false;
   if (tid < BM && tid < rows_avail) row_valid = g.sorted[pos0 + tid] < g.S;
   int nvalid = __syncthreads_count(row_valid);
-  if (g.merged && __syncthreads_or(row_valid && tid >= nvalid)) {
+  if (g.bma != bma && __syncthreads_or(row_valid && tid >= nvalid)) {
     for (int r0 = (BM - 1) / 64 * 64; r0 >= 0; r0 -= 64) {
       const int row = r0 + (tid & 63);
       const uint64_t slots = __ballot(row < rows_avail && g.sorted[pos0 + row] < g.S);
@@ -1302,7 +1307,8 @@ void w13_exact_kernel(GemmArgs g) {
 //     tile's first loads depend on (the block's expert and its neighbours', the
 //     slots, the row count) is read in one round trip instead of a chain of three;
 //   - one workgroup has its CU to itself and the whole LDS as its operand ring:
-//     up to six stages in flight instead of one;
+//     two to six stages in flight instead of one (up to nine of the smaller
+//     stages of a shared tile);
 //   - four waves only issue loads and four only compute: where every wave does
 //     both, a step is the time to queue its 37 loads (the CU's address unit takes
 //     64 B a cycle) plus the time to compute;
@@ -1322,7 +1328,7 @@ __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
   // within max_padded for every b of the grid (the entries past ntpp are not used)
   const int64_t blk = g.blk ? (b < n_blocks ? g.blk[b] : 0) : b;
   const int64_t pos0 = blk * T::BM;
-  const int e = g.eids[b];
+  const int word = g.eids[b], e = g.blk ? local_of_word(word) : word;
   const int before = b > 0 ? g.eids[b - 1] : -1;
   const int after = b + 1 < g.max_blocks ? g.eids[b + 1] : -1;
   bool row_valid = false;
@@ -1333,7 +1339,7 @@ __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
     if (part == 0) zero_tile<T, FUSED>(g, j, pos0, T::BM);
     return;
   }
-  const bool single = before != e && !(b + 1 < n_blocks && after == e);  // the expert's only row tile
+  const bool single = before != word && !(b + 1 < n_blocks && after == word);  // the expert's only row tile
   gemm_tile<T, FUSED, EXACT>(g, j, pos0, T::BM, e, nvalid, single, (int)part, (int)tile);
 }
 
@@ -1465,7 +1471,7 @@ static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int64_t E) {
 // What the layer knows of its blocks.
 static void set_blocks(GemmArgs& g, const LocalBlocks& local, int TM, int vshift) {
   g.blk = local.blocks;
-  g.merged = local.E_routed == 0 && TM > (g.bma >> vshift);
+  if (local.E_routed == 0 && TM > (g.bma >> vshift)) g.bma |= kMergedRuns;
   g.runs = local.runs;
   g.share = local.share;
   if (local.E_routed > 0) {
@@ -1599,7 +1605,6 @@ static int setup_plain(GemmArgs& g, int& TM, const void* A, const float* A_scale
   if (!A || !A_scale || !B || !B_scale || !sorted_ids || !expert_ids || !ntpp || !C)
     return kErrNullPointer;
   g = GemmArgs{};
-  g.merged = TM > BM;
   g.A = (const uint8_t*)A;
   g.As = A_scale;
   g.B = (const uint8_t*)B;
@@ -1615,7 +1620,7 @@ static int setup_plain(GemmArgs& g, int& TM, const void* A, const float* A_scale
   g.max_blocks = (max_padded + BM - 1) / BM;
   g.max_padded = max_padded;
   g.n_tiles = (N / 128 + 1) / 2;
-  g.bma = BM;
+  g.bma = TM > BM ? BM | kMergedRuns : BM;
   g.top_k = top_k;
   g.a_by_pos = a_by_pos ? 1 : 0;
   g.E = E;

@@ -40,11 +40,19 @@ inline int64_t blocks_bound(int64_t S, int64_t E, int64_t BM) {
 constexpr int kShareTiles = 128;
 constexpr int kShareRows = 64;
 
-// local_blocks holds [0] local blocks * BM, then the blocks, then their local
-// expert ids, then the experts that the ids select (a map may send several of
-// them to one local expert: listed one after another they are two runs, with
-// other blocks or padding between their slots), then a word per token whose bit
-// i says that slot i's expert is local.
+// local_blocks holds [0] local blocks * BM, then the blocks, then a word for each
+// with its expert, then a word per token whose bit i says that slot i's expert
+// is local.  A block's word has the local expert in its low bits and the expert
+// before the map above them: a map may send several to one local expert, whose
+// blocks, one after another in the list, are still runs of their own with other
+// blocks or padding between their slots.  One word holds both, so that a tile
+// has its run and its expert from one load.
+constexpr int kLocalExpertBits = 20;
+MOE_HOST_DEVICE int32_t block_word(int32_t e, int32_t local) {
+  const int32_t most = (1 << kLocalExpertBits) - 1;  // a local expert that is not here stays none
+  return e << kLocalExpertBits | (local < most ? local : most);
+}
+MOE_HOST_DEVICE int32_t local_of_word(int32_t w) { return w & ((1 << kLocalExpertBits) - 1); }
 inline const int32_t* local_rows(const int32_t* l) { return l; }
 template <class T>
 MOE_HOST_DEVICE T* local_blk(T* l) { return l + 1; }
@@ -52,11 +60,7 @@ template <class T>
 MOE_HOST_DEVICE T* local_eid(T* l, int64_t max_padded, int32_t BM) { return l + 1 + (max_padded + BM - 1) / BM; }
 
 template <class T>
-MOE_HOST_DEVICE T* local_rid(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 2 * ((max_padded + BM - 1) / BM); }
-// The same from the first two parts of the list, for a kernel that has them.
-MOE_HOST_DEVICE const int32_t* listed_rid(const int32_t* blk, const int32_t* eid) { return eid + (eid - blk); }
-template <class T>
-MOE_HOST_DEVICE T* local_mask(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 3 * ((max_padded + BM - 1) / BM); }
+MOE_HOST_DEVICE T* local_mask(T* l, int64_t max_padded, int32_t BM) { return l + 1 + 2 * ((max_padded + BM - 1) / BM); }
 
 int plain_gemm(const void* A, const float* A_scale, const void* B, const float* B_scale, const int32_t* sorted_ids,
                const int32_t* expert_ids, const int32_t* ntpp, const float* topk_weights, int64_t S, int32_t top_k,

@@ -26,7 +26,7 @@ static LocalBlocks local_of(const moe_layer* l) {
 
 extern "C" int64_t moe_layer_local_blocks_bytes(int64_t T, int64_t max_padded, int32_t BM) {
   if (T < 0 || max_padded < 0 || !block_m_ok(BM)) return -1;
-  return 4 * (1 + 3 * ((max_padded + BM - 1) / BM) + T);
+  return 4 * (1 + 2 * ((max_padded + BM - 1) / BM) + T);
 }
 
 extern "C" int64_t moe_layer_share_bytes(void) { return (4 + 2 * 128 * kShareRows) * (int64_t)kShareTiles; }
@@ -56,6 +56,7 @@ extern "C" int moe_layer_scales(const moe_layer* l, void* stream) {
 
 extern "C" int moe_layer_w13(const moe_layer* l, void* stream) {
   if (!l || (l->expert_map && !l->local_blocks)) return kErrNullPointer;
+  if (l->expert_map && l->E >> kLocalExpertBits) return kErrBadExperts;
   return w13_gemm(l->q1, l->s1_pos ? l->s1_pos : l->s1, l->w13, l->w13_scale, l->sorted_ids,
                   l->expert_map ? local_eid(l->local_blocks, l->max_padded, l->block_size_m) : l->expert_ids,
                   l->expert_map ? local_rows(l->local_blocks) : l->ntpp, l->T * l->top_k, l->top_k, l->Hp, l->I, l->E,
@@ -65,6 +66,7 @@ extern "C" int moe_layer_w13(const moe_layer* l, void* stream) {
 
 extern "C" int moe_layer_w2(const moe_layer* l, const float* topk_weights, void* stream) {
   if (!l || (l->expert_map && !l->local_blocks)) return kErrNullPointer;
+  if (l->expert_map && l->E >> kLocalExpertBits) return kErrBadExperts;
   return plain_gemm(l->hq, l->hs, l->w2, l->w2_scale, l->sorted_ids,
                     l->expert_map ? local_eid(l->local_blocks, l->max_padded, l->block_size_m) : l->expert_ids,
                     l->expert_map ? local_rows(l->local_blocks) : l->ntpp, topk_weights, l->T * l->top_k, 1, 1, l->Hp,

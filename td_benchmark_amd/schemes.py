@@ -185,6 +185,9 @@ def build(cfg: Any, ctx: Any, data: Any, scheme_cfg: Any) -> SchemeInstance:
         return live().run(hidden, wts, ids)
 
     def run_staged() -> StageResult:
+        # Each stage by itself: the sum is over what run() takes, which has quant
+        # and align in one launch up to 16384 slots and lets several workgroups
+        # share a tile of a small shared expert's W13.
         runner = live()
         if not isinstance(runner, ops.FusedExpertsRunner):
             return StageResult(output=run(), stage_ms={})
