@@ -402,8 +402,10 @@ def main() -> int:
         step()
     torch.cuda.synchronize()
     start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-    # The layer as a caller runs it: K steps, one event pair around each for the
-    # per-step samples and nothing between its launches.
+    # The layer, one stage after another: K steps, one event pair around each for
+    # the per-step samples and nothing between its launches.  (runner.run() takes
+    # the same kernels from one call, except that up to 16384 slots it runs quant
+    # and align in one launch: the layers of that size run faster so.)
     sev = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)) for _ in range(args.steps)]
     torch.cuda.synchronize()
     start.record()
