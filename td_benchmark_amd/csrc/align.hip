@@ -208,10 +208,11 @@ __global__ __launch_bounds__(256) void align_place_kernel(
 // slots in ascending order (each wave owns a contiguous stretch of the slots;
 // ballots give a slot its rank).  No workgroup waits on another one.
 // Bound by its chain of about four dependent steps, not by bytes.  Against the
-// three launches it replaces (kernel time): S = 8192, E = 64: 7.8 us with the
-// quant in the same launch, 19 us before (quant 5.0, count, scan and place 4.7
-// each); S = 2408, E = 128: 4.9 us, before 17; against the former single
-// workgroup for S <= 1024 with the quant: S = 128, E = 8: 3.1 us, before 6.6.
+// three launches it replaces (kernel time, with the table of runs and the other
+// notes that a layer's align leaves): S = 8192, E = 64: 7.8 us with the quant in
+// the same launch, 19 us before (quant 5.0, count, scan and place 4.7 each);
+// S = 2408, E = 128: 5.1 us, before 17; against the former single workgroup for
+// S <= 1024 with the quant: S = 128, E = 8: 3.9 us, before 6.6.
 struct AlignArgs {
   const int32_t* ids;
   const int32_t* expert_map;  // or null

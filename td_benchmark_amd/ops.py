@@ -580,24 +580,35 @@ def get_moe_config(num_tokens: int, num_experts: int, top_k: int) -> dict[str, i
     num_tokens * top_k / num_experts, by a sweep of the whole layer over
     block sizes 16-256 on MI355X (four expert shapes: H/I/E/top-k of
     DeepSeek-V3, Mixtral, Qwen3-30B-A3B and the reference's v1 GroupGEMM
-    sweep, 4-1024 rows per expert):
+    sweep, 4-500 rows per expert, even routing; us a layer):
 
     * avg <= 28: 32.  The layer streams its weights; the 32-row tile streams
-      them faster than the 16-row one and wastes less than taller blocks.
+      them faster than the 16-row one and wastes less than taller blocks
+      (DeepSeek-V3 at 16 rows: 1786, 2025 at 16 and 1980 at 64; at 4 rows
+      16-row blocks are 1-2 % faster on it and Qwen3, 4-13 % slower on the
+      others).
     * avg <= 44: 64.  Most experts now fill a 32-row block and spill into a
       second one; 64-row blocks keep them in one tile (40 rows per expert:
-      DeepSeek-V3 2151 us against 2588 at 32, Mixtral 336 against 402,
-      Qwen3 161 against 176, v1 186 against 198; within 2 % of the best
-      block size on all four shapes at 32 and 40 rows).
+      DeepSeek-V3 2083 against 2499 at 32, Mixtral 335 against 386, Qwen3 152
+      against 166, v1 172 against 184; the best size on all four).
     * avg <= 100: 128.  Most experts fit one block; a 128-row tile reads
-      fewer LDS bytes per MFMA than a 64-row one (v1 shape, 64 rows per
-      expert: 195 us against 209 at 64; DeepSeek-V3: 2208 against 2606).
+      fewer LDS bytes per MFMA than a 64-row one (64 rows per expert: v1 186
+      against 200 at 64, DeepSeek-V3 2216 against 2571; Qwen3 at 100 rows is
+      1.5 % faster with 256).
     * above: 256, so that an expert's rows stay in one tile instead of
-      spilling a few rows into a second one (128 rows per expert: 237 against
-      244 us at 128; Qwen3 at 160: 241 against 299) -- except when the average
-      sits at 240-288 rows, where half the experts would spill a few rows into
-      a second 256-row block and 128-row blocks split them evenly over two
-      256-row tiles instead (DeepSeek-V3 at 256: 3920 against 4058 us)."""
+      spilling a few rows into a second one (128 rows per expert: DeepSeek-V3
+      2765 against 2920 at 128, Qwen3 219 against 223, v1 223 against 219;
+      Qwen3 at 160: 245 against 269) -- except when the average sits at
+      240-288 rows, where half the experts would spill a few rows into a
+      second 256-row block and 128-row blocks split them evenly over two
+      256-row tiles instead (DeepSeek-V3 at 256: 3953 against 4025, at 288
+      4787 against 4685; Qwen3 at 256 345 against 336, the others even).
+
+    The rule does not see how uneven the routing is.  Under Zipf routing (1.2)
+    the size it picks is the best or within 3 % at 16 rows and at most of the
+    others, but 20-25 % slower than 32 rows at 40 rows of Qwen3 and v1 (182
+    and 203 us, 152 and 162), and 6-9 % slower than the other of 128 and 256
+    at 40 and 128 rows of DeepSeek-V3 and 256 of Qwen3."""
     avg = num_tokens * top_k / max(num_experts, 1)
     if avg <= 28:
         bm = 32
