@@ -882,6 +882,7 @@ class FusedExpertsRunner:
         self.runs = torch.empty(int(lib().moe_layer_runs_bytes(n_align)) // 4, dtype=torch.int32, device=dev)
         # tiles that several workgroups share: small decode
         self.share = _share_buffer(self.S, dev)
+        self._shared_share = _share_buffer(self.T, dev) if shared is not None else None
         if out is not None:
             _need(out, "out", torch.bfloat16)
             if tuple(out.shape) != (self.T, H):
@@ -957,7 +958,8 @@ class FusedExpertsRunner:
         # the native layer takes the width of its weights and rows from here
         if s.Hp != self.Hp or (self.Hp == self.H and s.H != self.H):
             raise ValueError(f"shared expert of hidden size {s.H} does not match the layer's {self.H}")
-        self._shared_share = _share_buffer(self.T, self.q1.device)
+        if self._shared_share is None:  # kept for later shared experts: a run on another stream may still use it
+            self._shared_share = _share_buffer(self.T, self.q1.device)
         self._shared_layer = MoeLayer(
             T=self.T, H=self.H, Hp=self.Hp, I=s.I, max_padded=a.max_padded, top_k=1, E=1, E_routed=1,
             block_size_m=s.BM, q1=_ptr(self.q1), s1=_ptr(self.s1), sorted_ids=_ptr(a.sorted_ids),
@@ -1260,7 +1262,8 @@ def fused_experts(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tenso
              "expert_ids": 4 * -(-mp // bm), "ntpp": 4, "workspace": int(L.moe_align_workspace_bytes(S, n_align)),
              "local_blocks": 0 if expert_map is None else int(L.moe_layer_local_blocks_bytes(T, mp, bm)),
              "runs": int(L.moe_layer_runs_bytes(n_align)),
-             "share": int(L.moe_layer_share_bytes()) if 0 < S <= _SHARE_MAX_SLOTS else 0, "hq": mp * I, "hs": 4 * mp * (I // 128), "D": 2 * S * H}
+             "share": int(L.moe_layer_share_bytes()) if 0 < S <= _SHARE_MAX_SLOTS else 0,
+             "hq": mp * I, "hs": 4 * mp * (I // 128), "D": 2 * S * H}
     block = torch.empty(sum((n + 255 & ~255) + 256 for n in sizes.values()), dtype=torch.uint8, device=w1.device)
     y = torch.empty((T, H), dtype=torch.bfloat16, device=w1.device)
     layer = MoeLayer(T=T, H=H, Hp=H, I=I, max_padded=mp, top_k=k, E=E, E_routed=n_align, block_size_m=bm, tile_m=0,
