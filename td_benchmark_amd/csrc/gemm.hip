@@ -1319,11 +1319,34 @@ void w13_exact_kernel(GemmArgs g) {
 // by 16 tiles of 256: half the CUs) 146 / 73; Qwen3, one token, W13 21.8 / 15.3
 // (11.3 shared, below), W2 11.4 / 6.8.  Over one tile a CU the second tile of a CU
 // waits for the whole first: there the launches below are faster.
-template <class T, bool FUSED, bool EXACT>
+// BY_COLUMN: each XCD takes a contiguous range of a list in which a column's
+// row tiles are next to each other.  In block order the row tiles of one expert,
+// which read the same weights, fall to one XCD only where n_tiles is a multiple
+// of 8; elsewhere every XCD's L2 fetched them.  W13 of 90 tokens on one expert in
+// 16-row blocks, K 7040, 31 n-tiles (us, weights from HBM / in the caches): 51.3
+// / 50.3 in block order, 39.0 / 24.6 by column, 41.8 / 30.9 in the map of many
+// tiles; 32-row blocks of two experts, 53.0 and 29.6 in the caches.  Where
+// experts have one row tile each there is nothing to share: up to 10 % slower by
+// column (blocks that the bound counts and the slots do not fill leave the XCDs
+// uneven shares).
+template <class T, bool FUSED, bool EXACT, bool BY_COLUMN>
 __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
   const int tid = thread_id<T>();
-  const uint32_t tile = blockIdx.x / T::PARTS, part = blockIdx.x % T::PARTS;
-  const int64_t b = tile / (uint32_t)g.n_tiles, j = tile % (uint32_t)g.n_tiles;
+  uint32_t tile, part;
+  int64_t b, j;
+  if constexpr (BY_COLUMN) {
+    const uint32_t n_b = (uint32_t)g.max_blocks, total = n_b * (uint32_t)g.n_tiles * T::PARTS;
+    const uint32_t t = blockIdx.x % kXcds * ((total + kXcds - 1) / kXcds) + blockIdx.x / kXcds;
+    part = t / n_b % T::PARTS;
+    b = t % n_b;
+    j = t / n_b / T::PARTS;
+    tile = (uint32_t)(b * g.n_tiles + j);
+  } else {
+    tile = blockIdx.x / T::PARTS;
+    part = blockIdx.x % T::PARTS;
+    b = tile / (uint32_t)g.n_tiles;
+    j = tile % (uint32_t)g.n_tiles;
+  }
   const int64_t n_blocks = *g.ntpp / T::BM;
   // within max_padded for every b of the grid (the entries past ntpp are not used)
   const int64_t blk = g.blk ? (b < n_blocks ? g.blk[b] : 0) : b;
@@ -1334,7 +1357,7 @@ __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
   bool row_valid = false;
   if (tid < T::BM && pos0 + tid < g.max_padded) row_valid = g.sorted[pos0 + tid] < g.S;
   const int nvalid = __syncthreads_count(row_valid);
-  if (b >= n_blocks) return;
+  if (b >= n_blocks || (BY_COLUMN && j >= g.n_tiles)) return;
   if (e < 0 || e >= g.E) {
     if (part == 0) zero_tile<T, FUSED>(g, j, pos0, T::BM);
     return;
@@ -1343,31 +1366,40 @@ __device__ __forceinline__ void flat_gemm_body(const GemmArgs& g) {
   gemm_tile<T, FUSED, EXACT>(g, j, pos0, T::BM, e, nvalid, single, (int)part, (int)tile);
 }
 
-template <int BM, int GROUPS, bool FUSED, bool EXACT, int W>
+template <int BM, int GROUPS, bool FUSED, bool EXACT, int W, bool BY_COLUMN>
 __global__ __launch_bounds__((Tile<BM, GROUPS, true, false, W>::THREADS))
 __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flat_gemm_kernel(GemmArgs g) {
-  flat_gemm_body<Tile<BM, GROUPS, true, false, W>, FUSED, EXACT>(g);
+  flat_gemm_body<Tile<BM, GROUPS, true, false, W>, FUSED, EXACT, BY_COLUMN>(g);
 }
 
 constexpr int64_t kCus = 256;
 constexpr int64_t kShareK = 1024;
 static_assert(kCus / 2 <= kShareTiles, "a counter for each shared tile");
 
-template <int BM, int GROUPS, bool FUSED, bool EXACT, int W = 128>
-static int launch_flat(const GemmArgs& args, hipStream_t st) {
+template <int BM, int GROUPS, bool FUSED, bool EXACT, int W, bool BY_COLUMN>
+static int launch_flat_as(const GemmArgs& a, int64_t grid, hipStream_t st) {
   using T = Tile<BM, GROUPS, true, false, W>;
-  const void* fn = (const void*)flat_gemm_kernel<BM, GROUPS, FUSED, EXACT, W>;
+  const void* fn = (const void*)flat_gemm_kernel<BM, GROUPS, FUSED, EXACT, W, BY_COLUMN>;
   static const hipError_t attr_rc =
       hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
   if (attr_rc != hipSuccess) return kErrLaunch;
+  hipLaunchKernelGGL((flat_gemm_kernel<BM, GROUPS, FUSED, EXACT, W, BY_COLUMN>), dim3((unsigned)grid),
+                     dim3(T::THREADS), T::LDS_BYTES, st, a);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+template <int BM, int GROUPS, bool FUSED, bool EXACT, int W = 128>
+static int launch_flat(const GemmArgs& args, hipStream_t st) {
   GemmArgs a = args;
   if (GROUPS == 1) a.n_tiles = a.N / 128;
-  const int64_t grid = a.max_blocks * a.n_tiles * T::PARTS;
+  const int64_t grid = a.max_blocks * a.n_tiles * (128 / W);
   if (grid <= 0) return kOk;
-  hipLaunchKernelGGL((flat_gemm_kernel<BM, GROUPS, FUSED, EXACT, W>), dim3((unsigned)grid), dim3(T::THREADS),
-                     T::LDS_BYTES, st, a);
-  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+  // By column where block order spreads an expert's row tiles over the XCDs and
+  // the experts' mean makes several of them likely (two from half a block on).
+  if (a.n_tiles * (128 / W) % kXcds != 0 && 2 * a.S > (int64_t)BM * a.E)
+    return launch_flat_as<BM, GROUPS, FUSED, EXACT, W, true>(a, (grid + kXcds - 1) / kXcds * kXcds, st);
+  return launch_flat_as<BM, GROUPS, FUSED, EXACT, W, false>(a, grid, st);
 }
 
 template <int BM, bool FUSED, bool EXACT>
