@@ -1182,16 +1182,24 @@ __device__ __forceinline__ int planned_run(const GemmArgs& g, int l) {
   const int n_runs = __builtin_amdgcn_readfirstlane(g.runs[0]);
   if (n_runs <= 0) return 0;
   const int longest = (__builtin_amdgcn_readfirstlane(g.runs[5]) + BM - 1) / BM;  // row tiles of the first run
+  // A run of more row tiles than a unit may have cannot be dealt out by n-tiles
+  // (few XCDs would get it, and each of them all of its A rows): then the units
+  // are whole runs, and each XCD takes an even contiguous range of all their
+  // tiles.  W13 in expert order, by units and so (us): one expert, 2016 tokens, H
+  // 6912, I 1280 92 / 120 / 64; 13052 slots on 128 experts, Zipf, 32-row blocks,
+  // one n-tile 32 / 50 / 33; 3072 tokens on 4 experts, one n-tile 21 / 29 / 15.
+  const bool spread = longest > 1 && longest > g.unit_tiles;
   int group = g.unit_tiles / longest;
-  group = group < 1 ? 1 : (group > kTileGroup ? kTileGroup : group);
+  group = spread ? n_tiles : group < 1 ? 1 : (group > kTileGroup ? kTileGroup : group);
   const int groups = (n_tiles + group - 1) / group;  // of n-tiles, as even as possible:
   const int per_group = (n_tiles + groups - 1) / groups;
   const int n_units = n_runs * groups;
+  const int stride = spread ? 1 : kXcds;
   const v4i* runs = reinterpret_cast<const v4i*>(g.runs + 4);
   v4i r;
   int w, n, incl;  // this lane's unit, its tiles, and those up to it
   auto look = [&](int k) {
-    w = kXcds * k + ((k & 1) ? kXcds - 1 - x : x);
+    w = spread ? k : kXcds * k + ((k & 1) ? kXcds - 1 - x : x);
     r = (v4i){0, 0, 0, 0};
     n = 0;
     if (w < n_units) {
@@ -1209,13 +1217,19 @@ __device__ __forceinline__ int planned_run(const GemmArgs& g, int l) {
   // this XCD's tiles, and the lane and the unit that tile l falls to
   auto tiles_of = [&] {
     int sum = 0;
-    for (int k0 = 0; kXcds * k0 < n_units; k0 += 64) {
+    for (int k0 = 0; stride * k0 < n_units; k0 += 64) {
       look(k0 + lane);
       sum += __builtin_amdgcn_readlane(incl, 63);
     }
     return sum;
   };
-  const int mine = tiles_of();
+  int mine = tiles_of(), start = 0;
+  if (spread) {
+    const int share = (mine + kXcds - 1) / kXcds;
+    start = x * share;
+    mine = mine - start < share ? mine - start : share;
+    if (mine <= 0) return 0;
+  }
   int wgs = mine, half = -1;
   if constexpr (BM >= 128 && !(EXACT && BM == 256)) {
     const int rest = mine % kXcdCus;
@@ -1228,24 +1242,31 @@ __device__ __forceinline__ int planned_run(const GemmArgs& g, int l) {
     }
   }
   if (l >= mine) return wgs;
+  l += start;
   int before = 0;
   uint64_t at = 0;
   for (int k0 = 0;; k0 += 64) {
-    if (n_units > 64 * kXcds) look(k0 + lane);  // else the lanes still hold all of them
+    if (n_units > 64 * stride) look(k0 + lane);  // else the lanes still hold all of them
     at = __ballot(before + incl > l);
     if (at) break;
     before += __builtin_amdgcn_readlane(incl, 63);
   }
   const int src = __ffsll((unsigned long long)at) - 1;
-  const int in = l - before - __builtin_amdgcn_readlane(incl - n, src);  // tile of the unit
+  int in = l - before - __builtin_amdgcn_readlane(incl - n, src);  // tile of the unit
   w = __builtin_amdgcn_readlane(w, src);
   n = __builtin_amdgcn_readlane(n, src);
   const int first = __builtin_amdgcn_readlane(r[0], src), cnt = __builtin_amdgcn_readlane(r[1], src);
   const int padded = __builtin_amdgcn_readlane(r[3], src);
   const int e = __builtin_amdgcn_readlane(r[2], src);
-  const int units = (cnt + BM - 1) / BM, gsz = n / units;
+  const int units = (cnt + BM - 1) / BM;
   const bool by_col = !FUSED && g.K >= kColMajorK;
-  const int64_t j = w % groups * per_group + (by_col ? in / units : in % gsz);
+  int j0 = w % groups * per_group, gsz = n / units;
+  if (spread) {  // n-tiles in groups, as the other maps take them
+    j0 = in / (kTileGroup * units) * kTileGroup;
+    gsz = n_tiles - j0 < kTileGroup ? n_tiles - j0 : kTileGroup;
+    in -= j0 * units;
+  }
+  const int64_t j = j0 + (by_col ? in / units : in % gsz);
   const int r0 = (by_col ? in % units : in / gsz) * BM;
   int64_t pos0 = first + r0;
   int nvalid = cnt - r0 < BM ? cnt - r0 : BM;

@@ -44,6 +44,8 @@ def _stream_handle(stream: torch.cuda.Stream | None = None) -> int:
 
 
 def _stream(stream: torch.cuda.Stream | None = None) -> ctypes.c_void_p:
+    if stream is None and _RAW_STREAM is not None and _CUR_DEVICE is not None:
+        return ctypes.c_void_p(_RAW_STREAM(_CUR_DEVICE()))
     return ctypes.c_void_p(_stream_handle(stream))
 
 

@@ -46,6 +46,12 @@ CASES = [
     (515, 256, 640, 2, 2, 128, 256, "one_expert", False),  # every token in both runs
     (257, 256, 256, 3, 1, 256, 256, "softmax", True),
     (2600, 256, 640, 5, 1, 128, 256, "zipf", False),       # a run of many row tiles: units of one n-tile
+    # a run of more row tiles than a unit may have: contiguous ranges of the runs' tiles
+    (2016, 384, 1280, 1, 1, 256, 0, "softmax", False),     # one expert
+    (3000, 256, 128, 40, 2, 32, 0, "zipf", False),         # one n-tile
+    (1200, 256, 128, 4, 4, 256, 0, "softmax", False),      # every token on each of four
+    (1500, 256, 640, 700, 1, 64, 0, "one_expert", False),
+    (900, 256, 384, 2, 1, 256, 0, "zipf", True),
 ]
 
 
