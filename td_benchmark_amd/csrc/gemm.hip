@@ -1525,7 +1525,11 @@ static int resolve_tile_m(int32_t tile_m, int32_t BM, int64_t S, int64_t E) {
 static void set_blocks(GemmArgs& g, const LocalBlocks& local, int TM, int vshift) {
   g.blk = local.blocks;
   if (local.E_routed == 0 && TM > (g.bma >> vshift)) g.bma |= kMergedRuns;
-  g.runs = local.runs;
+  // Tall tiles of experts with few rows (a block size far over the mean) are all
+  // alike, one short body each, and go in expert order: 5 rows an expert, 512
+  // experts in 256-row blocks 342 us a layer so and 360 dealt out; 11 rows, 1024
+  // experts 242 and 248.  From 64 rows an expert on dealing out gains (above).
+  g.runs = TM >= 128 && g.S < 32 * local.E_routed ? nullptr : local.runs;
   g.share = local.share;
   if (local.E_routed > 0) {
     const int64_t most = blocks_bound(g.S, local.E_routed, g.bma) << vshift;

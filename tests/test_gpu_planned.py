@@ -39,7 +39,8 @@ CASES = [
     (600, 256, 1152, 8, 2, 128, 256, "softmax", False),   # 256-row tiles over 128-row blocks, split rounds
     (700, 384, 640, 12, 2, 256, 0, "zipf", False),
     (500, 256, 2304, 6, 3, 64, 128, "zipf", False),
-    (900, 256, 1152, 300, 4, 128, 128, "softmax", False),  # 900 units
+    (900, 256, 1152, 300, 4, 128, 128, "softmax", False),  # 12 rows an expert in tall tiles: expert order
+    (2400, 256, 1152, 300, 4, 128, 128, "softmax", False),  # 32: 900 units
     (300, 256, 1152, 40, 4, 64, 0, "zipf", False),
     (310, 256, 2304, 40, 4, 32, 0, "zipf", False),
     (640, 256, 1152, 4, 2, 256, 0, "zipf", True),          # 128-row exact tiles, padding past the last tile
@@ -68,12 +69,13 @@ def test_planned_map_equals_the_expert_ordered_one(T, H, I, E, k, BM, tile_m, ro
     _compare(r, g, ids)
 
 
-def test_more_tiles_than_the_grid_allows_for():
+@pytest.mark.parametrize("T", [900, 1100])  # fewer than 32 rows an expert (expert order) and more
+def test_more_tiles_than_the_grid_allows_for(T):
     """One rank of 32 whose 8 experts get every token: four times the tiles the
     grid is sized for."""
     from td_benchmark_amd import ops
-    print("case: planned, every token to one rank of 32", flush=True)
-    T, E, k = 900, 256, 8
+    print(f"case: planned, every token to one rank of 32, T={T}", flush=True)
+    E, k = 256, 8
     c = make_case(T, 256, 2048, 8, k, 128, seed=9)
     g = to_gpu(c)
     w = (g["w13"], g["w13_s"], g["w2"], g["w2_s"])
